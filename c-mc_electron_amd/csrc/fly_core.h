@@ -48,9 +48,9 @@ EMC_HD inline void tally_add(unsigned long long* p, long long v) {
 EMC_HD inline long long fxd(double v, double scale) { return (long long)rint(v * scale); }
 
 struct Flight {
-  const BandDev& B;
-  const MeshDev& M;
-  const FieldsDev& F;
+  const EMC_CST BandDev& B;
+  const EMC_CST MeshDev& M;
+  const EMC_CST FieldsDev& F;
   const TallyDev& T;
   CloneRec* clones;
   unsigned long long* nclones;
@@ -67,7 +67,7 @@ struct Flight {
   long long n_events, n_phonon, n_impurity;
   Rng rng;
 
-  EMC_HD Flight(const BandDev& b, const MeshDev& m, const FieldsDev& f, const TallyDev& t)
+  EMC_HD Flight(const EMC_CST BandDev& b, const EMC_CST MeshDev& m, const EMC_CST FieldsDev& f, const TallyDev& t)
       : B(b), M(m), F(f), T(t), clones(nullptr), nclones(nullptr), clone_cap(0) {}
 
   EMC_HD EMC_INL double Random() { return rng.next(); }
@@ -95,15 +95,15 @@ struct Flight {
     zo = v[ms(2, isym) - 1] * ms(5, isym);
   }
   EMC_HD EMC_INL void GetV() {
-    const TetRec& r = B.tr[itet];
+    const EMC_GLB TetRec& r = B.tr[itet];
     out_wedge(vx, vy, vz, r.vt[0], r.vt[1], r.vt[2]);
   }
   EMC_HD EMC_INL void GetEnergy() {
     double dx, dy, dz;
     in_wedge(dx, dy, dz, kx, ky, kz);
-    const CornerRec& q = B.cr[itet];
+    const EMC_GLB CornerRec& q = B.cr[itet];
     dx -= q.x[0]; dy -= q.y[0]; dz -= q.z[0];
-    const TetRec& r = B.tr[itet];
+    const EMC_GLB TetRec& r = B.tr[itet];
     energy = r.vt[3] + r.vt[0] * dx + r.vt[1] * dy + r.vt[2] * dz;
   }
 
@@ -116,9 +116,9 @@ struct Flight {
     return 0.50 * sqrt(sbx * sbx + sby * sby + sbz * sbz);
   }
   EMC_HD EMC_INL double surf(double e, int it) const {
-    const CornerRec& q = B.cr[it];
+    const EMC_GLB CornerRec& q = B.cr[it];
     const int c0 = 0, c1 = 1, c2 = 2, c3 = 3;
-    const double *X = q.x, *Y = q.y, *Z = q.z;
+    const EMC_GLB double *X = q.x, *Y = q.y, *Z = q.z;
     const double e0 = q.e[0], e1 = q.e[1], e2 = q.e[2], e3 = q.e[3];
     double r;
     if (!(e > e0 && e < e3)) return 0.0;
@@ -158,7 +158,7 @@ struct Flight {
     return 0.0;
   }
   EMC_HD EMC_INL double fastsurf(double e, int it) { return fastsurf_r(e, it, B.sr[it]); }
-  EMC_HD EMC_INL double fastsurf_r(double e, int it, const SurfRec& s) {
+  EMC_HD EMC_INL double fastsurf_r(double e, int it, const EMC_GLB SurfRec& s) {
     double r = fastsurf_signed(e, it, s);
     if (r < 0.0) {
       if (T.counters) count(CNT_DROP0 + 6);
@@ -167,7 +167,7 @@ struct Flight {
     return r;
   }
   // FASTSURF before the clamp of a negative value (which fastsurf_r tallies)
-  EMC_HD EMC_INL double fastsurf_signed(double e, int it, const SurfRec& s) {
+  EMC_HD EMC_INL double fastsurf_signed(double e, int it, const EMC_GLB SurfRec& s) {
     const double e0 = s.e[0], e1 = s.e[1], e2 = s.e[2], e3 = s.e[3];
     double r = 0.0;
     if (e > e0 && e < e3) {
@@ -193,7 +193,7 @@ struct Flight {
   }
   // Band::CALDOS / CALDOSSUM (src/Band.cpp:2234-2295)
   EMC_HD EMC_INL double caldos(double e, int ib) const {
-    const double* d = &B.dos[(size_t)ib * NTAB1];
+    const EMC_GLB double* d = &B.dos[(size_t)ib * NTAB1];
     if (e <= 0e0) return d[0];
     if (e >= B.emax) return d[MTAB];
     const int itab = (int)(e / B.dtable);
@@ -241,7 +241,7 @@ struct Flight {
     }
   }
   EMC_HD EMC_INL double caldostetmax(double e, int ib) const {
-    const double* d = &B.dostetmax[(size_t)ib * NTAB1];
+    const EMC_GLB double* d = &B.dostetmax[(size_t)ib * NTAB1];
     if (e <= 0.0) return d[0];
     if (e >= B.emax) return d[MTAB];
     const int itab = (int)(e / B.dtable);
@@ -260,21 +260,21 @@ struct Flight {
 
   // ---- tetrahedron search (src/ParticleUtils.cpp:331-625)
   EMC_HD EMC_INL bool contains(int it, double a, double b, double c) const {
-    const TetRec& r = B.tr[it];
+    const EMC_GLB TetRec& r = B.tr[it];
     const double d1 = r.n[0][0] * a + r.n[0][1] * b + r.n[0][2] * c - r.n[0][3];
     const double d2 = r.n[1][0] * a + r.n[1][1] * b + r.n[1][2] * c - r.n[1][3];
     const double d3 = r.n[2][0] * a + r.n[2][1] * b + r.n[2][2] * c - r.n[2][3];
     const double d4 = r.n[3][0] * a + r.n[3][1] * b + r.n[3][2] * c - r.n[3][3];
     return (d1 >= -MY_ZERO) && (d2 >= -MY_ZERO) && (d3 >= -MY_ZERO) && (d4 >= -MY_ZERO);
   }
-  EMC_HD EMC_INL static bool in_sphere(const Sphere& s, double a, double b, double c) {
+  EMC_HD EMC_INL static bool in_sphere(const EMC_GLB Sphere& s, double a, double b, double c) {
     const double dx = a - s.cx, dy = b - s.cy, dz = c - s.cz;
     return dx * dx + dy * dy + dz * dz <= s.r2;
   }
   // first tetrahedron of list[p0 .. p0+nn-1] (in list order) that holds the point;
   // the sphere array runs alongside the list, so most candidates cost 32 bytes
   // read in order instead of a dependent load of their record
-  EMC_HD EMC_INL bool scan(const int* list, const Sphere* sph, int p0, int nn, double a, double b, double c) {
+  EMC_HD EMC_INL bool scan(const EMC_GLB int* list, const EMC_GLB Sphere* sph, int p0, int nn, double a, double b, double c) {
     const int end = p0 + nn;
     int itl = p0;
     // eight sphere tests per round, their loads independent of each other
@@ -303,18 +303,20 @@ struct Flight {
   // index), the last holding entry what the scan over all tetrahedra returns; the
   // buckets are tried in the scans' order: tlists bin, tlist bins ie, ie+1, ie-1.
   EMC_HD EMC_INL bool locate(double a, double b, double c) {
-    const TetIdxRoot& R = B.troot[iband];
+    const EMC_GLB TetIdxRoot& R = B.troot[iband];
     if (!(a >= R.lo[0] && a <= R.hi[0] && b >= R.lo[1] && b <= R.hi[1] && c >= R.lo[2] && c <= R.hi[2]))
       return false;  // outside every tetrahedron of the band
     double l0 = R.lo[0], l1 = R.lo[1], l2 = R.lo[2], h0 = R.hi[0], h1 = R.hi[1], h2 = R.hi[2];
-    TetIdxNode nd = B.tnode[R.node];
-    while (nd.count < 0) {
+    int nf = B.tnode[R.node].first, nc = B.tnode[R.node].count;
+    while (nc < 0) {
       const double m0 = 0.5 * (l0 + h0), m1 = 0.5 * (l1 + h1), m2 = 0.5 * (l2 + h2);
       int ch = 0;
       if (a >= m0) { ch |= 1; l0 = m0; } else h0 = m0;
       if (b >= m1) { ch |= 2; l1 = m1; } else h1 = m1;
       if (c >= m2) { ch |= 4; l2 = m2; } else h2 = m2;
-      nd = B.tnode[nd.first + ch];
+      const EMC_GLB TetIdxNode& nd = B.tnode[nf + ch];
+      nf = nd.first;
+      nc = nd.count;
     }
     int ies = (int)(energy * B.dlists);
     if (ies < 0) ies = 0;
@@ -323,8 +325,8 @@ struct Flight {
     if (ie < 0) ie = 0;
     if (ie >= MWLE) ie = MWLE - 1;
     int bs = -1, b0 = -1, bup = -1, bdn = -1, ball = -1;
-    for (int q = nd.first; q < nd.first + nd.count; ++q) {
-      const TetIdxEntry& E = B.tent[q];
+    for (int q = nf; q < nf + nc; ++q) {
+      const EMC_GLB TetIdxEntry& E = B.tent[q];
       if (!(a >= (double)E.lo[0] && a <= (double)E.hi[0] && b >= (double)E.lo[1] && b <= (double)E.hi[1] &&
             c >= (double)E.lo[2] && c <= (double)E.hi[2]))
         continue;
@@ -395,8 +397,8 @@ struct Flight {
 
   // ---- final state on the iso-energy surface (src/ParticleUtils.cpp:48-284)
   EMC_HD EMC_INL void getK() {
-    const CornerRec& q = B.cr[itet];
-    const double *X = q.x, *Y = q.y, *Z = q.z, *E = q.e;
+    const EMC_GLB CornerRec& q = B.cr[itet];
+    const EMC_GLB double *X = q.x, *Y = q.y, *Z = q.z, *E = q.e;
     const int c0 = 0, c1 = 1, c2 = 2, c3 = 3;
     const double rv1 = 1.0 - sqrt(Random());
     const double rv2 = Random() * (1.0 - rv1);
@@ -461,7 +463,7 @@ struct Flight {
     }
     const int nted = smallfl ? B.ntlists[itab * MNB + iband] : B.ntlist[itab * MNB + iband];
     const int base = smallfl ? B.ptlists[itab * MNB + iband] : B.ptlist[itab * MNB + iband];
-    const int* list = smallfl ? B.tlists : B.tlist;
+    const EMC_GLB int* list = smallfl ? B.tlists : B.tlist;
     if (nted == 0) { Flag_SelfScatter = 1; return; }
     int count2 = 0;
     // Rejection loop.  On the GPU every lane of the wave leaves it together
@@ -474,7 +476,7 @@ struct Flight {
       if (!again) continue;
       itet = list[(int)(nted * Random()) + base];
       count2++;
-      const SurfRec& sr = B.sr[itet];
+      const EMC_GLB SurfRec& sr = B.sr[itet];
       if ((count2 < 10000) && !((sr.e[0] < e) && (sr.e[3] > e))) continue;
       const double dostet = fastsurf_r(e, itet, sr) / sr.vgt;
       if (((Random() * maxdostet) > dostet) && (count2 < 10000)) continue;
@@ -513,10 +515,10 @@ struct Flight {
   }
   // one try of the loop: true when the search goes on
   EMC_HD EMC_INL bool gs_try(double e, double maxdostet, int nted, int base, bool small, int& count2) {
-    const int* list = small ? B.tlists : B.tlist;
+    const EMC_GLB int* list = small ? B.tlists : B.tlist;
     itet = list[(int)(nted * Random()) + base];
     count2++;
-    const SurfRec& sr = B.sr[itet];
+    const EMC_GLB SurfRec& sr = B.sr[itet];
     if ((count2 < GS_CAP) && !((sr.e[0] < e) && (sr.e[3] > e))) return true;
     const double dostet = fastsurf_r(e, itet, sr) / sr.vgt;
     if (((Random() * maxdostet) > dostet) && (count2 < GS_CAP)) return true;
@@ -531,9 +533,9 @@ struct Flight {
   // e, its DOS weight when it does and whether FASTSURF was negative there
   EMC_HD EMC_INL void gs_eval(double e, int nted, int base, bool small, double u, int& it, bool& span, bool& neg,
                               double& dostet) {
-    const int* list = small ? B.tlists : B.tlist;
+    const EMC_GLB int* list = small ? B.tlists : B.tlist;
     it = list[(int)(nted * u) + base];
-    const SurfRec& sr = B.sr[it];
+    const EMC_GLB SurfRec& sr = B.sr[it];
     span = (sr.e[0] < e) && (sr.e[3] > e);
     neg = false;
     dostet = 0.0;
@@ -753,7 +755,7 @@ struct Flight {
       else { it = (int)((ie - 11.0) + 0.5); it = it < 1 ? 1 : it > 60 ? 115 : it; ei = 35 + it; ed = 1.0; }  // > 60 jumps to 115, as the reference
     }
     const int R = tab < 2 ? 201 : 51;  // PTAB_ROWS
-    const double* col = B.ptab[tab] + (size_t)(ei - 1) * R;
+    const EMC_GLB double* col = B.ptab[tab] + (size_t)(ei - 1) * R;
     const double ran = Random();
     int i = 0;
     double ksum = 0.0;
@@ -857,10 +859,10 @@ struct Flight {
     const int is = iscat % np, f = iscat / np;
     const int ini = iband - (elec ? B.bandofE : B.bandofH);
     const int nb = elec ? 4 : 3;
-    const double* dos = elec ? B.dose : B.dosh;
-    const double* sc = elec ? B.scatte : B.scatth;
-    const double* ii = elec ? B.scattiie : B.scattiih;
-    const double* drow;
+    const EMC_GLB double* dos = elec ? B.dose : B.dosh;
+    const EMC_GLB double* sc = elec ? B.scatte : B.scatth;
+    const EMC_GLB double* ii = elec ? B.scattiie : B.scattiih;
+    const EMC_GLB double* drow;
     if (is < np - 1) {
       const double k = sc[((size_t)is * nb + f) * nb + ini];
       drow = &dos[((size_t)is * nb + f) * NTAB1];
@@ -1112,7 +1114,7 @@ struct Flight {
     double xkl, ykl, zkl, xfl, yfl, zfl;
     in_wedge(xkl, ykl, zkl, kx, ky, kz);
     in_wedge(xfl, yfl, zfl, Ex, Ey, Ez);
-    const TetRec& r = B.tr[itet];
+    const EMC_GLB TetRec& r = B.tr[itet];
     double best = 0.0;
     for (int f = 0; f < 4; ++f) {
       const double nf = r.n[f][0] * xfl + r.n[f][1] * yfl + r.n[f][2] * zfl;

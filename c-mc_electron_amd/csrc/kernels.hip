@@ -62,6 +62,10 @@ __device__ inline void finish_drop(const TallyDev& T, const Flight& f) {
 }
 
 // ------------------------------------------------------------------ flight
+// the flight's descriptors as constant memory (see EMC_CST)
+__device__ __forceinline__ const EMC_CST FlyConst& fly_const(const FlyConst* c) {
+  return *(const EMC_CST FlyConst*)c;
+}
 __device__ inline void load_particle(Flight& f, const FlyArgs& a, long long q, uint32_t pk) {
   f.clones = a.clones;
   f.nclones = a.nclones;
@@ -99,7 +103,7 @@ __global__ __launch_bounds__(256, 3) void k_fly_fast(AS as_) {
     if (q < a.n) {
       const uint32_t pk = a.P.pk[q];
       if (pk != PK_DEAD) {
-        Flight f(a.C->B, a.C->M, a.C->F, a.T);
+        Flight f(fly_const(a.C).B, fly_const(a.C).M, fly_const(a.C).F, a.T);
         load_particle(f, a, q, pk);
         Flight::Loop L;
         f.fly_begin(L);
@@ -259,7 +263,7 @@ __global__ __launch_bounds__(256) void k_fly_slow(AS as_) {
     const bool act = lane < lpw && e < ns;
     if (!__ballot(act)) break;
     long long q = 0;
-    Flight f(a.C->B, a.C->M, a.C->F, a.T);
+    Flight f(fly_const(a.C).B, fly_const(a.C).M, fly_const(a.C).F, a.T);
     if (act) {
       q = a.slow[e];
       load_particle(f, a, q, a.P.pk[q]);
@@ -294,7 +298,7 @@ __device__ __forceinline__ void fly_clone_range(const FlyArgs& a, unsigned long 
   if (lane < lpw) {
     for (long long q = (long long)begin + wave * lpw + lane; q < (long long)end; q += nwaves * lpw) {
       CloneRec& c = a.clones[q];
-      Flight f(a.C->B, a.C->M, a.C->F, a.T);
+      Flight f(fly_const(a.C).B, fly_const(a.C).M, fly_const(a.C).F, a.T);
       f.clones = a.clones;
       f.nclones = a.nclones;
       f.clone_cap = a.clone_cap;
@@ -685,8 +689,8 @@ __global__ __launch_bounds__(256) void k_deposit_tile(AS as_) {
     atomicAdd(&sc[3 * TILE_CELLS + lc], 1ull);
     if (want_stat) {
       const int isym = a.P.isym[q];
-      const double* vt = a.B.tr[a.P.itet[q]].vt;
-      const int* ms = a.B.matsym;
+      const auto* vt = a.B.tr[a.P.itet[q]].vt;
+      const auto* ms = a.B.matsym;
       const double v3[3] = {vt[0], vt[1], vt[2]};
       const double vx = v3[ms[0 * 48 + isym] - 1] * ms[3 * 48 + isym];
       const double vy = v3[ms[1 * 48 + isym] - 1] * ms[4 * 48 + isym];
@@ -1521,8 +1525,8 @@ __global__ __launch_bounds__(256) void k_sample_population(SampleArgs a) {
     }
     const uint32_t pk = a.gpk[lo];
     const int i = pk_i(pk), j = pk_j(pk), k = pk_k(pk);
-    const MeshDev& M = a.C->M;
-    Flight f(a.C->B, M, a.C->F, T);
+    const EMC_CST MeshDev& M = fly_const(a.C).M;
+    Flight f(fly_const(a.C).B, M, fly_const(a.C).F, T);
     const uint64_t key = init_key(a.seed, (uint64_t)s);
     f.rng.init(key, ~0ull);
     double lam = f.Random();
