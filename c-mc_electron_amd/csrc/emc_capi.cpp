@@ -197,6 +197,7 @@ struct BandBundle {
   std::vector<SurfRec> surfrec;
   std::vector<CornerRec> cornerrec;
   std::vector<Sphere> tsph, tlist_s, tlists_s, slist_s;
+  std::vector<uint32_t> symw;  // matsym packed, one word per operation
   TetIndex tix;         // empty when build_tet_index refused the tables
   std::string tix_why;  // why it refused
 };
@@ -260,7 +261,9 @@ static void fill_band_dev_host(emc_ctx* c, BandDev& B) {
   B.tet = b.tet.data();
   B.xkk = b.xkk.data(); B.ykk = b.ykk.data(); B.zkk = b.zkk.data(); B.eek = b.eek.data();
   B.vgt = b.vgt.data(); B.faclow = b.faclow.data(); B.facmed = b.facmedium.data(); B.fachigh = b.fachigh.data();
-  B.matsym = &b.matsym[0][0]; B.indmat = b.indmat; B.newisym = &b.newisym[0][0];
+  B.matsym = &b.matsym[0][0];
+  B.symw = c->bb->symw.data();
+  B.indmat = b.indmat; B.newisym = &b.newisym[0][0];
   B.xbz = &b.xbz[0][0]; B.ybz = &b.ybz[0][0]; B.zbz = &b.zbz[0][0];
   B.ntlist = b.ntlist.data(); B.ptlist = b.ptlist.data(); B.tlist = b.tlist.data();
   B.nslist = b.nslist.data(); B.pslist = b.pslist.data(); B.slist = b.slist.data();
@@ -294,6 +297,9 @@ static void fill_mesh_dev_scalars(emc_ctx* c, MeshDev& M) {
 
 static void build_tetrec(BandBundle& bb) {
   const Band& b = bb.band;
+  bb.symw.resize(NSYM);
+  for (int q = 0; q < NSYM; ++q)
+    bb.symw[q] = sym_word(b.matsym[0][q], b.matsym[1][q], b.matsym[2][q], b.matsym[3][q], b.matsym[4][q], b.matsym[5][q]);
   bb.tetrec.assign(b.nt, TetRec{});
   for (int it = 0; it < b.nt; ++it) {
     TetRec& r = bb.tetrec[it];
@@ -471,7 +477,9 @@ static std::string device_band(emc_ctx* c, std::shared_ptr<DevBand>& out) {
   B.tet = m.dup(b.tet);
   B.xkk = m.dup(b.xkk); B.ykk = m.dup(b.ykk); B.zkk = m.dup(b.zkk); B.eek = m.dup(b.eek);
   B.vgt = m.dup(b.vgt); B.faclow = m.dup(b.faclow); B.facmed = m.dup(b.facmedium); B.fachigh = m.dup(b.fachigh);
-  B.matsym = m.dup(&b.matsym[0][0], 6 * 48); B.indmat = m.dup(b.indmat, 729);
+  B.matsym = m.dup(&b.matsym[0][0], 6 * 48);
+  B.symw = m.dup(bb.symw);
+  B.indmat = m.dup(b.indmat, 729);
   B.newisym = m.dup(&b.newisym[0][0], 5 * 48);
   B.xbz = m.dup(&b.xbz[0][0], 5 * 48); B.ybz = m.dup(&b.ybz[0][0], 5 * 48); B.zbz = m.dup(&b.zbz[0][0], 5 * 48);
   B.ntlist = m.dup(b.ntlist); B.ptlist = m.dup(b.ptlist); B.tlist = m.dup(b.tlist);
@@ -519,6 +527,15 @@ static int gpu_setup(emc_ctx* c) {
   M.motion = m.dup(d.motion); M.attached = m.dup(d.attached); M.insurf = m.dup(d.insurf);
   M.nearest_surf = m.dup(d.nearest_surf); M.da = m.dup(d.da);
   M.surface_dir = m.dup(c->surface_dir);
+  {
+    std::vector<uint64_t> info(d.ncell);
+    for (size_t q = 0; q < info.size(); ++q) {
+      uint64_t w = (uint64_t)d.insurf[q] << 48;
+      for (int f = 0; f < 6; ++f) w |= (uint64_t)d.motion[6 * q + f] << (8 * f);
+      info[q] = w;
+    }
+    M.minfo = m.dup(info);
+  }
   g.dx = M.dx; g.dy = M.dy; g.dz = M.dz; g.da = M.da;
   g.cvol = m.dup(d.cvol);
   g.eeff = m.dup(d.eeff_dir);

@@ -21,6 +21,7 @@
 #include <type_traits>
 
 #include "fly_core.h"
+#include "fly_fast.h"
 #include "kernels.h"
 #include "qc.h"
 
@@ -82,14 +83,13 @@ __device__ inline void load_particle(Flight& f, const FlyArgs& a, long long q, u
   f.rng.init(f.key, a.step);
 }
 
-// Fast pass: particles whose step has only tetrahedron and plain cell crossings
-// (Flight::fast_step) finish here.  The others are listed, wave-compacted, for
-// k_fly_slow, which restarts them from the untouched state: the RNG is counter
-// based, so the full event loop draws the same numbers and the result equals one
-// pass of fly().  (Refilling finished lanes from a per-wave chunk, so that a
-// wave does not wait for its longest history, was measured slower: most
-// particles end after one or two events, so nearly every iteration paid for a
-// refill.)
+// Fast pass (FastFlight): particles whose step has only tetrahedron and plain cell
+// crossings finish here.  The others are listed, wave-compacted, for k_fly_slow,
+// which restarts them from the untouched state: the RNG is counter based, so the
+// full event loop draws the same numbers and the result equals one pass of fly().
+// (Refilling finished lanes from a per-wave chunk, so that a wave does not wait
+// for its longest history, was measured slower: most particles end after one or
+// two events, so nearly every iteration paid for a refill.)
 template <class AS>
 __global__ __launch_bounds__(256, 3) void k_fly_fast(AS as_) {
   const FlyArgs& a = kargs(as_);
@@ -103,22 +103,24 @@ __global__ __launch_bounds__(256, 3) void k_fly_fast(AS as_) {
     if (q < a.n) {
       const uint32_t pk = a.P.pk[q];
       if (pk != PK_DEAD) {
-        Flight f(fly_const(a.C).B, fly_const(a.C).M, fly_const(a.C).F, a.T);
-        load_particle(f, a, q, pk);
-        Flight::Loop L;
-        f.fly_begin(L);
-        int pend_kind = 0, pend_j = 0, r = Flight::FAST_DONE;
-        while (f.left_time > 0) {
-          r = f.fast_step(L, pend_kind, pend_j);
-          if (r != Flight::FAST_MORE) break;
-        }
-        if (r != Flight::FAST_BAIL) {
+        FastFlight f(fly_const(a.C).B, fly_const(a.C).M, fly_const(a.C).F);
+        f.x = a.P.x[q]; f.y = a.P.y[q]; f.z = a.P.z[q];
+        f.kx = a.P.kx[q]; f.ky = a.P.ky[q]; f.kz = a.P.kz[q];
+        f.energy = a.P.energy[q];
+        f.icell = pk_i(pk); f.jcell = pk_j(pk); f.kcell = pk_k(pk); f.type = pk_type(pk);
+        f.itet = a.P.itet[q]; f.isym = a.P.isym[q];
+        const uint64_t key = a.P.key[q];
+        f.k0 = (uint32_t)key; f.k1 = (uint32_t)(key >> 32);
+        f.c1 = (uint32_t)a.step; f.c2 = (uint32_t)(a.step >> 32);
+        f.left = f.M.dt;
+        if (f.run() == FastFlight::DONE) {
           ev += f.n_events;
-          f.commit_pending(pend_kind, pend_j);
+          if (f.pend_kind == 1) tally_add(&a.T.rcur[f.pend_j], fxd(a.P.charge[q], Flight::EMC_FX_CONTACT_));
+          else if (f.pend_kind == 2) tally_add(&a.T.lcur[f.pend_j], fxd(a.P.charge[q], Flight::EMC_FX_CONTACT_));
           a.P.x[q] = f.x; a.P.y[q] = f.y; a.P.z[q] = f.z;
           a.P.kx[q] = f.kx; a.P.ky[q] = f.ky; a.P.kz[q] = f.kz;
           a.P.energy[q] = f.energy;
-          const uint32_t pk2 = pk_make(f.par_type, f.icell, f.jcell, f.kcell);
+          const uint32_t pk2 = pk_make(f.type, f.icell, f.jcell, f.kcell);
           if (pk2 != pk) a.P.pk[q] = pk2;
           a.P.itet[q] = f.itet; a.P.isym[q] = f.isym;
         } else

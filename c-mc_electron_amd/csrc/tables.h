@@ -81,6 +81,13 @@ struct alignas(32) TetIdxEntry {
 };
 static_assert(sizeof(TetIdxEntry) == 32, "TetIdxEntry layout");
 
+// A symmetry operation in one word: bits 2r, 2r+1 the axis that output axis r takes
+// (matsym[r] - 1), bit 6 + r set where its sign (matsym[3 + r]) is -1.
+EMC_HD inline uint32_t sym_word(int m0, int m1, int m2, int s0, int s1, int s2) {
+  return (uint32_t)(m0 - 1) | (uint32_t)(m1 - 1) << 2 | (uint32_t)(m2 - 1) << 4 | (s0 < 0 ? 64u : 0u) |
+         (s1 < 0 ? 128u : 0u) | (s2 < 0 ? 256u : 0u);
+}
+
 struct BandDev {
   const EMC_GLB TetRec* tr;
   const EMC_GLB TetIdxRoot* troot; // [MNB] or null: no index, Getisym scans the lists
@@ -94,6 +101,7 @@ struct BandDev {
   const EMC_GLB double *xkk, *ykk, *zkk, *eek;
   const EMC_GLB double *vgt, *faclow, *facmed, *fachigh;
   const EMC_GLB int *matsym, *indmat, *newisym;
+  const EMC_GLB uint32_t* symw;  // [NSYM] matsym packed (sym_word)
   const EMC_GLB double *xbz, *ybz, *zbz;
   const EMC_GLB int *ntlist, *ptlist, *tlist, *nslist, *pslist, *slist, *ntlists, *ptlists, *tlists;
   const EMC_GLB int* ibt;
@@ -115,6 +123,7 @@ struct MeshDev {
   const EMC_GLB int* nearest_surf; // [ncell]
   const EMC_GLB double* da; // [ncell]
   const EMC_GLB int* surface_dir; // [nsurf]
+  const EMC_GLB uint64_t* minfo; // [ncell] motion rules of the six faces in bytes 0-5, insurf in byte 6
   int cnx, cny, cnz, pnx, pny, pnz, ncontact, flag_surface, flag_simp, pad0;
   double dt, eV0, conc0, scrt0, eps_si, frickel;
   double charge_sign[3];
