@@ -98,6 +98,36 @@ struct Flight {
     const EMC_GLB TetRec& r = B.tr[itet];
     out_wedge(vx, vy, vz, r.vt[0], r.vt[1], r.vt[2]);
   }
+  // What an event reads of the tetrahedron and the cell, loaded together: the
+  // event's reads then cost one memory round trip instead of one for each of its
+  // parts (velocity, four faces, rates, planes, surface data).
+  struct Event {
+    double n[4][4], vt[4], gam, e3, p[6], rough, sph;
+    int neib[4], insurf;
+  };
+  EMC_HD EMC_INL void load_event(Event& v) const {
+    const EMC_GLB TetRec& r = B.tr[itet];
+    for (int f = 0; f < 4; ++f)
+      for (int q = 0; q < 4; ++q) v.n[f][q] = r.n[f][q];
+    for (int q = 0; q < 4; ++q) v.vt[q] = r.vt[q];
+    v.gam = r.gam;
+    v.e3 = r.e3;
+    for (int f = 0; f < 4; ++f) v.neib[f] = r.neib[f];
+    v.p[0] = M.lx[icell]; v.p[1] = M.lx[icell + 1];
+    v.p[2] = M.ly[jcell]; v.p[3] = M.ly[jcell + 1];
+    v.p[4] = M.lz[kcell]; v.p[5] = M.lz[kcell + 1];
+    v.insurf = 0;
+    v.rough = v.sph = 0;
+    if (M.flag_surface) {
+      const size_t c = cell(icell, jcell, kcell);
+      v.insurf = M.insurf[c];
+      if (par_type == PELEC) { v.rough = F.e_rough[c]; v.sph = F.e_sph[c]; }
+      else { v.rough = F.h_rough[c]; v.sph = F.h_sph[c]; }
+    }
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" ::: "memory");  // the reads stay above their uses
+#endif
+  }
   EMC_HD EMC_INL void GetEnergy() {
     double dx, dy, dz;
     in_wedge(dx, dy, dz, kx, ky, kz);
@@ -275,24 +305,20 @@ struct Flight {
   // the sphere array runs alongside the list, so most candidates cost 32 bytes
   // read in order instead of a dependent load of their record
   EMC_HD EMC_INL bool scan(const EMC_GLB int* list, const EMC_GLB Sphere* sph, int p0, int nn, double a, double b, double c) {
+    // eight sphere tests per round, their loads independent of each other; one
+    // copy of the exact test serves all eight
     const int end = p0 + nn;
-    int itl = p0;
-    // eight sphere tests per round, their loads independent of each other
-    for (; itl + 8 <= end; itl += 8) {
-      bool h[8];
+    for (int itl = p0; itl < end; itl += 8) {
+      uint32_t hit = 0;
 #pragma unroll
-      for (int u = 0; u < 8; ++u) h[u] = in_sphere(sph[itl + u], a, b, c);
-#pragma unroll
-      for (int u = 0; u < 8; ++u)
-        if (h[u]) {
-          const int it = list[itl + u];
-          if (iband == B.tr[it].ibt && contains(it, a, b, c)) { itet = it; return true; }
-        }
-    }
-    for (; itl < end; ++itl) {
-      if (!in_sphere(sph[itl], a, b, c)) continue;
-      const int it = list[itl];
-      if (iband == B.tr[it].ibt && contains(it, a, b, c)) { itet = it; return true; }
+      for (int u = 0; u < 8; ++u) {
+        const int q = itl + u < end ? itl + u : end - 1;
+        if (itl + u < end && in_sphere(sph[q], a, b, c)) hit |= 1u << u;
+      }
+      for (; hit; hit &= hit - 1) {
+        const int it = list[itl + __builtin_ctz(hit)];
+        if (iband == B.tr[it].ibt && contains(it, a, b, c)) { itet = it; return true; }
+      }
     }
     return false;
   }
@@ -367,17 +393,19 @@ struct Flight {
       }
       return;
     }
-    int ie = (int)(energy * B.dlists);
-    if (ie < 0) ie = 0;
-    if (ie < MWLES && scan(B.tlists, B.tlists_s, B.ptlists[ie * MNB + iband], B.ntlists[ie * MNB + iband], a, b, c)) return;
-    ie = (int)(energy * B.dlist);
+    // tlists bin, then tlist bins ie, ie+1, ie-1: one scan serves the four
+    const int ies = (int)(energy * B.dlists) < 0 ? 0 : (int)(energy * B.dlists);
+    int ie = (int)(energy * B.dlist);
     if (ie < 0) ie = 0;
     if (ie >= MWLE) ie = MWLE - 1;
-    if (scan(B.tlist, B.tlist_s, B.ptlist[ie * MNB + iband], B.ntlist[ie * MNB + iband], a, b, c)) return;
-    if (ie + 1 < MWLE && scan(B.tlist, B.tlist_s, B.ptlist[(ie + 1) * MNB + iband], B.ntlist[(ie + 1) * MNB + iband], a, b, c))
-      return;
-    if (ie - 1 >= 0 && scan(B.tlist, B.tlist_s, B.ptlist[(ie - 1) * MNB + iband], B.ntlist[(ie - 1) * MNB + iband], a, b, c))
-      return;
+    for (int q = 0; q < 4; ++q) {
+      const int bin = q == 0 ? ies : q == 1 ? ie : q == 2 ? ie + 1 : ie - 1;
+      if (bin < 0 || bin >= (q == 0 ? MWLES : MWLE)) continue;
+      const int at = bin * MNB + iband;
+      if (scan(q == 0 ? B.tlists : B.tlist, q == 0 ? B.tlists_s : B.tlist_s, q == 0 ? B.ptlists[at] : B.ptlist[at],
+               q == 0 ? B.ntlists[at] : B.ntlist[at], a, b, c))
+        return;
+    }
     for (int it = 0; it < B.nt; ++it)
       if (in_sphere(B.tsph[it], a, b, c) && iband == B.tr[it].ibt && contains(it, a, b, c)) { itet = it; return; }
     Flag_Catch = 1;
@@ -892,10 +920,26 @@ struct Flight {
     }
     int iscat = -1;
     double dscat = 0.0;
-    while (drand > dscat) {
-      iscat = iscat + 1;
-      if (iscat >= nmax) { Flag_SelfScatter = 1; break; }
-      dscat = dscat + process_rate(elec, iscat, itab, intp, where);
+    // the rates of the next processes are formed eight at a time, their reads
+    // together, then added one by one in the reference's order
+    constexpr int RB = 8;
+    for (int first = 0; drand > dscat; first += RB) {
+      double rate[RB];
+#pragma unroll
+      for (int q = 0; q < RB; ++q)
+        rate[q] = process_rate(elec, first + q < nmax ? first + q : nmax - 1, itab, intp, where);
+      bool go = true;
+#pragma unroll
+      for (int q = 0; q < RB; ++q)
+        if (go) {
+          iscat = first + q;
+          if (iscat >= nmax) { Flag_SelfScatter = 1; go = false; }
+          else {
+            dscat = dscat + rate[q];
+            go = drand > dscat;
+          }
+        }
+      if (!go) break;
     }
     if (Flag_SelfScatter) return POST_NONE;
     return prep_process(iscat, np, elec, s0);
@@ -921,8 +965,8 @@ struct Flight {
     }
     return 0.0;
   }
-  EMC_HD EMC_INL double GetImpScGamma() const {
-    const double e0 = B.tr[itet].vt[3], e3 = B.tr[itet].e3;
+  EMC_HD EMC_INL double GetImpScGamma(const Event& r) const {
+    const double e0 = r.vt[3], e3 = r.e3;
     const double eemax = M.frickel * 4 * PI * Rho / (8.0 * B.melt * M.eps_si);
     double gammax;
     if (eemax < e0) gammax = GetImpScRate(e0);
@@ -1110,11 +1154,10 @@ struct Flight {
   }
 
   // TetTime (src/TetHit.cpp:4-106)
-  EMC_HD EMC_INL double TetTime() {
+  EMC_HD EMC_INL double TetTime(const Event& r) {
     double xkl, ykl, zkl, xfl, yfl, zfl;
     in_wedge(xkl, ykl, zkl, kx, ky, kz);
     in_wedge(xfl, yfl, zfl, Ex, Ey, Ez);
-    const EMC_GLB TetRec& r = B.tr[itet];
     double best = 0.0;
     for (int f = 0; f < 4; ++f) {
       const double nf = r.n[f][0] * xfl + r.n[f][1] * yfl + r.n[f][2] * zfl;
@@ -1129,8 +1172,8 @@ struct Flight {
     return best;
   }
   // HitTet (src/TetHit.cpp:109-142)
-  EMC_HD EMC_INL void HitTet() {
-    const int nb = B.tr[itet].neib[itetdir];
+  EMC_HD EMC_INL void HitTet(const Event& r) {
+    const int nb = itetdir == 0 ? r.neib[0] : itetdir == 1 ? r.neib[1] : itetdir == 2 ? r.neib[2] : r.neib[3];
     if (nb >= 0) itet = nb;
     else if (nb == -5 || nb == -6) {
       const int ii = -nb - 2;
@@ -1145,17 +1188,17 @@ struct Flight {
       isym = B.newisym[(-nb - 2) * 48 + isym];
   }
   // CellTime (src/CellHit.cpp:4-93)
-  EMC_HD EMC_INL double CellTime() {
+  EMC_HD EMC_INL double CellTime(const Event& r) {
     int ix, iy, iz;
     double tx, ty, tz, t;
-    if (vx > 0) { ix = DOWN; tx = (M.lx[icell + 1] - x) / vx; }
-    else if (vx < 0) { ix = UP; tx = -(x - M.lx[icell]) / vx; }
+    if (vx > 0) { ix = DOWN; tx = (r.p[1] - x) / vx; }
+    else if (vx < 0) { ix = UP; tx = -(x - r.p[0]) / vx; }
     else { ix = UP; tx = 1e99; }
-    if (vy > 0) { iy = RIGHT; ty = (M.ly[jcell + 1] - y) / vy; }
-    else if (vy < 0) { iy = LEFT; ty = -(y - M.ly[jcell]) / vy; }
+    if (vy > 0) { iy = RIGHT; ty = (r.p[3] - y) / vy; }
+    else if (vy < 0) { iy = LEFT; ty = -(y - r.p[2]) / vy; }
     else { iy = RIGHT; ty = 1e99; }
-    if (vz > 0) { iz = BACK; tz = (M.lz[kcell + 1] - z) / vz; }
-    else if (vz < 0) { iz = FRONT; tz = -(z - M.lz[kcell]) / vz; }
+    if (vz > 0) { iz = BACK; tz = (r.p[5] - z) / vz; }
+    else if (vz < 0) { iz = FRONT; tz = -(z - r.p[4]) / vz; }
     else { iz = FRONT; tz = 1e99; }
     idir = ix; t = tx;
     if (ty < t) { idir = iy; t = ty; }
@@ -1164,7 +1207,7 @@ struct Flight {
     return t;
   }
 
-  // particle_fly (src/mcmodel.cpp:1874-2161), split into the parts the fast path reuses.
+  // particle_fly (src/mcmodel.cpp:1874-2161), in parts.
   struct Loop {
     bool getTet, getCell, getPh, getImp, getSurf;
     double ssnl, imprnl, phrnl, TetTf, CellTf;
@@ -1182,27 +1225,26 @@ struct Flight {
     iband = B.tr[itet].ibt;
   }
   // candidate times of the current iteration; returns the Min(...) flag and Tf
-  EMC_HD EMC_INL int next_event(Loop& L, double& Tf, double& gam, size_t& c) {
-    if (L.getTet) { L.TetTf = TetTime(); L.getTet = false; }
-    if (L.getCell) { L.CellTf = CellTime(); L.getCell = false; }
+  EMC_HD EMC_INL int next_event(Loop& L, const Event& r, double& Tf, double& gam) {
+    if (L.getTet) { L.TetTf = TetTime(r); L.getTet = false; }
+    if (L.getCell) { L.CellTf = CellTime(r); L.getCell = false; }
     if (L.getPh) { L.phrnl = -dm_log(Random()); L.getPh = false; }
-    gam = B.tr[itet].gam;
+    gam = r.gam;
     const double PhScTf = L.phrnl / gam;
     double ImpScTf;
     if (iband == B.bandofE) {
       if (L.getImp) { L.imprnl = -dm_log(Random()); L.getImp = false; }
-      ImpScGamma = GetImpScGamma();
+      ImpScGamma = GetImpScGamma(r);
       ImpScTf = L.imprnl / ImpScGamma;
     } else {
       ImpScTf = 2 * M.dt;
       ImpScGamma = 1.0 / M.scrt0;
     }
-    c = cell(icell, jcell, kcell);
     double SurfScTf;
-    if (M.flag_surface && M.insurf[c]) {
+    if (r.insurf) {
       if (L.getSurf) { L.ssnl = -dm_log(Random()); L.getSurf = false; }
-      if (par_type == PELEC) { SurfRoughnessScRate = F.e_rough[c]; SurfPhononScRate = F.e_sph[c]; }
-      else { SurfRoughnessScRate = F.h_rough[c]; SurfPhononScRate = F.h_sph[c]; }
+      SurfRoughnessScRate = r.rough;
+      SurfPhononScRate = r.sph;
       SurfScGamma = SurfRoughnessScRate + SurfPhononScRate;
       SurfScTf = (SurfScGamma > 0 && L.ssnl > 0) ? L.ssnl / SurfScGamma : 2 * M.dt;
     } else
@@ -1235,20 +1277,21 @@ struct Flight {
   // loop; post says whether a final state is drawn), get_state() follows when
   // post is set, then event_tail() (false: the particle was caught).
   EMC_HD EMC_INL bool event_head(Loop& L, int& flag, int& post, Saved& s0) {
-    GetV();
+    Event r;
+    load_event(r);
+    out_wedge(vx, vy, vz, r.vt[0], r.vt[1], r.vt[2]);  // GetV
     L.loop++;
     n_events++;
     if (L.loop > FLY_LOOP_CAP) { Flag_Catch = 1; drop_reason = 3; return false; }
     double Tf, gam;
-    size_t c;
-    flag = next_event(L, Tf, gam, c);
+    flag = next_event(L, r, Tf, gam);
     if (Tf < MY_ZERO) { Flag_Catch = 1; drop_reason = 0; return false; }
     advance(L, Tf, gam);
     if (energy < 0) { Flag_Catch = 1; drop_reason = 1; return false; }
     post = POST_NONE;
     switch (flag) {
       case 1:
-        HitTet();
+        HitTet(r);
         L.getTet = L.getCell = true;
         break;
       case 2: {
@@ -1269,7 +1312,7 @@ struct Flight {
       case 5:
         // ParticleSurfaceScatter (src/ParSurfaceScatter.cpp:48-61)
         if (Random() * SurfScGamma < SurfRoughnessScRate) {
-          idir = M.surface_dir[M.nearest_surf[c]];
+          idir = M.surface_dir[M.nearest_surf[cell(icell, jcell, kcell)]];
           post = prep_diffuse(s0);
         } else {
           Flag_SelfScatter = 0;
