@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <cmath>
 #include <cstdio>
@@ -141,6 +142,8 @@ struct Gpu {
   double *r = nullptr, *p = nullptr, *p2 = nullptr, *q = nullptr, *z = nullptr, *scal = nullptr;
   double *part_a = nullptr, *part_pq = nullptr, *part_rr = nullptr, *part_rz0 = nullptr, *part_rz1 = nullptr;
   int* done = nullptr;
+  XcdSync* sync = nullptr;            // the one-launch solve's words (zero between launches)
+  int xcd = 0, ncu = 0;               // the XCD this context's solves run on; CUs of the GPU
   MgArgs mg{};                        // device view of the multigrid hierarchy
   // FP32 copies for the bulk of the mixed-precision solve, made on its first use:
   // the level-0 operator, the hierarchy's vectors, damped inverse diagonals and
@@ -510,6 +513,10 @@ static int gpu_setup(emc_ctx* c) {
     int ncu = 0;
     if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, g.device) == hipSuccess && ncu > 0)
       g.wave_slots = 4LL * ncu;
+    g.ncu = ncu;
+    // contexts that run side by side solve on different XCDs
+    static std::atomic<unsigned> contexts{0};
+    g.xcd = (int)(contexts++ % 8);
   }
   for (auto& e : g.ev) HIPCHECK(c, hipEventCreate(&e));
   const Device& d = c->dev;
@@ -588,6 +595,7 @@ static int gpu_setup(emc_ctx* c) {
   for (double** pp : {&g.part_a, &g.part_pq, &g.part_rr, &g.part_rz0, &g.part_rz1}) *pp = m.alloc<double>(3 * g.pcg_blocks);
   g.scal = m.alloc<double>(8);
   g.done = m.alloc<int>(1);
+  g.sync = m.alloc<XcdSync>(1);
   {
     const std::string e = ensure_mg(c);
     if (!e.empty()) return fail(c, EMC_ERR_DECK, e);
@@ -618,6 +626,8 @@ static int gpu_setup(emc_ctx* c) {
   }
   if (m.last != hipSuccess) return fail(c, EMC_ERR_HIP, std::string("device allocation: ") + hipGetErrorString(m.last));
   HIPCHECK(c, hipMemset(g.pot, 0, NN * sizeof(double)));
+  HIPCHECK(c, hipMemset(g.sync, 0, sizeof(XcdSync)));
+  HIPCHECK(c, hipMemset(g.done, 0, sizeof(int)));
   HIPCHECK(c, hipMemset(g.tcount, 0, g.ntile * sizeof(unsigned)));
   HIPCHECK(c, hipMemset(g.toff, 0, (g.ntile + 1) * sizeof(unsigned)));
   HIPCHECK(c, hipHostMalloc((void**)&g.n_host, sizeof(unsigned), hipHostMallocDefault));
@@ -1340,6 +1350,7 @@ static FlyArgs fly_args(emc_ctx* c, uint64_t step, int flag_heat) {
   a.dead = g.dead; a.ndead = g.ctr + 1; a.dead_cap = g.dead_cap;
   a.slow = g.slow; a.nslow = g.ctr + 3;
   a.wave_slots = g.wave_slots;
+  a.gate = g.pcg_pending ? g.done : nullptr;  // a step whose solve the host has not seen yet
   return a;
 }
 
@@ -1550,6 +1561,10 @@ static int run_pcg(emc_ctx* c, const double* b, double* x, double rtol, int maxi
   return run_pcg_with(c, pcg_args(c, b, x, rtol), g.mg, rtol, maxit, iters, relres, defer);
 }
 
+// Whether the context's solves go in one launch on one XCD (k_pcg_xcd): meshes whose
+// solve is bound by its launches.
+static bool xcd_solve(const emc_ctx* c) { return c->dev.nnode <= XCD_MAX_NODES && c->gpu->ncu >= 8; }
+
 // The solve on explicit work vectors: `a` and `mg` name every buffer the
 // kernels write (the solve of the context uses its own, emc_poisson_solve_ws a
 // caller's workspace).
@@ -1557,10 +1572,26 @@ template <class PA, class MA>
 static int run_pcg_with(emc_ctx* c, const PA& a, const MA& mg, double rtol, int maxit, int* iters, double* relres,
                         bool defer) {
   Gpu& g = *c->gpu;
+  double* sh = g.scal_host;
+  if (xcd_solve(c)) {
+    XcdArgsT<typename PA::real, typename MA::real> w{};
+    w.a = a;
+    w.m = emc_mg_start_args(a, mg);
+    w.sync = g.sync;
+    w.maxit = maxit;
+    w.nmem = emc_xcd_blocks(a.n, 1, g.ncu);
+    w.xcd = g.xcd;
+    HIPCHECK(c, emc_launch_pcg_xcd(w, g.stream));
+    HIPCHECK(c, hipMemcpyAsync(sh, a.scal, 8 * sizeof(double), hipMemcpyDeviceToHost, g.stream));
+    g.pcg_result = sh;
+    g.pcg_pending = true;
+    if (defer) return EMC_OK;
+    HIPCHECK(c, hipStreamSynchronize(g.stream));
+    return finish_pcg(c, rtol, iters, relres);
+  }
   // k_pcg_begin sets done when the start already meets the tolerance: the
   // queued iterations are then no-ops and the first check below stops the loop
   HIPCHECK(c, emc_launch_pcg_start(a, mg, g.stream));
-  double* sh = g.scal_host;
   // Each check reads the residual of the iteration before the one just queued, so
   // the GPU never waits for the host; the iteration the previous solve converged in
   // is checked as soon as it is queued instead, so that a solve converging there
@@ -2589,7 +2620,8 @@ struct emc_batch {
   unsigned char* d_tab = nullptr;
   unsigned char* h_tab = nullptr;     // pinned host image of d_tab
   size_t off_sort = 0, off_dep = 0, off_pcg = 0, off_mg = 0, off_fmg = 0, off_field = 0, off_fly = 0, off_cp = 0,
-         tab_bytes = 0;
+         off_xcd = 0, tab_bytes = 0;
+  int nmem = 0;                        // blocks per device of the one-launch solve, 0: kernel by kernel
   BatchTables bt{};
   const CopyArgs *cp_n = nullptr, *cp_scal = nullptr, *cp_tally = nullptr, *cp_zero = nullptr;
   unsigned long long* d_n = nullptr;   // [K] live counts after the sort
@@ -2672,6 +2704,8 @@ static int batch_setup(emc_batch* b) {
   b->off_fmg = place(f32 ? 3 * K * sizeof(MgArgsT<float>) : 0);
   b->off_field = place(K * sizeof(FieldArgs));
   b->off_cp = place(5 * K * sizeof(CopyArgs));
+  b->nmem = xcd_solve(c0) ? emc_xcd_blocks(b->nnode, K, g0.ncu) : 0;
+  b->off_xcd = place(!b->nmem ? 0 : K * (f32 ? sizeof(XcdArgsT<double, float>) : sizeof(XcdArgsT<double, double>)));
   b->tab_bytes = off;
   b->d_tab = b->mem.alloc<unsigned char>(off);
   b->d_n = b->mem.alloc<unsigned long long>(K);
@@ -2698,6 +2732,8 @@ static int batch_setup(emc_batch* b) {
     b->bt.fmg_even = fm + K;
     b->bt.fmg_odd = fm + 2 * K;
   }
+  if (b->nmem && f32) b->bt.fxcd = (const XcdArgsT<double, float>*)(b->d_tab + b->off_xcd);
+  else if (b->nmem) b->bt.xcd = (const XcdArgsT<double, double>*)(b->d_tab + b->off_xcd);
   b->bt.field = (const FieldArgs*)(b->d_tab + b->off_field);
   const CopyArgs* cp = (const CopyArgs*)(b->d_tab + b->off_cp);
   b->cp_n = cp;
@@ -2724,6 +2760,18 @@ static int batch_setup(emc_batch* b) {
       hfm[q] = emc_mg_start_args(hp[q], g.pmg);
       hfm[K + q] = emc_mg_iter_args(hp[q], g.pmg, 0);
       hfm[2 * K + q] = emc_mg_iter_args(hp[q], g.pmg, 1);
+    }
+    if (b->nmem) {
+      auto fill = [&](auto* t, const auto& start) {
+        t[q].a = hp[q];
+        t[q].m = start;
+        t[q].sync = g.sync;
+        t[q].maxit = c->opts.poisson_maxit;
+        t[q].nmem = b->nmem;
+        t[q].xcd = q % 8;
+      };
+      if (f32) fill((XcdArgsT<double, float>*)(b->h_tab + b->off_xcd), hfm[q]);
+      else fill((XcdArgsT<double, double>*)(b->h_tab + b->off_xcd), hm[q]);
     }
     hf[q] = field_args(c, g.pot, true);
     int st = sync_fly_const(c);
@@ -2779,9 +2827,15 @@ static int batch_one_step(emc_batch* b, emc_fly_tallies* acc, double tsum[5], in
   BHIP(b, hipEventRecord(b->ev[1], s));
   // the solve: as run_pcg, one iteration of every device per launch; the host
   // checks the iteration before the one just queued, for all devices at once
-  BHIP(b, emc_launch_pcg_start_b(b->bt, b->shape, b->nblocks, s));
-  const int maxit = b->c[0]->opts.poisson_maxit;
   int checked = -1, last = -1;
+  if (b->nmem) {
+    BHIP(b, emc_launch_pcg_xcd_b(b->bt, b->nmem, s));
+    BHIP(b, emc_launch_copy_b(b->cp_scal, K, 8, s));
+    BHIP(b, hipMemcpyAsync(b->h_scal, b->d_scal, 8 * K * sizeof(double), hipMemcpyDeviceToHost, s));
+    last = 0;
+  } else
+    BHIP(b, emc_launch_pcg_start_b(b->bt, b->shape, b->nblocks, s));
+  const int maxit = b->nmem ? 0 : b->c[0]->opts.poisson_maxit;
   for (int k = 0; k < maxit; ++k) {
     last = k;
     BHIP(b, emc_launch_pcg_iter_b(b->bt, b->shape, b->nblocks, k, s));
@@ -2816,6 +2870,7 @@ static int batch_one_step(emc_batch* b, emc_fly_tallies* acc, double tsum[5], in
     g.sorted_n = g.n;
     g.n_pending = false;
     hfl[q] = fly_args(c, step[q], 0);
+    hfl[q].gate = b->nmem ? g.done : nullptr;
     nmax = std::max(nmax, g.n);
   }
   BHIP(b, hipMemcpyAsync(b->d_tab + b->off_fly, b->h_tab + b->off_fly, K * sizeof(FlyArgs), hipMemcpyHostToDevice, s));

@@ -35,6 +35,7 @@ struct FlyArgs {
   uint32_t* slow;              // [cap] particles k_fly_fast hands to k_fly_slow
   unsigned long long* nslow;   // device counter, zero before the flight
   long long wave_slots;        // waves the GPU runs at once (CUs x 4 SIMDs)
+  const int* gate;             // may be null; *gate == 2: the step's solve failed, nothing flies
 };
 
 // Deposit tiles: TILE_I x TILE_J x TILE_K cells (i, j, k) per workgroup; a tile's
@@ -201,6 +202,21 @@ struct MgArgsT {
 };
 using MgArgs = MgArgsT<double>;
 
+// The words by which the blocks of the one-launch solve (k_pcg_xcd) find together;
+// zero before a launch and left zero by it.
+struct XcdSync {
+  unsigned arrive, state, xcc, bar, leave, pad[11];
+};
+
+template <class RA, class RM>
+struct XcdArgsT {
+  PcgArgsT<RA> a;
+  MgArgsT<RM> m;  // m.z: the cycle's output
+  XcdSync* sync;
+  int maxit, nmem;  // nmem: blocks per device
+  int xcd, pad;     // the XCD they run on
+};
+
 // Iterative refinement of the mixed-precision solve: r = b - A x in FP64, its
 // FP32 copy is the right-hand side of the FP32 bulk solve, whose correction d is
 // added to x in FP64.
@@ -263,6 +279,9 @@ struct BatchTables {
   const MgArgsT<float> *fmg_start, *fmg_even, *fmg_odd;
   const FieldArgs* field;
   const FlyArgs* fly;
+  // the one-launch solve's tables (null: the solve goes kernel by kernel)
+  const XcdArgsT<double, double>* xcd;
+  const XcdArgsT<double, float>* fxcd;
 };
 
 }  // namespace emc
@@ -280,6 +299,19 @@ hipError_t emc_launch_pcg_iter(const emc::PcgArgsT<float>& a, const emc::MgArgsT
 hipError_t emc_launch_refine_resid(const emc::RefineArgs& r, hipStream_t s);
 hipError_t emc_launch_refine_add(const emc::RefineArgs& r, hipStream_t s);
 hipError_t emc_launch_zero_f32(float* p, size_t n, hipStream_t s);
+// The whole solve in one launch; blocks per device for K devices on a GPU of ncu CUs.
+// Up to XCD_MAX_NODES the solve is bound by its launches and goes in one (us per solve
+// kernel by kernel and in one launch, 6 to 7 iterations: 9.1 k nodes 385 and 250,
+// 11.2 k 368 and 270, 18.8 k 387 and 313; above, 32 CUs are too few: 69 k 489 and 574,
+// 96 k 576 and 715).  Eight devices of 11.2 k nodes in a batch: 413 and 312.
+namespace emc {
+constexpr size_t XCD_MAX_NODES = 32768;
+}
+int emc_xcd_blocks(size_t n, int K, int ncu);
+hipError_t emc_launch_pcg_xcd(const emc::XcdArgsT<double, double>& a, hipStream_t s);
+hipError_t emc_launch_pcg_xcd(const emc::XcdArgsT<double, float>& a, hipStream_t s);
+hipError_t emc_launch_pcg_xcd(const emc::XcdArgsT<float, float>& a, hipStream_t s);
+hipError_t emc_launch_pcg_xcd_b(const emc::BatchTables& t, int nmem, hipStream_t s);
 hipError_t emc_launch_pcg_start_b(const emc::BatchTables& t, const emc::MgArgs& shape, int nblocks, hipStream_t s);
 hipError_t emc_launch_pcg_iter_b(const emc::BatchTables& t, const emc::MgArgs& shape, int nblocks, int it,
                                  hipStream_t s);

@@ -93,6 +93,7 @@ __device__ inline void load_particle(Flight& f, const FlyArgs& a, long long q, u
 template <class AS>
 __global__ __launch_bounds__(256, 3) void k_fly_fast(AS as_) {
   const FlyArgs& a = kargs(as_);
+  if (a.gate && *a.gate == 2) return;  // no particle is listed, none flies
   const long long stride = (long long)gridDim.x * blockDim.x;
   long long ev = 0;
   const int lane = threadIdx.x & 63;
@@ -899,17 +900,16 @@ __device__ inline void mem_fence_compiler() {
   __builtin_amdgcn_sched_barrier(0);
 }
 
-template <class PA>
-__device__ inline double apply_op(const PA& a, const typename PA::real* __restrict__ x, size_t n, int i, int j,
-                                  int k) {
+template <class PA, class XA>
+__device__ inline double apply_op(const PA& a, const XA& x, size_t n, int i, int j, int k) {
   // every neighbour is loaded from a clamped address and a missing one adds 0.0,
   // so the loads carry no branches and issue together (the sum is the same, term
   // for term, as over the present neighbours only)
   const size_t sx = a.pnz, sy = (size_t)a.pnx * a.pnz;
   const bool ip = i + 1 < a.pnx, im = i > 0, jp = j + 1 < a.pny, jm = j > 0, kp = k + 1 < a.pnz, km = k > 0;
   const size_t nim = im ? n - sx : n, njm = jm ? n - sy : n, nkm = km ? n - 1 : n;
-  const double x0 = x[n], x1 = x[ip ? n + sx : n], x2 = x[nim], x3 = x[jp ? n + sy : n], x4 = x[njm],
-               x5 = x[kp ? n + 1 : n], x6 = x[nkm];
+  const double x0 = x(n), x1 = x(ip ? n + sx : n), x2 = x(nim), x3 = x(jp ? n + sy : n), x4 = x(njm),
+               x5 = x(kp ? n + 1 : n), x6 = x(nkm);
   const double c0 = a.diag[n], c1 = a.cx[n], c2 = a.cx[nim], c3 = a.cy[n], c4 = a.cy[njm], c5 = a.cz[n], c6 = a.cz[nkm];
   mem_fence_compiler();
   double v = c0 * x0;
@@ -1030,7 +1030,7 @@ __global__ __launch_bounds__(256) void k_pcg_resid(AS as_) {
   GRID_LOOP(n, a.n) {
     int i, j, k;
     node_ijk(a, n, i, j, k);
-    const double r = (double)a.b[n] - apply_op(a, a.x, n, i, j, k);
+    const double r = (double)a.b[n] - apply_op(a, [&](size_t q) -> double { return a.x[q]; }, n, i, j, k);
     a.r[n] = (R)r;
     if (a.r32) a.r32[n] = (float)r;
     rr += r * r;
@@ -1055,6 +1055,52 @@ __global__ __launch_bounds__(256) void k_pcg_begin(AS as_) {
   }
 }
 
+// A phase runs over the nodes of a level on the threads of a loop policy, which
+// also reads the vectors that other threads of the cycle write.
+struct GridLoop {
+  __device__ static size_t start() { return (size_t)blockIdx.x * blockDim.x + threadIdx.x; }
+  __device__ static size_t stride() { return (size_t)gridDim.x * blockDim.x; }
+  template <class R>
+  __device__ static R ld(const R* p) { return *p; }
+};
+
+// p and q = A p at node n, p.q added to pq.  z in the CG's precision, or the FP32
+// cycle's output.  Every neighbour is loaded from a clamped address and a missing
+// one adds 0.0, so the loads of a node issue together (as in apply_op).
+template <bool FIRST, class PA, class Z, class R, class LP>
+__device__ inline void spmvp_node(const PA& a, const Z* z, const R* p_in, R* p_out, double beta, size_t n, double& pq,
+                                  LP lp) {
+  const size_t sx = a.pnz, sy = (size_t)a.pnx * a.pnz;
+  int i, j, k;
+  node_ijk(a, n, i, j, k);
+  const bool ip = i + 1 < a.pnx, im = i > 0, jp = j + 1 < a.pny, jm = j > 0, kp = k + 1 < a.pnz, km = k > 0;
+  const size_t nb[7] = {n, ip ? n + sx : n, im ? n - sx : n, jp ? n + sy : n, jm ? n - sy : n,
+                        kp ? n + 1 : n, km ? n - 1 : n};
+  double zv[7], pv[7];
+#pragma unroll
+  for (int o = 0; o < 7; ++o) zv[o] = lp.ld(&z[nb[o]]);
+  if (!FIRST) {
+#pragma unroll
+    for (int o = 0; o < 7; ++o) pv[o] = lp.ld(&p_in[nb[o]]);
+  }
+  const double c0 = a.diag[n], c1 = a.cx[n], c2 = a.cx[nb[2]], c3 = a.cy[n], c4 = a.cy[nb[4]], c5 = a.cz[n],
+               c6 = a.cz[nb[6]];
+  mem_fence_compiler();
+  double p[7];
+#pragma unroll
+  for (int o = 0; o < 7; ++o) p[o] = FIRST ? zv[o] : zv[o] + beta * pv[o];
+  double q = c0 * p[0];
+  q += ip ? c1 * p[1] : 0.0;
+  q += im ? c2 * p[2] : 0.0;
+  q += jp ? c3 * p[3] : 0.0;
+  q += jm ? c4 * p[4] : 0.0;
+  q += kp ? c5 * p[5] : 0.0;
+  q += km ? c6 * p[6] : 0.0;
+  p_out[n] = (R)p[0];
+  a.q[n] = (R)q;
+  pq += p[0] * q;
+}
+
 // p = z + beta p_in (p = z in the first iteration), beta = r.z(new) / r.z(old),
 // then q = A p and the partial p.q.  p at the six neighbours is recomputed from
 // z and p_in with the same operations, so p_out is written once and p_in never
@@ -1077,43 +1123,10 @@ __global__ __launch_bounds__(256) void k_pcg_spmvp(AS as_, int it) {
     total_first2(rz_old, rz_new, a.nblocks, to, tn);
     beta = (to != 0.0) ? tn / to : 0.0;
   }
-  const size_t sx = a.pnz, sy = (size_t)a.pnx * a.pnz;
   double pq = 0;
-  // z in the CG's precision, or the FP32 cycle's output.  Every neighbour is
-  // loaded from a clamped address and a missing one adds 0.0, so the loads of a
-  // node issue together (as in apply_op).
   auto pass = [&](const auto* __restrict__ z, auto first_c) {
     constexpr bool FIRST = decltype(first_c)::value;
-    GRID_LOOP(n, a.n) {
-      int i, j, k;
-      node_ijk(a, n, i, j, k);
-      const bool ip = i + 1 < a.pnx, im = i > 0, jp = j + 1 < a.pny, jm = j > 0, kp = k + 1 < a.pnz, km = k > 0;
-      const size_t nb[7] = {n, ip ? n + sx : n, im ? n - sx : n, jp ? n + sy : n, jm ? n - sy : n,
-                            kp ? n + 1 : n, km ? n - 1 : n};
-      double zv[7], pv[7];
-#pragma unroll
-      for (int o = 0; o < 7; ++o) zv[o] = z[nb[o]];
-      if (!FIRST) {
-#pragma unroll
-        for (int o = 0; o < 7; ++o) pv[o] = p_in[nb[o]];
-      }
-      const double c0 = a.diag[n], c1 = a.cx[n], c2 = a.cx[nb[2]], c3 = a.cy[n], c4 = a.cy[nb[4]], c5 = a.cz[n],
-                   c6 = a.cz[nb[6]];
-      mem_fence_compiler();
-      double p[7];
-#pragma unroll
-      for (int o = 0; o < 7; ++o) p[o] = FIRST ? zv[o] : zv[o] + beta * pv[o];
-      double q = c0 * p[0];
-      q += ip ? c1 * p[1] : 0.0;
-      q += im ? c2 * p[2] : 0.0;
-      q += jp ? c3 * p[3] : 0.0;
-      q += jm ? c4 * p[4] : 0.0;
-      q += kp ? c5 * p[5] : 0.0;
-      q += km ? c6 * p[6] : 0.0;
-      p_out[n] = (R)p[0];
-      a.q[n] = (R)q;
-      pq += p[0] * q;
-    }
+    GRID_LOOP(n, a.n) spmvp_node<FIRST>(a, z, p_in, p_out, beta, n, pq, GridLoop());
   };
   using T1 = std::integral_constant<bool, true>;
   using T0 = std::integral_constant<bool, false>;
@@ -1154,10 +1167,6 @@ __global__ __launch_bounds__(256) void k_pcg_update(AS as_, int it) {
 // The phases of the cycle are written once per node (grid-stride loops, one
 // launch per phase).  A single workgroup walking the small levels was measured
 // slower (latency bound) than one launch per phase.
-struct GridLoop {
-  __device__ static size_t start() { return (size_t)blockIdx.x * blockDim.x + threadIdx.x; }
-  __device__ static size_t stride() { return (size_t)gridDim.x * blockDim.x; }
-};
 
 template <class LV>
 __device__ inline void lvl_ijk(const LV& L, size_t n, int& i, int& j, int& k) {
@@ -1219,46 +1228,46 @@ __device__ inline double mg_Ax(const MA& m, const LV& L, const XA& xa, size_t n,
 
 // t = x1 + wdinv (b - A x1) with x1 = wdinv b: two Jacobi sweeps from zero
 template <bool FINE, class LP, class MA, class LV>
-__device__ inline void ph_pre2(const MA& m, const LV& L) {
-  auto x1 = [&](size_t q) -> double { return (double)L.wdinv[q] * (double)L.b[q]; };
-  for (size_t n = LP::start(); n < L.n; n += LP::stride()) {
+__device__ inline void ph_pre2(const MA& m, const LV& L, LP lp) {
+  auto x1 = [&](size_t q) -> double { return (double)L.wdinv[q] * (double)lp.ld(&L.b[q]); };
+  for (size_t n = lp.start(); n < L.n; n += lp.stride()) {
     int i, j, k;
     lvl_ijk(L, n, i, j, k);
-    L.t[n] = x1(n) + (double)L.wdinv[n] * ((double)L.b[n] - mg_Ax<FINE>(m, L, x1, n, i, j, k));
+    L.t[n] = x1(n) + (double)L.wdinv[n] * ((double)lp.ld(&L.b[n]) - mg_Ax<FINE>(m, L, x1, n, i, j, k));
   }
 }
 
 // dst = src + wdinv (b - A src)
 template <bool FINE, class LP, class MA, class LV, class R>
-__device__ inline void ph_sweep(const MA& m, const LV& L, const R* src, R* dst) {
-  auto xs = [&](size_t q) -> double { return src[q]; };
-  for (size_t n = LP::start(); n < L.n; n += LP::stride()) {
+__device__ inline void ph_sweep(const MA& m, const LV& L, const R* src, R* dst, LP lp) {
+  auto xs = [&](size_t q) -> double { return lp.ld(&src[q]); };
+  for (size_t n = lp.start(); n < L.n; n += lp.stride()) {
     int i, j, k;
     lvl_ijk(L, n, i, j, k);
-    dst[n] = (double)src[n] + (double)L.wdinv[n] * ((double)L.b[n] - mg_Ax<FINE>(m, L, xs, n, i, j, k));
+    dst[n] = (double)lp.ld(&src[n]) + (double)L.wdinv[n] * ((double)lp.ld(&L.b[n]) - mg_Ax<FINE>(m, L, xs, n, i, j, k));
   }
 }
 
 // r = b - A t
 template <bool FINE, class LP, class MA, class LV>
-__device__ inline void ph_resid(const MA& m, const LV& L) {
-  auto xs = [&](size_t q) -> double { return L.t[q]; };
-  for (size_t n = LP::start(); n < L.n; n += LP::stride()) {
+__device__ inline void ph_resid(const MA& m, const LV& L, LP lp) {
+  auto xs = [&](size_t q) -> double { return lp.ld(&L.t[q]); };
+  for (size_t n = lp.start(); n < L.n; n += lp.stride()) {
     int i, j, k;
     lvl_ijk(L, n, i, j, k);
-    L.r[n] = (double)L.b[n] - mg_Ax<FINE>(m, L, xs, n, i, j, k);
+    L.r[n] = (double)lp.ld(&L.b[n]) - mg_Ax<FINE>(m, L, xs, n, i, j, k);
   }
 }
 
 // r = b - A x1 with x1 = wdinv b: one Jacobi sweep from zero and its residual
 // (levels >= 1: the restriction stored x1 in x)
 template <bool FINE, class LP, class MA, class LV>
-__device__ inline void ph_resid1(const MA& m, const LV& L) {
-  auto x1 = [&](size_t q) -> double { return L.x[q]; };
-  for (size_t n = LP::start(); n < L.n; n += LP::stride()) {
+__device__ inline void ph_resid1(const MA& m, const LV& L, LP lp) {
+  auto x1 = [&](size_t q) -> double { return lp.ld(&L.x[q]); };
+  for (size_t n = lp.start(); n < L.n; n += lp.stride()) {
     int i, j, k;
     lvl_ijk(L, n, i, j, k);
-    L.r[n] = (double)L.b[n] - mg_Ax<FINE>(m, L, x1, n, i, j, k);
+    L.r[n] = (double)lp.ld(&L.b[n]) - mg_Ax<FINE>(m, L, x1, n, i, j, k);
   }
 }
 
@@ -1269,8 +1278,8 @@ __device__ inline double pw1(int f, int C) { return f == 2 * C ? 1.0 : 0.5; }
 // also x_C = wdinv_C b_C, the first sweep from zero on the coarse level.  Fine
 // nodes off the mesh are read at a clamped address and add 0.0.
 template <class LP, class LV>
-__device__ inline void ph_restrict(const LV& F, const LV& C) {
-  for (size_t I = LP::start(); I < C.n; I += LP::stride()) {
+__device__ inline void ph_restrict(const LV& F, const LV& C, LP lp) {
+  for (size_t I = lp.start(); I < C.n; I += lp.stride()) {
     int ci, cj, ck;
     lvl_ijk(C, I, ci, cj, ck);
     double r[27];
@@ -1284,7 +1293,7 @@ __device__ inline void ph_restrict(const LV& F, const LV& C) {
           const int o = ((dj + 1) * 3 + (di + 1)) * 3 + (dk + 1);
           const int fj = 2 * cj + dj, fi = 2 * ci + di, fk = 2 * ck + dk;
           ok[o] = (unsigned)fj < (unsigned)F.ny && (unsigned)fi < (unsigned)F.nx && (unsigned)fk < (unsigned)F.nz;
-          r[o] = F.r[ok[o] ? ((size_t)fj * F.nx + fi) * F.nz + fk : 0];
+          r[o] = lp.ld(&F.r[ok[o] ? ((size_t)fj * F.nx + fi) * F.nz + fk : 0]);
         }
     mem_fence_compiler();
     double v = 0;
@@ -1308,9 +1317,9 @@ __device__ inline void ph_restrict(const LV& F, const LV& C) {
 // before the correction is the sweep from zero, t_F = wdinv b + P e (fixed
 // nodes 0).  Fine node f takes coarse node f/2 when f is even, (f-1)/2 and
 // (f+1)/2 with weight 1/2 each when odd; absent terms add 0.0.
-template <class LP, bool FROM_ZERO = false, class LV, class R>
-__device__ inline void ph_prolong(const LV& F, const LV& C, const R* e) {
-  for (size_t n = LP::start(); n < F.n; n += LP::stride()) {
+template <bool FROM_ZERO, class LP, class LV, class R>
+__device__ inline void ph_prolong(const LV& F, const LV& C, const R* e, LP lp) {
+  for (size_t n = lp.start(); n < F.n; n += lp.stride()) {
     const double wd = F.wdinv[n];
     if (wd == 0.0) {
       if (FROM_ZERO) F.t[n] = 0.0;
@@ -1329,7 +1338,7 @@ __device__ inline void ph_prolong(const LV& F, const LV& C, const R* e) {
 #pragma unroll
         for (int c = 0; c < 2; ++c) {
           const bool ok = okj[a] && oki[b] && okk[c];
-          ev[(a * 2 + b) * 2 + c] = e[ok ? ((size_t)cj[a] * C.nx + ci[b]) * C.nz + ck[c] : 0];
+          ev[(a * 2 + b) * 2 + c] = lp.ld(&e[ok ? ((size_t)cj[a] * C.nx + ci[b]) * C.nz + ck[c] : 0]);
         }
     mem_fence_compiler();
     double v = 0;
@@ -1342,8 +1351,8 @@ __device__ inline void ph_prolong(const LV& F, const LV& C, const R* e) {
         for (int c = 0; c < 2; ++c)
           v += (okj[a] && oki[b] && okk[c]) ? w * pw1(k, ck[c]) * ev[(a * 2 + b) * 2 + c] : 0.0;
       }
-    if (FROM_ZERO) F.t[n] = wd * (double)F.b[n] + v;
-    else F.t[n] = (double)F.t[n] + v;
+    if (FROM_ZERO) F.t[n] = wd * (double)lp.ld(&F.b[n]) + v;
+    else F.t[n] = (double)lp.ld(&F.t[n]) + v;
   }
 }
 
@@ -1351,8 +1360,8 @@ __device__ inline void ph_prolong(const LV& F, const LV& C, const R* e) {
 // the waves taking part.  A lane sums its columns lane, lane + 64, ... in that
 // order; the loads of eight of them are issued before the first multiply, so a
 // row costs a few memory round trips instead of one per 64 columns.
-template <class MA, class R>
-__device__ inline void ph_coarse(const MA& m, const R* in, R* out, size_t wave, size_t nwaves) {
+template <class LP, class MA, class R>
+__device__ inline void ph_coarse(const MA& m, const R* in, R* out, size_t wave, size_t nwaves, LP lp) {
   const int nc = m.nc;
   const int lane = threadIdx.x & 63;
   constexpr int U = 8;
@@ -1365,12 +1374,12 @@ __device__ inline void ph_coarse(const MA& m, const R* in, R* out, size_t wave, 
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         rv[u] = row[c + 64 * u];
-        xv[u] = in[c + 64 * u];
+        xv[u] = lp.ld(&in[c + 64 * u]);
       }
 #pragma unroll
       for (int u = 0; u < U; ++u) v += rv[u] * xv[u];
     }
-    for (; c < nc; c += 64) v += (double)row[c] * (double)in[c];
+    for (; c < nc; c += 64) v += (double)row[c] * (double)lp.ld(&in[c]);
     v = wave_sum(v);
     if (lane == 0) out[r] = v;
   }
@@ -1403,14 +1412,14 @@ __global__ __launch_bounds__(256) void k_mg_pre2(AS ms_) {
   using R = typename std::decay_t<decltype(m)>::real;
   if (*m.done) return;
   book_residual(m);
-  ph_pre2<true, GridLoop>(m, m.L[0]);
+  ph_pre2<true>(m, m.L[0], GridLoop());
 }
 template <class AS>
 __global__ __launch_bounds__(256) void k_mg_resid(AS ms_) {
   const auto& m = kargs(ms_);
   using R = typename std::decay_t<decltype(m)>::real;
   if (*m.done) return;
-  ph_resid<true, GridLoop>(m, m.L[0]);
+  ph_resid<true>(m, m.L[0], GridLoop());
 }
 // levels >= 1: sweep from zero and residual in one pass
 template <class AS>
@@ -1418,28 +1427,28 @@ __global__ __launch_bounds__(256) void k_mg_resid1(AS ms_, int l) {
   const auto& m = kargs(ms_);
   using R = typename std::decay_t<decltype(m)>::real;
   if (*m.done) return;
-  ph_resid1<false, GridLoop>(m, m.L[l]);
+  ph_resid1<false>(m, m.L[l], GridLoop());
 }
 template <class AS>
 __global__ __launch_bounds__(256) void k_mg_restrict(AS ms_, int l) {
   const auto& m = kargs(ms_);
   using R = typename std::decay_t<decltype(m)>::real;
   if (*m.done) return;
-  ph_restrict<GridLoop>(m.L[l], m.L[l + 1]);
+  ph_restrict(m.L[l], m.L[l + 1], GridLoop());
 }
 template <class AS>
 __global__ __launch_bounds__(256) void k_mg_prolong(AS ms_) {
   const auto& m = kargs(ms_);
   using R = typename std::decay_t<decltype(m)>::real;
   if (*m.done) return;
-  ph_prolong<GridLoop>(m.L[0], m.L[1], mg_result(m, 1));
+  ph_prolong<false>(m.L[0], m.L[1], mg_result(m, 1), GridLoop());
 }
 template <class AS>
 __global__ __launch_bounds__(256) void k_mg_prolong1(AS ms_, int l) {
   const auto& m = kargs(ms_);
   using R = typename std::decay_t<decltype(m)>::real;
   if (*m.done) return;
-  ph_prolong<GridLoop, true>(m.L[l], m.L[l + 1], mg_result(m, l + 1));
+  ph_prolong<true>(m.L[l], m.L[l + 1], mg_result(m, l + 1), GridLoop());
 }
 // levels >= 1: one sweep t -> x
 template <class AS>
@@ -1447,14 +1456,14 @@ __global__ __launch_bounds__(256) void k_mg_post1(AS ms_, int l) {
   const auto& m = kargs(ms_);
   using R = typename std::decay_t<decltype(m)>::real;
   if (*m.done) return;
-  ph_sweep<false, GridLoop>(m, m.L[l], m.L[l].t, m.L[l].x);
+  ph_sweep<false>(m, m.L[l], m.L[l].t, m.L[l].x, GridLoop());
 }
 template <class AS>
 __global__ __launch_bounds__(256) void k_mg_post0a(AS ms_) {
   const auto& m = kargs(ms_);
   using R = typename std::decay_t<decltype(m)>::real;
   if (*m.done) return;
-  ph_sweep<true, GridLoop>(m, m.L[0], m.L[0].t, m.L[0].x);
+  ph_sweep<true>(m, m.L[0], m.L[0].t, m.L[0].x, GridLoop());
 }
 
 // last sweep of level 0 into z, with the partial r.z of the CG (r = b of level 0)
@@ -1486,7 +1495,7 @@ __global__ __launch_bounds__(256) void k_mg_coarse(AS ms_) {
   using R = typename std::decay_t<decltype(m)>::real;
   if (*m.done) return;
   const auto& L = m.L[m.nl - 1];
-  ph_coarse(m, L.b, L.x, ((size_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6, ((size_t)gridDim.x * blockDim.x) >> 6);
+  ph_coarse(m, L.b, L.x, GridLoop::start() >> 6, GridLoop::stride() >> 6, GridLoop());
 }
 
 // single-level hierarchy: z = C^-1 r over the grid, then the partial r.z
@@ -1497,7 +1506,7 @@ __global__ __launch_bounds__(256) void k_mg_coarse_z(AS ms_) {
   R* z = m.z;
   if (*m.done) return;
   book_residual(m);
-  ph_coarse(m, m.L[0].b, z, ((size_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6, ((size_t)gridDim.x * blockDim.x) >> 6);
+  ph_coarse(m, m.L[0].b, z, GridLoop::start() >> 6, GridLoop::stride() >> 6, GridLoop());
 }
 template <class AS>
 __global__ __launch_bounds__(256) void k_mg_dot_rz(AS ms_) {
@@ -1510,6 +1519,267 @@ __global__ __launch_bounds__(256) void k_mg_dot_rz(AS ms_) {
   double rz = 0;
   for (size_t n = GridLoop::start(); n < L.n; n += GridLoop::stride()) rz += (double)L.b[n] * (double)z[n];
   block_reduce1(rz, part_rz);
+}
+
+// ------------------------------------------------------------------ the solve on one XCD
+// The whole solve in one launch for meshes whose kernels are bound by their launches:
+// a phase of the 11 k-node mesh takes 3 to 5 us as a kernel of its own, nearly all of
+// it the launch, and a solve is about a hundred of them.  Here the blocks of one XCD
+// (one per CU) walk the phases together with a barrier of their own after each
+// (about 1.2 us with the phase's first reads): they share an L2, so data another
+// block wrote is seen once its store has reached the L2 and the read passes the L1
+// by (XcdLoop::ld).  The same operations in the same order as the kernels above,
+// down to the partial sums of 256 threads, so the two forms agree bit for bit.
+//
+// Which blocks: workgroups go to the XCDs in turn, so of XCD_COUNT * nmem blocks every
+// XCD_COUNT-th lands on one XCD.  Those are the candidates; the others leave at once.
+// The candidates check that they do share an XCD and wait until all have arrived;
+// if they do not (another placement, or the GPU held by other work for XCD_GATHER
+// ticks), the first candidate solves alone, which needs no one.  Once all are
+// resident each runs to its end, so the barriers' waits end; they are bounded all
+// the same (XCD_SPIN) and a bound reached fails the solve.
+constexpr int XCD_COUNT = 8, XCD_THREADS = 512;
+constexpr long long XCD_GATHER = 2000000, XCD_SPIN = 20000000;  // 20 ms and 0.2 s of the 100 MHz clock
+enum { XCD_OPEN = 0, XCD_GO = 1, XCD_ALONE = 2 };
+
+template <class T>
+__device__ __forceinline__ T ld_l2(const T* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+struct XcdLoop {
+  size_t first, step;
+  __device__ size_t start() const { return first; }
+  __device__ size_t stride() const { return step; }
+  template <class R>
+  __device__ R ld(const R* p) const { return ld_l2(p); }
+};
+
+struct XcdTeam {
+  XcdSync* s;
+  int nmem, me;
+  unsigned epoch;
+  double (*sh)[4];  // [4][4] block sums
+  int* dead;        // shared: a wait ran into its bound
+  int flip;
+
+  // every store of the team before it is seen by the team's reads after it
+  __device__ void barrier() {
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (nmem > 1) {
+      if (threadIdx.x == 0 && !*dead) {
+        const unsigned want = ++epoch * (unsigned)nmem;
+        __hip_atomic_fetch_add(&s->bar, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (ld_l2(&s->bar) < want) {
+          const long long t0 = wall_clock64();
+          while (ld_l2(&s->bar) < want)
+            if (wall_clock64() - t0 > XCD_SPIN) {
+              *dead = 1;
+              break;
+            }
+        }
+      }
+      __syncthreads();
+    }
+    asm volatile("" ::: "memory");
+  }
+  // block_reduce1's partial of virtual block vb (256 threads, half of this block)
+  __device__ void partial(double v, int vb, int nb, double* part, int pstride) {
+    double* b = sh[2 * flip + (threadIdx.x >> 8)];
+    flip ^= 1;
+    v = wave_sum(v);
+    if ((threadIdx.x & 63) == 0) b[(threadIdx.x >> 6) & 3] = v;
+    __syncthreads();
+    if ((threadIdx.x & 255) == 0 && vb < nb) {
+      double t = 0;
+      for (int q = 0; q < 4; ++q) t += b[q];
+      part[(size_t)vb * pstride] = t;
+    }
+  }
+  // total1 of two partial arrays, one per half of the block
+  __device__ void totals(const double* pa, const double* pb, int pstride, int nb, double& ta, double& tb) {
+    const double* p = threadIdx.x < 256 ? pa : pb;
+    double* b = sh[2 * flip + (threadIdx.x >> 8)];
+    double v = 0;
+    for (int q = threadIdx.x & 255; q < nb; q += 256) v += ld_l2(&p[(size_t)q * pstride]);
+    v = wave_sum(v);
+    if ((threadIdx.x & 63) == 0) b[(threadIdx.x >> 6) & 3] = v;
+    __syncthreads();
+    ta = tb = 0;
+    for (int q = 0; q < 4; ++q) { ta += sh[2 * flip][q]; tb += sh[2 * flip + 1][q]; }
+    flip ^= 1;
+  }
+};
+
+// f(n, acc) over the nodes of each virtual block of 256 threads as GRID_LOOP gives
+// them to it, then the block's partial
+template <class F>
+__device__ __forceinline__ void xcd_reduce(XcdTeam& t, size_t n, int nb, double* part, F f) {
+  const int sub = threadIdx.x >> 8, th = threadIdx.x & 255;
+  for (int v0 = 2 * t.me; v0 < nb; v0 += 2 * t.nmem) {
+    const int vb = v0 + sub;
+    double acc = 0;
+    if (vb < nb)
+      for (size_t q = (size_t)vb * 256 + th; q < n; q += (size_t)nb * 256) f(q, acc);
+    t.partial(acc, vb, nb, part, 1);
+  }
+}
+
+// z = M r and its partials r.z (launch_vcycle's phases)
+template <class MA>
+__device__ __forceinline__ void xcd_cycle(XcdTeam& t, const MA& m, XcdLoop lp, double* part_rz, int nb) {
+  using R = typename MA::real;
+  const auto& L0 = m.L[0];
+  if (m.nl == 1) {
+    ph_coarse(m, L0.b, m.z, lp.first >> 6, lp.step >> 6, lp);
+    t.barrier();
+    xcd_reduce(t, L0.n, nb, part_rz,
+               [&](size_t q, double& acc) { acc += (double)lp.ld(&L0.b[q]) * (double)lp.ld(&m.z[q]); });
+    t.barrier();
+    return;
+  }
+  ph_pre2<true>(m, L0, lp);
+  t.barrier();
+  ph_resid<true>(m, L0, lp);
+  t.barrier();
+  ph_restrict(L0, m.L[1], lp);
+  t.barrier();
+  for (int l = 1; l < m.nl - 1; ++l) {
+    ph_resid1<false>(m, m.L[l], lp);
+    t.barrier();
+    ph_restrict(m.L[l], m.L[l + 1], lp);
+    t.barrier();
+  }
+  ph_coarse(m, m.L[m.nl - 1].b, m.L[m.nl - 1].x, lp.first >> 6, lp.step >> 6, lp);
+  t.barrier();
+  for (int l = m.nl - 2; l > 0; --l) {
+    ph_prolong<true>(m.L[l], m.L[l + 1], mg_result(m, l + 1), lp);
+    t.barrier();
+    ph_sweep<false>(m, m.L[l], m.L[l].t, m.L[l].x, lp);
+    t.barrier();
+  }
+  ph_prolong<false>(L0, m.L[1], mg_result(m, 1), lp);
+  t.barrier();
+  ph_sweep<true>(m, L0, L0.t, L0.x, lp);
+  t.barrier();
+  // k_mg_sweep_last
+  const R* src = L0.x;
+  auto xs = [&](size_t q) -> double { return lp.ld(&src[q]); };
+  xcd_reduce(t, L0.n, nb, part_rz, [&](size_t q, double& acc) {
+    int i, j, k;
+    lvl_ijk(L0, q, i, j, k);
+    const double b = lp.ld(&L0.b[q]);
+    const double v = xs(q) + (double)L0.wdinv[q] * (b - mg_Ax<true>(m, L0, xs, q, i, j, k));
+    m.z[q] = (R)v;
+    acc += b * v;
+  });
+  t.barrier();
+}
+
+template <class AS>
+__global__ __launch_bounds__(XCD_THREADS) void k_pcg_xcd(AS as_) {
+  const auto& w = kargs(as_);
+  const auto& a = w.a;
+  const auto& m = w.m;
+  using RA = typename std::decay_t<decltype(a)>::real;
+  __shared__ double sh[4][4];
+  __shared__ int s_state, dead;
+  const int nmem = w.nmem;
+  const unsigned lane8 = (blockIdx.x + XCD_COUNT - (unsigned)w.xcd) % XCD_COUNT;
+  if (lane8 != 0) return;
+  const int me = blockIdx.x / XCD_COUNT;
+  XcdSync* s = w.sync;
+  if (threadIdx.x == 0) {
+    dead = 0;
+    // HW_REG_XCC_ID, bits 0-3
+    const unsigned xcc = ((unsigned)__builtin_amdgcn_s_getreg((3 << 11) | 20) & 15u) + 1u;
+    const unsigned old = atomicCAS(&s->xcc, 0u, xcc);
+    if (old != 0u && old != xcc) atomicCAS(&s->state, (unsigned)XCD_OPEN, (unsigned)XCD_ALONE);
+    if (atomicAdd(&s->arrive, 1u) + 1u == (unsigned)nmem)
+      atomicCAS(&s->state, (unsigned)XCD_OPEN, (unsigned)XCD_GO);
+    const long long t0 = wall_clock64();
+    unsigned st;
+    while ((st = ld_l2(&s->state)) == XCD_OPEN)
+      if (wall_clock64() - t0 > XCD_GATHER) atomicCAS(&s->state, (unsigned)XCD_OPEN, (unsigned)XCD_ALONE);
+    s_state = (int)st;
+  }
+  __syncthreads();
+  const bool alone = s_state == XCD_ALONE;
+  if (!alone || me == 0) {
+    XcdTeam t{s, alone ? 1 : nmem, me, 0u, sh, &dead, 0};
+    const XcdLoop lp{(size_t)me * XCD_THREADS + threadIdx.x, (size_t)t.nmem * XCD_THREADS};
+    const int nb = a.nblocks;
+    const RA* ax = a.x;
+    // k_pcg_fix, k_pcg_resid
+    for (size_t n = lp.start(); n < a.n; n += lp.stride())
+      if (a.kind[n] != 0) a.x[n] = a.b[n];
+    t.barrier();
+    {
+      auto resid = [&](size_t n) -> double {
+        int i, j, k;
+        node_ijk(a, n, i, j, k);
+        return (double)a.b[n] - apply_op(a, [&](size_t q) -> double { return lp.ld(&ax[q]); }, n, i, j, k);
+      };
+      xcd_reduce(t, a.n, nb, a.part_a, [&](size_t n, double& acc) {
+        const double r = resid(n);
+        a.r[n] = (RA)r;
+        if (a.r32) a.r32[n] = (float)r;
+        acc += r * r;
+      });
+      xcd_reduce(t, a.n, nb, a.part_a + nb,
+                 [&](size_t n, double& acc) { acc += (double)a.b[n] * (double)a.b[n]; });
+    }
+    t.barrier();
+    xcd_cycle(t, m, lp, a.part_rz0, nb);
+    // k_pcg_begin
+    double rr, bb, rz, rz_prev = 0, pq, unused;
+    t.totals(a.part_a, a.part_a + nb, 1, nb, rr, bb);
+    t.totals(a.part_rz0, a.part_rz0, 1, nb, rz, unused);
+    const double tol = a.rtol * a.rtol * bb;
+    int it = 0;
+    for (; !(rr <= tol) && it < w.maxit && !dead && isfinite(rr); ++it) {
+      double* rz_out = (it & 1) ? a.part_rz0 : a.part_rz1;
+      RA* p_out = (it & 1) ? a.p2 : a.p;
+      const RA* p_in = (it & 1) ? a.p : a.p2;
+      const double beta = it == 0 ? 0.0 : (rz_prev != 0.0) ? rz / rz_prev : 0.0;
+      auto spmvp = [&](const auto* z) {
+        xcd_reduce(t, a.n, nb, a.part_pq, [&](size_t n, double& acc) {
+          if (it == 0) spmvp_node<true>(a, z, p_in, p_out, beta, n, acc, lp);
+          else spmvp_node<false>(a, z, p_in, p_out, beta, n, acc, lp);
+        });
+      };
+      spmvp((const typename std::decay_t<decltype(m)>::real*)m.z);
+      t.barrier();
+      // k_pcg_update
+      t.totals(a.part_pq, a.part_pq, 1, nb, pq, unused);
+      const double alpha = (pq != 0.0) ? rz / pq : 0.0;
+      const RA* p = p_out;
+      xcd_reduce(t, a.n, nb, a.part_rr, [&](size_t n, double& acc) {
+        a.x[n] = (RA)((double)lp.ld(&a.x[n]) + alpha * (double)lp.ld(&p[n]));
+        const double r = (double)lp.ld(&a.r[n]) - alpha * (double)lp.ld(&a.q[n]);
+        a.r[n] = (RA)r;
+        if (a.r32) a.r32[n] = (float)r;
+        acc += r * r;
+      });
+      t.barrier();
+      t.totals(a.part_rr, a.part_rr, 1, nb, rr, unused);
+      if (rr <= tol || !isfinite(rr)) { ++it; break; }
+      xcd_cycle(t, m, lp, rz_out, nb);
+      rz_prev = rz;
+      t.totals(rz_out, rz_out, 1, nb, rz, unused);
+    }
+    if (me == 0 && threadIdx.x == 0) {
+      a.scal[0] = rr; a.scal[1] = rz; a.scal[2] = bb; a.scal[3] = it; a.scal[4] = tol;
+      *a.done = dead || !isfinite(rr) ? 2 : 1;  // 2: the step's flight is not to run
+    }
+    if (dead && threadIdx.x == 0) a.scal[0] = __builtin_nan("");
+  }
+  // the last candidate leaves the words as the next launch needs them
+  __syncthreads();
+  if (threadIdx.x == 0 && atomicAdd(&s->leave, 1u) + 1u == (unsigned)nmem) {
+    s->arrive = 0; s->state = XCD_OPEN; s->xcc = 0; s->bar = 0; s->leave = 0;
+  }
 }
 
 // ------------------------------------------------------------------ initial population
@@ -1560,7 +1830,7 @@ __global__ __launch_bounds__(256) void k_refine_resid(RefineArgs ra) {
   GRID_LOOP(n, a.n) {
     int i, j, k;
     node_ijk(a, n, i, j, k);
-    const double r = a.kind[n] != 0 ? 0.0 : a.b[n] - apply_op(a, a.x, n, i, j, k);
+    const double r = a.kind[n] != 0 ? 0.0 : a.b[n] - apply_op(a, [&](size_t q) -> double { return a.x[q]; }, n, i, j, k);
     a.r[n] = r;
     ra.r32[n] = (float)r;
     rr += r * r;
@@ -1802,6 +2072,32 @@ hipError_t emc_launch_pcg_iter(const PcgArgsT<float>& a, const MgArgsT<float>& m
 }
 hipError_t emc_launch_pcg_iter(const PcgArgs& a, const MgArgsT<float>& m, int it, hipStream_t s) {
   return launch_pcg_iter(a, m, it, s);
+}
+
+// ---- the solve in one launch
+// One block per node thread, shared CUs divided among the devices of an XCD (us a
+// solve, 11.2 k nodes: 8 blocks 368, 16 317, 24 270, 32 285; 16 devices: 16 blocks
+// each 377, 32 614, 8 427).
+int emc_xcd_blocks(size_t n, int K, int ncu) {
+  const int cus = ncu / XCD_COUNT > 1 ? ncu / XCD_COUNT : 1;   // of one XCD
+  const int per = (K + XCD_COUNT - 1) / XCD_COUNT;              // devices that share it
+  const int most = cus / per > 4 ? cus / per : cus < 4 ? cus : 4;
+  const size_t want = (n + XCD_THREADS - 1) / XCD_THREADS;      // a node a thread
+  return want < (size_t)most ? (int)want : most;
+}
+template <class A>
+static hipError_t launch_pcg_xcd(const A& a, hipStream_t s) {
+  hipLaunchKernelGGL(k_pcg_xcd<A>, dim3(XCD_COUNT * a.nmem), dim3(XCD_THREADS), 0, s, a);
+  return hipGetLastError();
+}
+hipError_t emc_launch_pcg_xcd(const XcdArgsT<double, double>& a, hipStream_t s) { return launch_pcg_xcd(a, s); }
+hipError_t emc_launch_pcg_xcd(const XcdArgsT<double, float>& a, hipStream_t s) { return launch_pcg_xcd(a, s); }
+hipError_t emc_launch_pcg_xcd(const XcdArgsT<float, float>& a, hipStream_t s) { return launch_pcg_xcd(a, s); }
+hipError_t emc_launch_pcg_xcd_b(const BatchTables& t, int nmem, hipStream_t s) {
+  const dim3 g(XCD_COUNT * nmem, (unsigned)t.K);
+  if (t.fxcd) hipLaunchKernelGGL((k_pcg_xcd<const XcdArgsT<double, float>*>), g, dim3(XCD_THREADS), 0, s, t.fxcd);
+  else hipLaunchKernelGGL((k_pcg_xcd<const XcdArgsT<double, double>*>), g, dim3(XCD_THREADS), 0, s, t.xcd);
+  return hipGetLastError();
 }
 
 // ---- iterative refinement of the mixed-precision solve
