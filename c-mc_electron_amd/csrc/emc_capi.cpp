@@ -657,6 +657,10 @@ static int gpu_setup(emc_ctx* c) {
     a.pnx = d.pnx; a.pny = d.pny; a.pnz = d.pnz;
     a.qnodes = m.dup(q.qnodes);
     a.flag = m.dup(q.flag);
+    a.nchunk = (int)q.chunks.size();
+    a.chunks = m.dup(q.chunks);
+    a.shape = m.dup(q.shape);
+    a.row_shape = m.dup(q.row_shape);
     for (int ax = 0; ax < 3; ++ax) {
       a.wlen[ax] = q.wlen[ax];
       a.lo[ax] = m.dup(q.lo[ax]);

@@ -5,6 +5,7 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include "qc.h"
 #include "tables.h"
 
 namespace emc {
@@ -100,6 +101,9 @@ struct QcArgs {
   int pnx, pny, pnz;
   int wlen[3];                              // window length per axis (table row stride)
   const int* qnodes;                        // [nq] node indices
+  const QcChunk* chunks;                    // [nchunk] blocks of targets (nchunk 0: a lane per node, no staging)
+  int nchunk, pad0;
+  const uint8_t *shape, *row_shape;         // QcTables::shape, row_shape
   const uint16_t* flag;                     // [nnode] init_p_mat flags
   const int* lo[3];                         // per axis: window start of each target index
   const int* hi[3];                         // per axis: window end (inclusive)

@@ -797,9 +797,9 @@ __global__ __launch_bounds__(256) void k_deposit_gather(AS as_) {
 // One lane per node of the quantum region; the window's sources are read in the
 // reference's loop order (i, then j, then k) and every term is formed as
 // ((V + Eb) * wz) * wy * wx, so the sum is the oracle's to the last bit.
-// Neighbouring lanes are neighbouring nodes (k fastest) whose windows overlap
-// almost entirely: the loads are served by L2.
-__global__ __launch_bounds__(256) void k_qc_potential(QcArgs a) {
+// Reads every term's five words from memory; only for windows that do not fit a
+// block's LDS (k_qc_potential).
+__global__ __launch_bounds__(256) void k_qc_potential_nodes(QcArgs a) {
   const long long stride = (long long)gridDim.x * blockDim.x;
   for (long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x; q < a.nq; q += stride) {
     const int p = a.qnodes[q];
@@ -831,6 +831,127 @@ __global__ __launch_bounds__(256) void k_qc_potential(QcArgs a) {
   }
 }
 
+
+// The same sum, a block per chunk of up to 128 targets of one i plane, two lanes a
+// target.  Per source plane i the block stages the potential (0 where nothing is
+// summed: the term then adds a zero) and the shapes of the chunk's union window in
+// LDS, the next plane's loads issued before the current one is summed; the chunk's j
+// and k weights stay in LDS throughout.  The two lanes of a target form consecutive
+// terms, hand them over (quad permutes) and both add them in the order of the sum
+// above: only the additions are a serial chain.
+// Bound by the latency of its LDS reads and of that chain.  60 k targets of the
+// 60 x 120 x 36-cell device: a lane per node that read five words per term through
+// L1 785 us, a lane per target from LDS 221, two lanes 196, four lanes 263 (more
+// vector instructions); 40 x 72 x 22 cells 326 and 80 us.
+template <int CTRL>
+__device__ __forceinline__ double quad_get(double v) {  // v of the lane that the quad permute CTRL names
+  const uint64_t u = __builtin_bit_cast(uint64_t, v);
+  const int lo = __builtin_amdgcn_mov_dpp((int)(uint32_t)u, CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_mov_dpp((int)(uint32_t)(u >> 32), CTRL, 0xf, 0xf, true);
+  return __builtin_bit_cast(double, ((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo);
+}
+constexpr int QC_THREADS = 2 * QC_CHUNK;
+__global__ __launch_bounds__(QC_THREADS) void k_qc_potential(QcArgs a) {
+  __shared__ double v[2][QC_PLANE];
+  __shared__ uint8_t sh[2][QC_PLANE];
+  __shared__ double wt[QC_TABLE];
+  const QcChunk c = a.chunks[blockIdx.x];
+  const int tid = threadIdx.x, tgt = tid >> 1, g = tid & 1;
+  const bool on = tgt < c.count;
+  const int p = a.qnodes[c.start + (on ? tgt : 0)];
+  const int pk = p % a.pnz, pj = p / a.pnz / a.pnx;
+  // a k row of weights is one word longer in LDS, so that the targets' rows start on
+  // different banks
+  const int lz = 4 * a.wlen[2], ny = 4 * c.ntj * a.wlen[1], nz = c.ntk * lz;
+  for (int e = tid; e < ny; e += QC_THREADS) wt[e] = a.w[1][(size_t)c.tj0 * a.wlen[1] * 4 + e];
+  for (int e = tid; e < nz; e += QC_THREADS) wt[ny + e + e / lz] = a.w[2][(size_t)c.tk0 * lz + e];
+  const double* WY = wt + 4 * (pj - c.tj0) * a.wlen[1];
+  const double* WZ = wt + ny + (pk - c.tk0) * (lz + 1);
+  const double* WX = a.w[0] + (size_t)c.pi * a.wlen[0] * 4;
+  const int i0 = a.lo[0][c.pi], i1 = a.hi[0][c.pi];
+  const int j0 = a.lo[1][pj], j1 = on ? a.hi[1][pj] : j0 - 1;
+  const int k0 = a.lo[2][pk], nk = a.hi[2][pk] - k0 + 1;
+  const int np = c.nj * c.nk;
+  constexpr int E = QC_PLANE / QC_THREADS;
+  double pv[E];
+  uint8_t ps[E];
+  auto fetch = [&](int i) {
+#pragma unroll
+    for (int u = 0; u < E; ++u) {
+      const int e = tid + u * QC_THREADS;
+      pv[u] = 0.0;
+      ps[u] = 0;
+      if (e < np) {
+        const int j = c.j0 + e / c.nk, k = c.k0 + e % c.nk;
+        const size_t s = ((size_t)j * a.pnx + i) * a.pnz + k;
+        const uint16_t f = a.flag[s];
+        const double eb = ((f & QN_OXIDE) && !(f & QN_SILICON)) ? -a.eb : 0.0;
+        const double x = a.pot[s] + eb;
+        pv[u] = (f & (QN_OXIDE | QN_SILICON)) ? x : 0.0;
+        ps[u] = a.shape[s];
+      }
+    }
+  };
+  auto put = [&](int b) {
+#pragma unroll
+    for (int u = 0; u < E; ++u) {
+      const int e = tid + u * QC_THREADS;
+      if (e < np) {
+        v[b][e] = pv[u];
+        sh[b][e] = ps[u];
+      }
+    }
+  };
+  fetch(i0);
+  put(0);
+  __syncthreads();
+  double ret = 0.0;
+  for (int i = i0; i <= i1; ++i) {
+    const int b = (i - i0) & 1;
+    if (i < i1) fetch(i + 1);
+    const double* wx = WX + (i - i0) * 4;
+    const double x0 = wx[0], x1 = wx[1], x2 = wx[2], x3 = wx[3];
+    int next = a.row_shape[(size_t)j0 * a.pnx + i];
+    for (int j = j0; j <= j1; ++j) {
+      const int row = next;
+      if (j < j1) next = a.row_shape[(size_t)(j + 1) * a.pnx + i];
+      const double* V = v[b] + (j - c.j0) * c.nk + (k0 - c.k0);
+      const uint8_t* S = sh[b] + (j - c.j0) * c.nk + (k0 - c.k0);
+      const double* wy = WY + (j - j0) * 4;
+      // the pair's two terms at a time, added in their order by both lanes
+      auto add2 = [&](double t) {
+        ret += quad_get<0xa0>(t);  // lanes 0 0 2 2
+        ret += quad_get<0xf5>(t);  // lanes 1 1 3 3
+      };
+      if (row != QC_MIXED) {
+        // the row's sources share their i and j shape
+        const double y = wy[(row >> 2) & 3], x = (row & 2) ? (row & 1) ? x3 : x2 : (row & 1) ? x1 : x0;
+        int k = g;
+        for (; k - g + 4 <= nk; k += 4) {
+          const double t0 = V[k] * WZ[k * 4 + (S[k] >> 4)] * y * x;
+          const double t1 = V[k + 2] * WZ[(k + 2) * 4 + (S[k + 2] >> 4)] * y * x;
+          add2(t0);
+          add2(t1);
+        }
+        for (; k - g < nk; k += 2) {
+          const int q = k < nk ? k : 0;
+          const double t = V[q] * WZ[q * 4 + (S[q] >> 4)] * y * x;
+          add2(k < nk ? t : 0.0);
+        }
+      } else {
+        for (int k = g; k - g < nk; k += 2) {
+          const int q = k < nk ? k : 0, s = S[q];
+          const double t = V[q] * WZ[q * 4 + (s >> 4)] * wy[(s >> 2) & 3] *
+                           ((s & 2) ? (s & 1) ? x3 : x2 : (s & 1) ? x1 : x0);
+          add2(k < nk ? t : 0.0);
+        }
+      }
+    }
+    if (i < i1) put(b ^ 1);
+    __syncthreads();
+  }
+  if (on && g == 0) a.qc_pot[p] = ret * 0.125;
+}
 
 __global__ void k_rhs(RhsArgs a) {
   const size_t stride = (size_t)gridDim.x * blockDim.x;
@@ -1942,7 +2063,8 @@ hipError_t emc_launch_rhs(const RhsArgs& a, hipStream_t s) {
 }
 hipError_t emc_launch_qc_potential(const QcArgs& a, hipStream_t s) {
   if (a.nq <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_qc_potential, dim3(grid_for(a.nq, 256)), dim3(256), 0, s, a);
+  if (a.nchunk > 0) hipLaunchKernelGGL(k_qc_potential, dim3(a.nchunk), dim3(QC_THREADS), 0, s, a);
+  else hipLaunchKernelGGL(k_qc_potential_nodes, dim3(grid_for(a.nq, 256)), dim3(256), 0, s, a);
   return hipGetLastError();
 }
 hipError_t emc_launch_field(const FieldArgs& a, hipStream_t s) {

@@ -30,6 +30,46 @@ void axis_window(const std::vector<double>& l, double r, std::vector<int>& lo, s
   }
 }
 
+// The targets in blocks of at most QC_CHUNK nodes of one i plane whose union window and
+// weights fit the block's LDS; no chunks when even a single target's do not.
+void build_chunks(int nx, int nz, QcTables& t) {
+  t.chunks.clear();
+  const size_t n = t.qnodes.size();
+  for (size_t s = 0; s < n;) {
+    QcChunk c{};
+    for (size_t e = s; e < n && e - s < (size_t)QC_CHUNK; ++e) {
+      const int p = t.qnodes[e], k = p % nz, i = p / nz % nx, j = p / nz / nx;
+      QcChunk w{(int)s, (int)(e - s) + 1, i, t.lo[1][j], 0, t.lo[2][k], 0, j, 1, k, 1, 0};
+      int j1 = t.hi[1][j], k1 = t.hi[2][k], tj1 = j, tk1 = k;
+      if (e > s) {
+        if (i != c.pi) break;
+        j1 = std::max(j1, c.j0 + c.nj - 1);
+        k1 = std::max(k1, c.k0 + c.nk - 1);
+        tj1 = std::max(tj1, c.tj0 + c.ntj - 1);
+        tk1 = std::max(tk1, c.tk0 + c.ntk - 1);
+        w.j0 = std::min(w.j0, c.j0);
+        w.k0 = std::min(w.k0, c.k0);
+        w.tj0 = std::min(w.tj0, c.tj0);
+        w.tk0 = std::min(w.tk0, c.tk0);
+      }
+      w.nj = j1 - w.j0 + 1;
+      w.nk = k1 - w.k0 + 1;
+      w.ntj = tj1 - w.tj0 + 1;
+      w.ntk = tk1 - w.tk0 + 1;
+      if ((long long)w.nj * w.nk > QC_PLANE ||
+          4LL * w.ntj * t.wlen[1] + (4LL * t.wlen[2] + 1) * w.ntk > QC_TABLE)
+        break;
+      c = w;
+    }
+    if (c.count == 0) {
+      t.chunks.clear();
+      return;
+    }
+    t.chunks.push_back(c);
+    s += (size_t)c.count;
+  }
+}
+
 }  // namespace
 
 std::string build_qc_tables(const Device& d, QcTables& t) {
@@ -92,8 +132,26 @@ std::string build_qc_tables(const Device& d, QcTables& t) {
     }
   }
   t.qnodes.clear();
-  for (size_t n = 0; n < NN; ++n)
-    if (t.flag[n] & QN_QUANTUM) t.qnodes.push_back((int)n);
+  for (int i = 0; i < nx; ++i)
+    for (int j = 0; j < ny; ++j)
+      for (int k = 0; k < nz; ++k)
+        if (t.flag[d.node(i, j, k)] & QN_QUANTUM) t.qnodes.push_back((int)d.node(i, j, k));
+  // shapes per node and per row
+  t.shape.assign(NN, 0);
+  t.row_shape.assign((size_t)nx * ny, 0);
+  for (int j = 0; j < ny; ++j)
+    for (int i = 0; i < nx; ++i) {
+      int row = -1;
+      for (int k = 0; k < nz; ++k) {
+        const uint16_t f = t.flag[d.node(i, j, k)];
+        if (!(f & (QN_OXIDE | QN_SILICON))) continue;
+        const int ij = qc_shape(f, 0) | qc_shape(f, 1) << 2;
+        t.shape[d.node(i, j, k)] = (uint8_t)(ij | qc_shape(f, 2) << 4);
+        row = row < 0 || row == ij ? ij : QC_MIXED;
+      }
+      t.row_shape[(size_t)j * nx + i] = (uint8_t)(row < 0 ? 0 : row);
+    }
+  build_chunks(nx, nz, t);
   t.eb = d.qc_eb;
   (void)nz;
   return "";

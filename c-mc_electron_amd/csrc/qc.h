@@ -24,6 +24,19 @@ namespace emc {
 constexpr uint16_t QN_SILICON = 1, QN_OXIDE = 2, QN_UP = 4, QN_DOWN = 8, QN_FRONT = 16, QN_BACK = 32,
                    QN_LEFT = 64, QN_RIGHT = 128, QN_QUANTUM = 256;
 
+// Targets of one block of k_qc_potential: up to QC_CHUNK nodes of one i plane, in
+// (j, k) order, and the union of their source windows in j and k.
+constexpr int QC_CHUNK = 128;   // targets per block, two lanes each
+constexpr int QC_PLANE = 1536;  // source nodes of one i plane in a chunk's union window
+constexpr int QC_TABLE = 3072;  // doubles of a chunk's j and k weights together
+constexpr int QC_MIXED = 255;   // row_shape: the row's sources differ in their i or j shape
+struct QcChunk {
+  int start, count, pi;  // qnodes[start .. start+count-1]
+  int j0, nj, k0, nk;    // union window
+  int tj0, ntj, tk0, ntk;  // range of the targets
+  int pad;
+};
+
 struct QcTables {
   std::vector<uint16_t> flag;     // [nnode]
   std::vector<int> lo[3], hi[3];  // per axis (x=i, y=j, z=k): source window [lo, hi] of each target index
@@ -32,7 +45,11 @@ struct QcTables {
   // source s seen from target t, box shape v (bit 0: low side at the region edge,
   // bit 1: high side at the region edge)
   std::vector<double> w[3];
-  std::vector<int> qnodes;        // nodes of the quantum region, ascending
+  std::vector<int> qnodes;        // nodes of the quantum region, ascending in (i, j, k)
+  std::vector<QcChunk> chunks;    // they in blocks; empty when a window does not fit
+  // [pny][pnx]: i shape | j shape << 2 of every solid node of the row (i, j), or QC_MIXED
+  std::vector<uint8_t> row_shape;
+  std::vector<uint8_t> shape;     // [nnode] i | j << 2 | k << 4 shapes, 0 where not solid
   double eb = 0;                  // normalised barrier, added at oxide-only nodes as -Eb
 };
 
