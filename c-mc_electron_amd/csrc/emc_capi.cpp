@@ -103,7 +103,9 @@ struct Gpu {
   // particles added since after them from slot sorted_n on
   bool seg_valid = false;
   long long sorted_n = 0;
-  unsigned long long* blk = nullptr;
+  unsigned *ioff = nullptr, *itile = nullptr;  // the deposit's work items
+  unsigned long long* blk = nullptr;           // their blocks
+  long long item_cap = 0;                      // work items blk and itile hold
   unsigned* n_host = nullptr;         // pinned: live count after the last sort
   hipEvent_t n_ready = nullptr;
   bool n_pending = false;
@@ -581,7 +583,7 @@ static int gpu_setup(emc_ctx* c) {
   g.toff = m.alloc<unsigned>(g.ntile + 1);
   g.tstay = m.alloc<unsigned>(g.ntile);
   g.toff_old = m.alloc<unsigned>(g.ntile + 1);
-  g.blk = m.alloc<unsigned long long>((size_t)g.ntile * DEP_NQ * TILE_NODES);
+  g.ioff = m.alloc<unsigned>(g.ntile + 1);
   g.T.contact = g.contact; g.T.counters = g.counters; g.T.rcur = g.rcur; g.T.lcur = g.lcur;
   g.T.heat_e = g.heat_e; g.T.heat_h = g.heat_h;
 
@@ -1469,6 +1471,7 @@ static SortArgs sort_args(emc_ctx* c) {
   a.P = g.P; a.Q = g.P2; a.n = g.n;
   a.ntx = g.ntx; a.nty = g.nty; a.ntz = g.ntz; a.ntile = g.ntile;
   a.tcount = g.tcount; a.toff = g.toff; a.tcursor = g.tcursor; a.tstay = g.tstay; a.toff_old = g.toff_old;
+  a.ioff = g.ioff; a.itile = g.itile;
   a.seg_valid = seg_usable(g) ? 1 : 0;
   return a;
 }
@@ -1478,9 +1481,30 @@ static long long sort_nappend(emc_ctx* c) {
   return seg_usable(g) ? std::max(0LL, g.n - g.sorted_n) : g.n;
 }
 
+// The deposit's work items for the slots of the population: their blocks grow with
+// it (in use on the device only between a sort and its deposit).
+static int ensure_items(emc_ctx* c) {
+  Gpu& g = *c->gpu;
+  const long long need = dep_items_most(g.ntile, g.n);
+  if (need <= g.item_cap) return EMC_OK;
+  const long long cap = dep_items_most(g.ntile, std::max(g.cap, g.n));
+  HIPCHECK(c, hipStreamSynchronize(g.stream));
+  DevBuf& m = g.mem;
+  m.release(g.itile);
+  m.release(g.blk);
+  g.item_cap = 0;
+  g.itile = m.alloc<unsigned>(cap);
+  g.blk = m.alloc<unsigned long long>((size_t)cap * DEP_SLOT);
+  if (m.last != hipSuccess) return fail(c, EMC_ERR_HIP, std::string("deposit blocks: ") + hipGetErrorString(m.last));
+  g.item_cap = cap;
+  return EMC_OK;
+}
+
 static int run_sort(emc_ctx* c) {
   Gpu& g = *c->gpu;
   int st = settle_n(c);
+  if (st) return st;
+  st = ensure_items(c);
   if (st) return st;
   SortArgs a = sort_args(c);
   HIPCHECK(c, emc_launch_tile_sort(a, sort_nappend(c), g.stream));
@@ -1498,7 +1522,7 @@ static DepositArgs deposit_args(emc_ctx* c, int stat_accumulate) {
   a.B = g.B; a.M = g.M; a.P = g.P;
   a.nnode = c->dev.nnode; a.ncell = c->dev.ncell;
   a.ntx = g.ntx; a.nty = g.nty; a.ntz = g.ntz; a.ntile = g.ntile;
-  a.toff = g.toff; a.blk = g.blk;
+  a.toff = g.toff; a.ioff = g.ioff; a.itile = g.itile; a.blk = g.blk;
   a.node_q = g.node_q; a.node_stat = g.node_stat; a.cell_q = g.cell_q; a.cell_n = g.cell_n;
   a.stat_accumulate = stat_accumulate;
   return a;
@@ -2263,7 +2287,7 @@ int emc_deposit(emc_ctx* c, int64_t* node_q, int64_t* node_stat, int64_t* cell_q
   const size_t NN = c->dev.nnode, NC = c->dev.ncell;
   int st = run_sort(c);
   if (st) return st;
-  HIPCHECK(c, emc_launch_deposit(deposit_args(c, 0), g.stream));
+  HIPCHECK(c, emc_launch_deposit(deposit_args(c, 0), dep_items_most(g.ntile, g.n), g.stream));
   HIPCHECK(c, hipStreamSynchronize(g.stream));
   st = settle_n(c);
   if (st) return st;
@@ -2510,7 +2534,7 @@ static int one_step(emc_ctx* c, bool heat_phase, emc_fly_tallies* acc, double ts
   DepositArgs da = deposit_args(c, 1);
   da.st = stat_args(c, heat_phase);
   if (!heat_phase) da.rhs = RhsArgs{NN, g.node_q, g.pvol, g.pdop, g.dirichlet, g.corr, g.kind, g.rhs, nullptr};
-  HIPCHECK(c, emc_launch_deposit(da, g.stream));
+  HIPCHECK(c, emc_launch_deposit(da, dep_items_most(g.ntile, g.n), g.stream));
   HIPCHECK(c, hipEventRecord(g.ev[1], g.stream));
   if (!heat_phase) {
     if (c->opts.poisson_fp32 == 1)
@@ -2800,7 +2824,7 @@ static int batch_one_step(emc_batch* b, emc_fly_tallies* acc, double tsum[5], in
   SortArgs* hs = (SortArgs*)(b->h_tab + b->off_sort);
   DepositArgs* hd = (DepositArgs*)(b->h_tab + b->off_dep);
   FlyArgs* hfl = (FlyArgs*)(b->h_tab + b->off_fly);
-  long long nmax = 0;
+  long long nmax = 0, nitem = 0;
   int guess = 0;
   for (int q = 0; q < K; ++q) {
     emc_ctx* c = b->c[q];
@@ -2810,6 +2834,9 @@ static int batch_one_step(emc_batch* b, emc_fly_tallies* acc, double tsum[5], in
     if (st) return bfail(b, st, c->err);
     st = grow_if_full(c);
     if (st) return bfail(b, st, c->err);
+    st = ensure_items(c);
+    if (st) return bfail(b, st, c->err);
+    nitem = std::max(nitem, dep_items_most(b->ntile, g.n));
     hs[q] = sort_args(c);
     nmax = std::max(nmax, sort_nappend(c));
     g.seg_valid = true;
@@ -2827,7 +2854,7 @@ static int batch_one_step(emc_batch* b, emc_fly_tallies* acc, double tsum[5], in
   BHIP(b, emc_launch_copy_b(b->cp_n, K, 1, s));
   BHIP(b, hipMemcpyAsync(b->h_n, b->d_n, K * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
   BHIP(b, hipEventRecord(b->ev_n, s));
-  BHIP(b, emc_launch_deposit_b(b->bt, b->ntile, b->nnode, s));
+  BHIP(b, emc_launch_deposit_b(b->bt, b->ntile, nitem, b->nnode, s));
   BHIP(b, hipEventRecord(b->ev[1], s));
   // the solve: as run_pcg, one iteration of every device per launch; the host
   // checks the iteration before the one just queued, for all devices at once

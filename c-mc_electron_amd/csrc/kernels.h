@@ -46,6 +46,13 @@ constexpr int TILE_I = 4, TILE_J = 8, TILE_K = 4;
 constexpr int TILE_NODES = (TILE_I + 1) * (TILE_J + 1) * (TILE_K + 1);
 constexpr int TILE_CELLS = TILE_I * TILE_J * TILE_K;
 constexpr int DEP_NQ = 11;  // node charge + 5 statistics x 2 carrier types
+// A tile's particles are deposited by one workgroup per DEP_ITEM of them (rounded up,
+// shares of equal length; an empty tile has one for its cells), a work item.  The
+// densest tiles set the time of a workgroup per tile: 64 particles a cell in the
+// 20x40x12-cell sweep devices, ten times the mean in the fin of the 80x160x48 one.
+constexpr int DEP_ITEM = 768;
+constexpr int DEP_SLOT = DEP_NQ * TILE_NODES + 4 * TILE_CELLS;  // words of an item's block
+inline long long dep_items_most(long long ntile, long long n) { return ntile + n / DEP_ITEM; }
 
 // Counting sort of the particles by tile (drops empty slots).
 // The population P was left by the previous sort in tile segments: slots
@@ -65,6 +72,8 @@ struct SortArgs {
   unsigned* tcursor;          // [ntile] zeroed by k_tile_scan
   unsigned* tstay;            // [ntile] stayers of each tile (k_tile_hist)
   unsigned* toff_old;         // [ntile + 1] the segments of the previous sort (k_tile_scan; all 0 without)
+  unsigned* ioff;             // [ntile + 1] first work item of each tile (k_tile_scan)
+  unsigned* itile;            // tile of each work item (k_tile_scan)
   int seg_valid, pad;
 };
 
@@ -120,7 +129,8 @@ struct DepositArgs {
   size_t nnode, ncell;
   int ntx, nty, ntz, ntile;
   const unsigned* toff;       // [ntile + 1]
-  unsigned long long* blk;    // [ntile][TILE_NODES][DEP_NQ] per-tile node sums
+  const unsigned *ioff, *itile;  // work items (SortArgs)
+  unsigned long long* blk;    // [items][DEP_SLOT]: [TILE_NODES][DEP_NQ] node sums, then the cell sums of a tile's share
   unsigned long long *node_q, *node_stat, *cell_q, *cell_n;  // any may be null
   int stat_accumulate;        // 1: node_stat += this step's sums, 0: node_stat = sums
   int pad0;
@@ -320,7 +330,7 @@ hipError_t emc_launch_pcg_start_b(const emc::BatchTables& t, const emc::MgArgs& 
 hipError_t emc_launch_pcg_iter_b(const emc::BatchTables& t, const emc::MgArgs& shape, int nblocks, int it,
                                  hipStream_t s);
 hipError_t emc_launch_tile_sort_b(const emc::BatchTables& t, int ntile, long long nappend_max, hipStream_t s);
-hipError_t emc_launch_deposit_b(const emc::BatchTables& t, int ntile, size_t nnode, hipStream_t s);
+hipError_t emc_launch_deposit_b(const emc::BatchTables& t, int ntile, long long nitem, size_t nnode, hipStream_t s);
 hipError_t emc_launch_field_b(const emc::BatchTables& t, size_t ncell, hipStream_t s);
 hipError_t emc_launch_fly_b(const emc::BatchTables& t, long long nmax, long long wave_slots, hipStream_t s);
 hipError_t emc_launch_copy_b(const emc::CopyArgs* t, int K, size_t nwords, hipStream_t s);
@@ -337,7 +347,8 @@ hipError_t emc_launch_clones_dev(const emc::FlyArgs& a, hipStream_t s);
 // nappend: an upper bound of the movers outside the segments (slots from the
 // previous sort's total on, or every slot without segments), for the grid
 hipError_t emc_launch_tile_sort(const emc::SortArgs& a, long long nappend, hipStream_t s);
-hipError_t emc_launch_deposit(const emc::DepositArgs& a, hipStream_t s);
+// nitem: an upper bound of the work items
+hipError_t emc_launch_deposit(const emc::DepositArgs& a, long long nitem, hipStream_t s);
 hipError_t emc_launch_rhs(const emc::RhsArgs& a, hipStream_t s);
 hipError_t emc_launch_qc_potential(const emc::QcArgs& a, hipStream_t s);
 hipError_t emc_launch_field(const emc::FieldArgs& a, hipStream_t s);

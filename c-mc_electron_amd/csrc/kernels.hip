@@ -509,9 +509,30 @@ __global__ __launch_bounds__(256) void k_tile_hist(AS as_) {
   }
 }
 
+// Exclusive prefix of v over a block of 1024 threads; total: the sum.
+__device__ inline unsigned block_prefix1024(unsigned v, unsigned* wsum, unsigned& total) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  unsigned in = v;
+  for (int o = 1; o < 64; o <<= 1) {
+    const unsigned u = __shfl_up(in, o, 64);
+    if (lane >= o) in += u;
+  }
+  if (lane == 63) wsum[w] = in;
+  __syncthreads();
+  unsigned before = 0;
+  total = 0;
+  for (int q = 0; q < 16; ++q) {
+    if (q < w) before += wsum[q];
+    total += wsum[q];
+  }
+  __syncthreads();
+  return before + in - v;
+}
+
 // One block of 1024 threads: the tile counts (stayers + movers) are scanned into
 // toff, whose previous contents (the segments the scatter reads) go to toff_old;
-// the mover counts and cursors are cleared for the next sort.
+// the mover counts and cursors are cleared for the next sort.  The deposit's work
+// items of each tile are counted the same way.
 template <class AS>
 __global__ __launch_bounds__(1024) void k_tile_scan(AS as_) {
   const SortArgs& a = kargs(as_);
@@ -519,22 +540,18 @@ __global__ __launch_bounds__(1024) void k_tile_scan(AS as_) {
   const int nt = a.ntile;
   const int tid = threadIdx.x;
   const int chunk = (nt + 1023) / 1024;
-  const int b0 = tid * chunk, b1 = min(nt, b0 + chunk);
+  const int b0 = min(nt, tid * chunk), b1 = min(nt, b0 + chunk);
   const unsigned old_total = a.toff[nt];
-  unsigned loc = 0;
-  for (int t = b0; t < b1; ++t) loc += a.tstay[t] + a.tcount[t];
-  // inclusive scan of loc over the block
-  const int lane = tid & 63, w = tid >> 6;
-  unsigned v = loc;
-  for (int o = 1; o < 64; o <<= 1) {
-    const unsigned u = __shfl_up(v, o, 64);
-    if (lane >= o) v += u;
+  auto items = [](unsigned cnt) { return cnt > (unsigned)DEP_ITEM ? (cnt + DEP_ITEM - 1) / DEP_ITEM : 1u; };
+  unsigned loc = 0, iloc = 0;
+  for (int t = b0; t < b1; ++t) {
+    const unsigned cnt = a.tstay[t] + a.tcount[t];
+    loc += cnt;
+    iloc += items(cnt);
   }
-  if (lane == 63) wsum[w] = v;
-  __syncthreads();
-  unsigned woff = 0;
-  for (int q = 0; q < w; ++q) woff += wsum[q];
-  unsigned run = woff + v - loc;  // exclusive prefix of this thread's chunk
+  unsigned tot, itot;
+  unsigned run = block_prefix1024(loc, wsum, tot);
+  unsigned irun = block_prefix1024(iloc, wsum, itot);
   for (int t = b0; t < b1; ++t) {
     const unsigned cnt = a.tstay[t] + a.tcount[t];
     a.toff_old[t] = a.seg_valid ? a.toff[t] : 0u;
@@ -542,12 +559,13 @@ __global__ __launch_bounds__(1024) void k_tile_scan(AS as_) {
     run += cnt;
     a.tcount[t] = 0;
     a.tcursor[t] = 0;
+    a.ioff[t] = irun;
+    for (const unsigned e = irun + items(cnt); irun < e; ++irun) a.itile[irun] = (unsigned)t;
   }
   if (tid == 1023) {
-    unsigned tot = 0;
-    for (int q = 0; q < 16; ++q) tot += wsum[q];
     a.toff_old[nt] = a.seg_valid ? old_total : 0u;
     a.toff[nt] = tot;
+    a.ioff[nt] = itot;
   }
 }
 
@@ -650,9 +668,14 @@ __device__ inline void stat_node(const StatArgs& a, size_t q) {
 // ------------------------------------------------------------------ deposit
 // statistic (src/mcmodel.cpp:1167-1408), particle_to_density (:348-417) and
 // compute_cell_charge (:2664-2712) in one pass over the tile-sorted particles.
-// One workgroup per tile sums the fixed-point contributions in LDS; each cell
-// belongs to one tile and is stored directly, the node block goes to `blk` and
-// k_deposit_gather adds the (up to 8) blocks that share a node.  Integer sums:
+// One workgroup per work item (a tile's particles, or a share of a dense tile's) sums
+// the fixed-point contributions in LDS; the node block goes to `blk` and
+// k_deposit_gather adds the blocks of the (up to 8) tiles that share a node.  A cell
+// belongs to one tile: it is stored directly, or added up there when the tile is
+// shared out.  A workgroup per tile ended with its densest: 752 us for the sixteen
+// 20x40x12-cell devices of the sweep (300 k particles each, 4000 a tile) and 187 us for
+// 3.0 M particles at 80x160x48 cells (600 a tile, 3500 in the fin), 195 and 140 us in
+// items.  Bound by LDS atomics now (51 a particle, 2.7 a clock and CU).  Integer sums:
 // the result does not depend on the order of the particles.  In a step the
 // gather also forms the Poisson right-hand side and statistic()'s potential and
 // heat sums of each node, and the cell pass adds the cell counts to the window.
@@ -661,10 +684,14 @@ __global__ __launch_bounds__(256) void k_deposit_tile(AS as_) {
   const DepositArgs& a = kargs(as_);
   __shared__ unsigned long long sn[DEP_NQ * TILE_NODES];
   __shared__ unsigned long long sc[4 * TILE_CELLS];
-  const int t = blockIdx.x;
+  if (blockIdx.x >= a.ioff[a.ntile]) return;
+  const int t = (int)a.itile[blockIdx.x];
   const int tk = t % a.ntz, ti = (t / a.ntz) % a.ntx, tj = t / (a.ntz * a.ntx);
   const int i0 = ti * TILE_I, j0 = tj * TILE_J, k0 = tk * TILE_K;
-  const unsigned p0 = a.toff[t], p1 = a.toff[t + 1];
+  // this item's share of the tile's particles
+  const unsigned nit = a.ioff[t + 1] - a.ioff[t], cnt = a.toff[t + 1] - a.toff[t];
+  const unsigned len = (cnt + nit - 1) / nit;
+  const unsigned p0 = min(a.toff[t] + (blockIdx.x - a.ioff[t]) * len, a.toff[t + 1]), p1 = min(p0 + len, a.toff[t + 1]);
   const size_t NC = a.ncell;
   for (int e = threadIdx.x; e < DEP_NQ * TILE_NODES; e += blockDim.x) sn[e] = 0;
   for (int e = threadIdx.x; e < 4 * TILE_CELLS; e += blockDim.x) sc[e] = 0;
@@ -726,7 +753,11 @@ __global__ __launch_bounds__(256) void k_deposit_tile(AS as_) {
     atomicAdd(&sc[2 * TILE_CELLS + lc], (unsigned long long)fxd(fabs(charge), 281474976710656.0));
   }
   __syncthreads();
-  for (int e = threadIdx.x; e < TILE_CELLS; e += blockDim.x) {
+  // the cells of a tile with one item are final; k_deposit_gather adds the others up
+  unsigned long long* slot = a.blk + (size_t)blockIdx.x * DEP_SLOT;
+  if (nit > 1)
+    for (int e = threadIdx.x; e < 4 * TILE_CELLS; e += blockDim.x) slot[DEP_NQ * TILE_NODES + e] = sc[e];
+  else for (int e = threadIdx.x; e < TILE_CELLS; e += blockDim.x) {
     const int lk = e % TILE_K, li = (e / TILE_K) % TILE_I, lj = e / (TILE_K * TILE_I);
     const int i = i0 + li, j = j0 + lj, k = k0 + lk;
     if (i >= a.M.cnx || j >= a.M.cny || k >= a.M.cnz) continue;
@@ -739,18 +770,40 @@ __global__ __launch_bounds__(256) void k_deposit_tile(AS as_) {
       a.cell_q[2 * NC + c] = sc[2 * TILE_CELLS + e];
     }
   }
-  if (p1 > p0) {
+  if (cnt > 0) {
     // node-major in memory ([node][quantity]): the gather reads a node's sums
     // from one 88-byte run
-    unsigned long long* b = a.blk + (size_t)t * DEP_NQ * TILE_NODES;
     for (int e = threadIdx.x; e < DEP_NQ * TILE_NODES; e += blockDim.x) {
       const int ln = e / DEP_NQ, q = e - ln * DEP_NQ;
-      b[e] = sn[q * TILE_NODES + ln];
+      slot[e] = sn[q * TILE_NODES + ln];
     }
   }
 }
 
-// One thread per node: sum the node's entries of the non-empty tiles around it.
+// The items of a tile with several are added into the block of its first, a workgroup
+// per further item taking an equal share of the block's words.  (Left to the gather,
+// whose threads would walk a tile's items one after another, the gather took 200 us
+// for the 16 devices of the sweep and 97 us at 80x160x48 cells, against 47 and
+// 22 us here and 31 and 72 in the gather.)
+template <class AS>
+__global__ __launch_bounds__(256) void k_deposit_merge(AS as_) {
+  const DepositArgs& a = kargs(as_);
+  if (blockIdx.x >= a.ioff[a.ntile]) return;
+  const unsigned t = a.itile[blockIdx.x], first = a.ioff[t], nit = a.ioff[t + 1] - first;
+  if (blockIdx.x == first) return;
+  const unsigned share = (DEP_SLOT + nit - 2) / (nit - 1), e0 = (blockIdx.x - first - 1) * share;
+  const unsigned e1 = min(e0 + share, (unsigned)DEP_SLOT);
+  for (unsigned e = e0 + threadIdx.x; e < e1; e += blockDim.x) {
+    unsigned long long* d = a.blk + (size_t)first * DEP_SLOT + e;
+    unsigned long long v = 0;
+#pragma unroll 4
+    for (unsigned it = 0; it < nit; ++it) v += d[(size_t)it * DEP_SLOT];
+    *d = v;
+  }
+}
+
+// One thread per node (there are more nodes than cells): sum the node's entries of
+// the non-empty tiles around it, and the cell's where its tile has several items.
 template <class AS>
 __global__ __launch_bounds__(256) void k_deposit_gather(AS as_) {
   const DepositArgs& a = kargs(as_);
@@ -774,7 +827,7 @@ __global__ __launch_bounds__(256) void k_deposit_gather(AS as_) {
           const int t = (ty[b] * a.ntx + tx[aa]) * a.ntz + tz[c];
           if (a.toff[t + 1] == a.toff[t]) continue;
           const int ln = (ly[b] * (TILE_I + 1) + lx[aa]) * (TILE_K + 1) + lz[c];
-          const unsigned long long* blk = a.blk + ((size_t)t * TILE_NODES + ln) * DEP_NQ;
+          const unsigned long long* blk = a.blk + (size_t)a.ioff[t] * DEP_SLOT + ln * DEP_NQ;
 #pragma unroll
           for (int q = 0; q < DEP_NQ; ++q) s[q] += blk[q];
         }
@@ -786,6 +839,26 @@ __global__ __launch_bounds__(256) void k_deposit_gather(AS as_) {
       for (int q = 0; q < 10; ++q) {
         unsigned long long* dst = a.node_stat + (size_t)q * NN + n;
         *dst = (a.stat_accumulate ? *dst : 0ull) + s[1 + q];
+      }
+    }
+    // cell n, where its tile's particles were shared out
+    if (n < a.ncell) {
+      const int k = (int)(n % a.M.cnz), i = (int)((n / a.M.cnz) % a.M.cnx), j = (int)(n / ((size_t)a.M.cnz * a.M.cnx));
+      const int t = ((j / TILE_J) * a.ntx + i / TILE_I) * a.ntz + k / TILE_K;
+      const unsigned first = a.ioff[t];
+      if (a.ioff[t + 1] - first > 1) {
+        const int lc = ((j % TILE_J) * TILE_I + i % TILE_I) * TILE_K + k % TILE_K;
+        const unsigned long long* c = a.blk + (size_t)first * DEP_SLOT + DEP_NQ * TILE_NODES + lc;
+        unsigned long long v[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) v[q] = c[q * TILE_CELLS];
+        if (a.cell_n) a.cell_n[n] = v[3];
+        if (a.st.stat_enum) a.st.stat_enum[n] += v[3];
+        if (a.cell_q) {
+          a.cell_q[n] = v[0];
+          a.cell_q[a.ncell + n] = v[1];
+          a.cell_q[2 * a.ncell + n] = v[2];
+        }
       }
     }
   }
@@ -2052,8 +2125,10 @@ hipError_t emc_launch_tile_sort(const SortArgs& a, long long nappend, hipStream_
   hipLaunchKernelGGL(k_tile_scatter<SortArgs>, dim3(g), dim3(512), 0, s, a);
   return hipGetLastError();
 }
-hipError_t emc_launch_deposit(const DepositArgs& a, hipStream_t s) {
-  hipLaunchKernelGGL(k_deposit_tile<DepositArgs>, dim3(a.ntile), dim3(256), 0, s, a);
+hipError_t emc_launch_deposit(const DepositArgs& a, long long nitem, hipStream_t s) {
+  hipLaunchKernelGGL(k_deposit_tile<DepositArgs>, dim3((unsigned)nitem), dim3(256), 0, s, a);
+  // no tile has two items while all particles fit one
+  if (nitem > a.ntile) hipLaunchKernelGGL(k_deposit_merge<DepositArgs>, dim3((unsigned)nitem), dim3(256), 0, s, a);
   hipLaunchKernelGGL(k_deposit_gather<DepositArgs>, dim3(grid_for((long long)a.nnode, 256)), dim3(256), 0, s, a);
   return hipGetLastError();
 }
@@ -2267,9 +2342,10 @@ hipError_t emc_launch_tile_sort_b(const BatchTables& t, int ntile, long long nap
   hipLaunchKernelGGL(k_tile_scatter<const SortArgs*>, dim3(g, K), dim3(512), 0, s, t.sort);
   return hipGetLastError();
 }
-hipError_t emc_launch_deposit_b(const BatchTables& t, int ntile, size_t nnode, hipStream_t s) {
+hipError_t emc_launch_deposit_b(const BatchTables& t, int ntile, long long nitem, size_t nnode, hipStream_t s) {
   const unsigned K = (unsigned)t.K;
-  hipLaunchKernelGGL(k_deposit_tile<const DepositArgs*>, dim3(ntile, K), dim3(256), 0, s, t.dep);
+  hipLaunchKernelGGL(k_deposit_tile<const DepositArgs*>, dim3((unsigned)nitem, K), dim3(256), 0, s, t.dep);
+  if (nitem > ntile) hipLaunchKernelGGL(k_deposit_merge<const DepositArgs*>, dim3((unsigned)nitem, K), dim3(256), 0, s, t.dep);
   hipLaunchKernelGGL(k_deposit_gather<const DepositArgs*>, dim3(grid_for((long long)nnode, 256), K), dim3(256), 0, s,
                      t.dep);
   return hipGetLastError();

@@ -118,7 +118,7 @@ double estimate_bytes(const emc_mesh_view& m, const std::string& deck, double ca
   const double ne = deck_number(deck, "ElectronNumber", 0), nh = deck_number(deck, "HoleNumber", 0);
   const double slots = (ne + nh + 2.0 * (double)m.ncell) * std::max(1.0, capacity_factor) + 1024;
   const double nc = std::max(600.0, std::min(2500.0, (double)m.nnode / 300));
-  return 320.0 * (double)m.nnode + 360.0 * (double)m.ncell + 190.0 * slots + 8.0 * nc * nc + (8 << 20);
+  return 320.0 * (double)m.nnode + 360.0 * (double)m.ncell + 222.0 * slots + 8.0 * nc * nc + (8 << 20);
 }
 
 void finish_window(Req* r) {
