@@ -170,8 +170,9 @@ def _pmc_pass(counter, args, outdir):
 
 # kernels of each phase of a step (the flight's headline pair first)
 PHASE_KERNELS = {
-    "flight": ("k_fly_fast", "k_fly_slow", "k_fly_clones_dev", "k_clone_range", "k_merge_dev"),
-    "deposit": ("k_tile_hist", "k_tile_scan", "k_tile_scatter", "k_deposit_tile", "k_deposit_gather"),
+    "flight": ("k_fly_fast", "k_fly_slow", "k_fly_clones_dev", "k_merge_dev"),
+    "deposit": ("k_tile_hist", "k_tile_scan", "k_tile_scatter", "k_deposit_tile", "k_deposit_merge",
+                "k_deposit_gather"),
     "poisson": ("k_pcg_", "k_mg_"),
 }
 

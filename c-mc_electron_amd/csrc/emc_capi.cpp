@@ -103,7 +103,7 @@ struct Gpu {
   // particles added since after them from slot sorted_n on
   bool seg_valid = false;
   long long sorted_n = 0;
-  unsigned *ioff = nullptr, *itile = nullptr;  // the deposit's work items
+  unsigned *ioff = nullptr, *itile = nullptr, *xtile = nullptr, *slot = nullptr;  // the deposit's work items
   unsigned long long* blk = nullptr;           // their blocks
   long long item_cap = 0;                      // work items blk and itile hold
   unsigned* n_host = nullptr;         // pinned: live count after the last sort
@@ -114,7 +114,7 @@ struct Gpu {
   long long* dead = nullptr;
   unsigned long long dead_cap = 0;
   unsigned long long* ctr = nullptr;  // [0] nclones [1] ndead [2] ticket [3] slow-list length
-                                      // [4] [5] clone range of the next pass [6] clone passes with work
+                                      // [4] clones of clones [5] theirs and later ones
   unsigned long long* ctr_host = nullptr;    // pinned copy of ctr after the flight
   unsigned long long* tally_host = nullptr;  // pinned copy of contact + counters after the flight
   bool pcg_pending = false;           // the step's PCG result is still to be read
@@ -584,6 +584,7 @@ static int gpu_setup(emc_ctx* c) {
   g.tstay = m.alloc<unsigned>(g.ntile);
   g.toff_old = m.alloc<unsigned>(g.ntile + 1);
   g.ioff = m.alloc<unsigned>(g.ntile + 1);
+  g.slot = m.alloc<unsigned>(g.ntile);
   g.T.contact = g.contact; g.T.counters = g.counters; g.T.rcur = g.rcur; g.T.lcur = g.lcur;
   g.T.heat_e = g.heat_e; g.T.heat_h = g.heat_h;
 
@@ -1387,16 +1388,18 @@ static int finish_fly(emc_ctx* c, const FlyArgs& a) {
   Gpu& g = *c->gpu;
   unsigned long long* h = g.ctr_host;
   g.last_full_loop = (long long)h[3];
-  int passes = (int)h[6];
-  if (h[5] > h[4]) {
-    const unsigned long long first = h[4];
-    unsigned long long begin = h[4], end = h[5];
+  // the buffer ranges of the generations, as clone_range has them
+  const unsigned long long n1 = std::min(h[0], g.clone_cap), first = n1 + std::min(h[4], g.clone_cap - n1);
+  int passes = (n1 > 0) + (first > n1);
+  if (first < g.clone_cap && h[5] > 0) {
+    ++passes;
+    unsigned long long begin = first, end = std::min(first + h[5], g.clone_cap);
     while (end > begin) {
       HIPCHECK(c, emc_launch_fly_clones(a, begin, end, g.stream));
       HIPCHECK(c, hipMemcpyAsync(h, g.ctr, 8 * sizeof(unsigned long long), hipMemcpyDeviceToHost, g.stream));
       HIPCHECK(c, hipStreamSynchronize(g.stream));
       begin = end;
-      end = std::min(h[0], g.clone_cap);
+      end = std::min(first + h[5], g.clone_cap);
       if (end > begin && ++passes > 64) return fail(c, EMC_ERR_STATE, "clone passes do not terminate");
     }
     HIPCHECK(c, emc_launch_merge(a, first, end, g.ctr + 1, g.ctr + 2, g.stream));
@@ -1471,7 +1474,7 @@ static SortArgs sort_args(emc_ctx* c) {
   a.P = g.P; a.Q = g.P2; a.n = g.n;
   a.ntx = g.ntx; a.nty = g.nty; a.ntz = g.ntz; a.ntile = g.ntile;
   a.tcount = g.tcount; a.toff = g.toff; a.tcursor = g.tcursor; a.tstay = g.tstay; a.toff_old = g.toff_old;
-  a.ioff = g.ioff; a.itile = g.itile;
+  a.ioff = g.ioff; a.itile = g.itile; a.xtile = g.xtile; a.slot = g.slot;
   a.seg_valid = seg_usable(g) ? 1 : 0;
   return a;
 }
@@ -1491,9 +1494,11 @@ static int ensure_items(emc_ctx* c) {
   HIPCHECK(c, hipStreamSynchronize(g.stream));
   DevBuf& m = g.mem;
   m.release(g.itile);
+  m.release(g.xtile);
   m.release(g.blk);
   g.item_cap = 0;
   g.itile = m.alloc<unsigned>(cap);
+  g.xtile = m.alloc<unsigned>(cap);
   g.blk = m.alloc<unsigned long long>((size_t)cap * DEP_SLOT);
   if (m.last != hipSuccess) return fail(c, EMC_ERR_HIP, std::string("deposit blocks: ") + hipGetErrorString(m.last));
   g.item_cap = cap;
@@ -1522,7 +1527,7 @@ static DepositArgs deposit_args(emc_ctx* c, int stat_accumulate) {
   a.B = g.B; a.M = g.M; a.P = g.P;
   a.nnode = c->dev.nnode; a.ncell = c->dev.ncell;
   a.ntx = g.ntx; a.nty = g.nty; a.ntz = g.ntz; a.ntile = g.ntile;
-  a.toff = g.toff; a.ioff = g.ioff; a.itile = g.itile; a.blk = g.blk;
+  a.toff = g.toff; a.ioff = g.ioff; a.itile = g.itile; a.xtile = g.xtile; a.slot = g.slot; a.blk = g.blk;
   a.node_q = g.node_q; a.node_stat = g.node_stat; a.cell_q = g.cell_q; a.cell_n = g.cell_n;
   a.stat_accumulate = stat_accumulate;
   return a;

@@ -54,7 +54,7 @@ struct Flight {
   const TallyDev& T;
   CloneRec* clones;
   unsigned long long* nclones;
-  unsigned long long clone_cap;
+  unsigned long long clone_cap, clone_base;  // clones go to clone_base + *nclones of the buffer
 
   // particle
   double x, y, z, kx, ky, kz, energy, charge, left_time;
@@ -68,7 +68,7 @@ struct Flight {
   Rng rng;
 
   EMC_HD Flight(const EMC_CST BandDev& b, const EMC_CST MeshDev& m, const EMC_CST FieldsDev& f, const TallyDev& t)
-      : B(b), M(m), F(f), T(t), clones(nullptr), nclones(nullptr), clone_cap(0) {}
+      : B(b), M(m), F(f), T(t), clones(nullptr), nclones(nullptr), clone_cap(0), clone_base(0) {}
 
   EMC_HD EMC_INL double Random() { return rng.next(); }
   EMC_HD EMC_INL int ms(int r, int s) const { return B.matsym[r * 48 + s]; }
@@ -1066,9 +1066,9 @@ struct Flight {
     neighbour(ii, jj, kk);
     const int ord = nclone++;
 #if defined(__HIP_DEVICE_COMPILE__)
-    const unsigned long long slot = atomicAdd(nclones, 1ull);
+    const unsigned long long slot = clone_base + atomicAdd(nclones, 1ull);
 #else
-    const unsigned long long slot = (*nclones)++;
+    const unsigned long long slot = clone_base + (*nclones)++;
 #endif
     if (slot >= clone_cap) { count(CNT_DROP0 + 8); return; }
     CloneRec& c = clones[slot];

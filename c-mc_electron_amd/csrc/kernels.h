@@ -51,6 +51,7 @@ constexpr int DEP_NQ = 11;  // node charge + 5 statistics x 2 carrier types
 // densest tiles set the time of a workgroup per tile: 64 particles a cell in the
 // 20x40x12-cell sweep devices, ten times the mean in the fin of the 80x160x48 one.
 constexpr int DEP_ITEM = 768;
+constexpr unsigned DEP_NONE = 0xFFFFFFFFu, DEP_SHARED = 0x80000000u;
 constexpr int DEP_SLOT = DEP_NQ * TILE_NODES + 4 * TILE_CELLS;  // words of an item's block
 inline long long dep_items_most(long long ntile, long long n) { return ntile + n / DEP_ITEM; }
 
@@ -74,6 +75,8 @@ struct SortArgs {
   unsigned* toff_old;         // [ntile + 1] the segments of the previous sort (k_tile_scan; all 0 without)
   unsigned* ioff;             // [ntile + 1] first work item of each tile (k_tile_scan)
   unsigned* itile;            // tile of each work item (k_tile_scan)
+  unsigned* xtile;            // the same over the items that are not their tile's first
+  unsigned* slot;             // [ntile] a tile's first block, DEP_SHARED set when it has several, DEP_NONE: no particles
   int seg_valid, pad;
 };
 
@@ -129,7 +132,7 @@ struct DepositArgs {
   size_t nnode, ncell;
   int ntx, nty, ntz, ntile;
   const unsigned* toff;       // [ntile + 1]
-  const unsigned *ioff, *itile;  // work items (SortArgs)
+  const unsigned *ioff, *itile, *xtile, *slot;  // work items (SortArgs)
   unsigned long long* blk;    // [items][DEP_SLOT]: [TILE_NODES][DEP_NQ] node sums, then the cell sums of a tile's share
   unsigned long long *node_q, *node_stat, *cell_q, *cell_n;  // any may be null
   int stat_accumulate;        // 1: node_stat += this step's sums, 0: node_stat = sums

@@ -291,9 +291,25 @@ __global__ __launch_bounds__(256) void k_fly_slow(AS as_) {
   flush_counters(a.T, ev, ph, im, ca);
 }
 
+// Where generation gen lies in the clone buffer: the particles' clones (counted in
+// ctr[0]), their clones (ctr[4]), and theirs and later ones (ctr[5]), one after the
+// other, each cut at the buffer's end.
+struct CloneRange { unsigned long long begin, end; };
+__device__ __forceinline__ CloneRange clone_range(const FlyArgs& a, int gen) {
+  const unsigned long long* ctr = a.nclones;
+  CloneRange r{0, ctr[0] < a.clone_cap ? ctr[0] : a.clone_cap};
+  for (int g = 1; g <= gen; ++g) {
+    const unsigned long long made = ctr[3 + g], room = a.clone_cap - r.end;
+    r = CloneRange{r.end, r.end + (made < room ? made : room)};
+  }
+  return r;
+}
+
 // Clones [begin, end) of the clone buffer fly the remaining time of the step;
-// `lpw` clones per wave, as in k_fly_slow.
-__device__ __forceinline__ void fly_clone_range(const FlyArgs& a, unsigned long long begin, unsigned long long end, int lpw) {
+// `lpw` clones per wave, as in k_fly_slow.  The clones they make go to `base` +
+// *made of the buffer.
+__device__ __forceinline__ void fly_clone_range(const FlyArgs& a, unsigned long long begin, unsigned long long end, int lpw,
+                                                unsigned long long base, unsigned long long* made) {
   long long ev = 0, ph = 0, im = 0, ca = 0;
   const int lane = threadIdx.x & 63;
   const long long wave = ((long long)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
@@ -303,7 +319,8 @@ __device__ __forceinline__ void fly_clone_range(const FlyArgs& a, unsigned long 
       CloneRec& c = a.clones[q];
       Flight f(fly_const(a.C).B, fly_const(a.C).M, fly_const(a.C).F, a.T);
       f.clones = a.clones;
-      f.nclones = a.nclones;
+      f.nclones = made;
+      f.clone_base = base;
       f.clone_cap = a.clone_cap;
       f.x = c.x; f.y = c.y; f.z = c.z; f.kx = c.kx; f.ky = c.ky; f.kz = c.kz;
       f.energy = c.energy; f.charge = c.charge; f.left_time = c.left_time;
@@ -329,37 +346,24 @@ __device__ __forceinline__ void fly_clone_range(const FlyArgs& a, unsigned long 
   flush_counters(a.T, ev, ph, im, ca);
 }
 
-// clones [begin, end): the host-driven pass
+// clones [begin, end): the host-driven pass; theirs follow the third generation's
 __global__ __launch_bounds__(256) void k_fly_clones(FlyArgs a, unsigned long long begin, unsigned long long end,
                                                     int lpw) {
-  fly_clone_range(a, begin, end, lpw);
+  fly_clone_range(a, begin, end, lpw, clone_range(a, 2).begin, a.nclones + 5);
 }
 
-// Clone passes without the host: ctr[4] .. ctr[5] is the range the next pass
-// flies.  k_clone_range moves it on to the clones created since and counts the
-// non-empty ranges in ctr[6] (one thread).
+// Generation gen (0: the particles' clones, 1: those clones' clones) flown without the
+// host, spread as k_fly_slow spreads its list.  Each generation has a counter of its
+// own, so the range a launch flies does not move while it makes the next.
 template <class AS>
-__global__ void k_clone_range(AS as_) {
+__global__ __launch_bounds__(256) void k_fly_clones_dev(AS as_, int gen) {
   const FlyArgs& a = kargs(as_);
-  unsigned long long* ctr = a.nclones;
-  const unsigned long long cap = a.clone_cap;
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    ctr[4] = ctr[5];
-    ctr[5] = ctr[0] < cap ? ctr[0] : cap;
-    if (ctr[5] > ctr[4]) ctr[6] += 1;
-  }
-}
-
-// k_fly_clones over ctr[4] .. ctr[5], spread as k_fly_slow spreads its list
-template <class AS>
-__global__ __launch_bounds__(256) void k_fly_clones_dev(AS as_) {
-  const FlyArgs& a = kargs(as_);
-  const unsigned long long* ctr = a.nclones;
-  const long long begin = (long long)ctr[4], n = (long long)ctr[5] - begin;
+  const CloneRange r = clone_range(a, gen);
+  const long long n = (long long)(r.end - r.begin);
   if (n <= 0) return;
   const long long slots = a.wave_slots > 0 ? a.wave_slots : 1;
   const int lpw = (int)(n <= slots ? 1 : ((n + slots - 1) / slots < 64 ? (n + slots - 1) / slots : 64));
-  fly_clone_range(a, (unsigned long long)begin, (unsigned long long)(begin + n), lpw);
+  fly_clone_range(a, r.begin, r.end, lpw, r.end, a.nclones + 4 + gen);
 }
 
 // Surviving clones take the slots of caught particles first, then go past n:
@@ -387,12 +391,12 @@ __global__ __launch_bounds__(256) void k_merge(FlyArgs a, unsigned long long beg
   }
 }
 
-// k_merge over the clones flown by the device-driven passes: [0, ctr[4])
+// k_merge over the clones flown by the device-driven passes: the first two generations
 template <class AS>
 __global__ __launch_bounds__(256) void k_merge_dev(AS as_) {
   const FlyArgs& a = kargs(as_);
   unsigned long long* ctr = a.nclones;
-  const unsigned long long end = ctr[4], ndead = ctr[1];
+  const unsigned long long end = clone_range(a, 1).end, ndead = ctr[1];
   const long long stride = (long long)gridDim.x * blockDim.x;
   for (long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x; q < (long long)end; q += stride) {
     const CloneRec& c = a.clones[q];
@@ -559,8 +563,14 @@ __global__ __launch_bounds__(1024) void k_tile_scan(AS as_) {
     run += cnt;
     a.tcount[t] = 0;
     a.tcursor[t] = 0;
+    const unsigned ni = items(cnt);
     a.ioff[t] = irun;
-    for (const unsigned e = irun + items(cnt); irun < e; ++irun) a.itile[irun] = (unsigned)t;
+    a.slot[t] = cnt == 0 ? DEP_NONE : ni > 1 ? irun | DEP_SHARED : irun;
+    a.itile[irun++] = (unsigned)t;
+    for (unsigned e = 1; e < ni; ++e, ++irun) {
+      a.itile[irun] = (unsigned)t;
+      a.xtile[irun - (unsigned)t - 1] = (unsigned)t;  // every tile so far has one first item
+    }
   }
   if (tid == 1023) {
     a.toff_old[nt] = a.seg_valid ? old_total : 0u;
@@ -783,23 +793,35 @@ __global__ __launch_bounds__(256) void k_deposit_tile(AS as_) {
 // The items of a tile with several are added into the block of its first, a workgroup
 // per further item taking an equal share of the block's words.  (Left to the gather,
 // whose threads would walk a tile's items one after another, the gather took 200 us
-// for the 16 devices of the sweep and 97 us at 80x160x48 cells, against 47 and
-// 22 us here and 31 and 72 in the gather.)
+// for the 16 devices of the sweep and 97 us at 80x160x48 cells, against 38 and
+// 18 us here and 28 and 68 in the gather; 9 us here at 60x138x42 cells.)
 template <class AS>
 __global__ __launch_bounds__(256) void k_deposit_merge(AS as_) {
   const DepositArgs& a = kargs(as_);
-  if (blockIdx.x >= a.ioff[a.ntile]) return;
-  const unsigned t = a.itile[blockIdx.x], first = a.ioff[t], nit = a.ioff[t + 1] - first;
-  if (blockIdx.x == first) return;
-  const unsigned share = (DEP_SLOT + nit - 2) / (nit - 1), e0 = (blockIdx.x - first - 1) * share;
+  if (blockIdx.x >= a.ioff[a.ntile] - (unsigned)a.ntile) return;
+  const unsigned t = a.xtile[blockIdx.x], first = a.ioff[t], nit = a.ioff[t + 1] - first;
+  const unsigned share = (DEP_SLOT + nit - 2) / (nit - 1), e0 = (blockIdx.x - (first - t)) * share;
   const unsigned e1 = min(e0 + share, (unsigned)DEP_SLOT);
-  for (unsigned e = e0 + threadIdx.x; e < e1; e += blockDim.x) {
-    unsigned long long* d = a.blk + (size_t)first * DEP_SLOT + e;
-    unsigned long long v = 0;
+  unsigned long long* base = a.blk + (size_t)first * DEP_SLOT;
+  // W words of a thread at a time, their reads together
+  auto merge = [&](auto w) {
+    constexpr int W = decltype(w)::value;
+    for (unsigned e = e0 + threadIdx.x; e < e1; e += W * blockDim.x) {
+      unsigned long long v[W];
+#pragma unroll
+      for (int u = 0; u < W; ++u) v[u] = e + u * blockDim.x < e1 ? base[e + u * blockDim.x] : 0;
 #pragma unroll 4
-    for (unsigned it = 0; it < nit; ++it) v += d[(size_t)it * DEP_SLOT];
-    *d = v;
-  }
+      for (unsigned it = 1; it < nit; ++it)
+#pragma unroll
+        for (int u = 0; u < W; ++u)
+          if (e + u * blockDim.x < e1) v[u] += base[(size_t)it * DEP_SLOT + e + u * blockDim.x];
+#pragma unroll
+      for (int u = 0; u < W; ++u)
+        if (e + u * blockDim.x < e1) base[e + u * blockDim.x] = v[u];
+    }
+  };
+  if (nit <= 3) merge(std::integral_constant<int, 6>());
+  else merge(std::integral_constant<int, 1>());
 }
 
 // One thread per node (there are more nodes than cells): sum the node's entries of
@@ -825,9 +847,10 @@ __global__ __launch_bounds__(256) void k_deposit_gather(AS as_) {
       for (int aa = 0; aa < nx; ++aa)
         for (int c = 0; c < nz; ++c) {
           const int t = (ty[b] * a.ntx + tx[aa]) * a.ntz + tz[c];
-          if (a.toff[t + 1] == a.toff[t]) continue;
+          const unsigned slot = a.slot[t];
+          if (slot == DEP_NONE) continue;
           const int ln = (ly[b] * (TILE_I + 1) + lx[aa]) * (TILE_K + 1) + lz[c];
-          const unsigned long long* blk = a.blk + (size_t)a.ioff[t] * DEP_SLOT + ln * DEP_NQ;
+          const unsigned long long* blk = a.blk + (size_t)(slot & ~DEP_SHARED) * DEP_SLOT + ln * DEP_NQ;
 #pragma unroll
           for (int q = 0; q < DEP_NQ; ++q) s[q] += blk[q];
         }
@@ -845,10 +868,10 @@ __global__ __launch_bounds__(256) void k_deposit_gather(AS as_) {
     if (n < a.ncell) {
       const int k = (int)(n % a.M.cnz), i = (int)((n / a.M.cnz) % a.M.cnx), j = (int)(n / ((size_t)a.M.cnz * a.M.cnx));
       const int t = ((j / TILE_J) * a.ntx + i / TILE_I) * a.ntz + k / TILE_K;
-      const unsigned first = a.ioff[t];
-      if (a.ioff[t + 1] - first > 1) {
+      const unsigned slot = a.slot[t];
+      if (slot != DEP_NONE && (slot & DEP_SHARED)) {
         const int lc = ((j % TILE_J) * TILE_I + i % TILE_I) * TILE_K + k % TILE_K;
-        const unsigned long long* c = a.blk + (size_t)first * DEP_SLOT + DEP_NQ * TILE_NODES + lc;
+        const unsigned long long* c = a.blk + (size_t)(slot & ~DEP_SHARED) * DEP_SLOT + DEP_NQ * TILE_NODES + lc;
         unsigned long long v[4];
 #pragma unroll
         for (int q = 0; q < 4; ++q) v[q] = c[q * TILE_CELLS];
@@ -2099,15 +2122,13 @@ hipError_t emc_launch_merge(const FlyArgs& a, unsigned long long begin, unsigned
 }
 // Two clone passes (clones, then the clones they made) and the merge of what
 // they flew, with every range read on the device: no host round trip.  ctr[4]
-// and ctr[5] must read zero on entry; afterwards ctr[4] .. ctr[5] holds clones
-// of a third generation still to fly (almost always empty).
+// and ctr[5] must read zero on entry; afterwards ctr[5] counts clones of a third
+// generation still to fly (almost always none).  A kernel between the passes that
+// moved the range on cost 5.5 us each time, 16 us a step.
 hipError_t emc_launch_clones_dev(const FlyArgs& a, hipStream_t s) {
   const long long blocks = a.wave_slots > 4 ? a.wave_slots / 4 : 1;
-  for (int pass = 0; pass < 2; ++pass) {
-    hipLaunchKernelGGL(k_clone_range<FlyArgs>, dim3(1), dim3(64), 0, s, a);
-    hipLaunchKernelGGL(k_fly_clones_dev<FlyArgs>, dim3((unsigned)blocks), dim3(256), 0, s, a);
-  }
-  hipLaunchKernelGGL(k_clone_range<FlyArgs>, dim3(1), dim3(64), 0, s, a);
+  for (int gen = 0; gen < 2; ++gen)
+    hipLaunchKernelGGL(k_fly_clones_dev<FlyArgs>, dim3((unsigned)blocks), dim3(256), 0, s, a, gen);
   hipLaunchKernelGGL(k_merge_dev<FlyArgs>, dim3((unsigned)blocks), dim3(256), 0, s, a);
   return hipGetLastError();
 }
@@ -2128,7 +2149,8 @@ hipError_t emc_launch_tile_sort(const SortArgs& a, long long nappend, hipStream_
 hipError_t emc_launch_deposit(const DepositArgs& a, long long nitem, hipStream_t s) {
   hipLaunchKernelGGL(k_deposit_tile<DepositArgs>, dim3((unsigned)nitem), dim3(256), 0, s, a);
   // no tile has two items while all particles fit one
-  if (nitem > a.ntile) hipLaunchKernelGGL(k_deposit_merge<DepositArgs>, dim3((unsigned)nitem), dim3(256), 0, s, a);
+  if (nitem > a.ntile)
+    hipLaunchKernelGGL(k_deposit_merge<DepositArgs>, dim3((unsigned)(nitem - a.ntile)), dim3(256), 0, s, a);
   hipLaunchKernelGGL(k_deposit_gather<DepositArgs>, dim3(grid_for((long long)a.nnode, 256)), dim3(256), 0, s, a);
   return hipGetLastError();
 }
@@ -2345,7 +2367,8 @@ hipError_t emc_launch_tile_sort_b(const BatchTables& t, int ntile, long long nap
 hipError_t emc_launch_deposit_b(const BatchTables& t, int ntile, long long nitem, size_t nnode, hipStream_t s) {
   const unsigned K = (unsigned)t.K;
   hipLaunchKernelGGL(k_deposit_tile<const DepositArgs*>, dim3((unsigned)nitem, K), dim3(256), 0, s, t.dep);
-  if (nitem > ntile) hipLaunchKernelGGL(k_deposit_merge<const DepositArgs*>, dim3((unsigned)nitem, K), dim3(256), 0, s, t.dep);
+  if (nitem > ntile)
+    hipLaunchKernelGGL(k_deposit_merge<const DepositArgs*>, dim3((unsigned)(nitem - ntile), K), dim3(256), 0, s, t.dep);
   hipLaunchKernelGGL(k_deposit_gather<const DepositArgs*>, dim3(grid_for((long long)nnode, 256), K), dim3(256), 0, s,
                      t.dep);
   return hipGetLastError();
@@ -2360,11 +2383,8 @@ hipError_t emc_launch_fly_b(const BatchTables& t, long long nmax, long long wave
   if (nmax > 0) hipLaunchKernelGGL(k_fly_fast<const FlyArgs*>, dim3(grid_for(nmax, 256), K), dim3(256), 0, s, t.fly);
   const long long blocks = wave_slots > 4 ? wave_slots / 4 : 1;
   hipLaunchKernelGGL(k_fly_slow<const FlyArgs*>, dim3((unsigned)blocks, K), dim3(256), 0, s, t.fly);
-  for (int pass = 0; pass < 2; ++pass) {
-    hipLaunchKernelGGL(k_clone_range<const FlyArgs*>, dim3(1, K), dim3(64), 0, s, t.fly);
-    hipLaunchKernelGGL(k_fly_clones_dev<const FlyArgs*>, dim3((unsigned)blocks, K), dim3(256), 0, s, t.fly);
-  }
-  hipLaunchKernelGGL(k_clone_range<const FlyArgs*>, dim3(1, K), dim3(64), 0, s, t.fly);
+  for (int gen = 0; gen < 2; ++gen)
+    hipLaunchKernelGGL(k_fly_clones_dev<const FlyArgs*>, dim3((unsigned)blocks, K), dim3(256), 0, s, t.fly, gen);
   hipLaunchKernelGGL(k_merge_dev<const FlyArgs*>, dim3((unsigned)blocks, K), dim3(256), 0, s, t.fly);
   return hipGetLastError();
 }
