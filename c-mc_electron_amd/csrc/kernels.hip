@@ -1638,20 +1638,12 @@ __global__ __launch_bounds__(256) void k_mg_resid(AS ms_) {
   if (*m.done) return;
   ph_resid<true>(m, m.L[0], GridLoop());
 }
-// levels >= 1: sweep from zero and residual in one pass
 template <class AS>
-__global__ __launch_bounds__(256) void k_mg_resid1(AS ms_, int l) {
+__global__ __launch_bounds__(256) void k_mg_restrict(AS ms_) {
   const auto& m = kargs(ms_);
   using R = typename std::decay_t<decltype(m)>::real;
   if (*m.done) return;
-  ph_resid1<false>(m, m.L[l], GridLoop());
-}
-template <class AS>
-__global__ __launch_bounds__(256) void k_mg_restrict(AS ms_, int l) {
-  const auto& m = kargs(ms_);
-  using R = typename std::decay_t<decltype(m)>::real;
-  if (*m.done) return;
-  ph_restrict(m.L[l], m.L[l + 1], GridLoop());
+  ph_restrict(m.L[0], m.L[1], GridLoop());
 }
 template <class AS>
 __global__ __launch_bounds__(256) void k_mg_prolong(AS ms_) {
@@ -1659,21 +1651,6 @@ __global__ __launch_bounds__(256) void k_mg_prolong(AS ms_) {
   using R = typename std::decay_t<decltype(m)>::real;
   if (*m.done) return;
   ph_prolong<false>(m.L[0], m.L[1], mg_result(m, 1), GridLoop());
-}
-template <class AS>
-__global__ __launch_bounds__(256) void k_mg_prolong1(AS ms_, int l) {
-  const auto& m = kargs(ms_);
-  using R = typename std::decay_t<decltype(m)>::real;
-  if (*m.done) return;
-  ph_prolong<true>(m.L[l], m.L[l + 1], mg_result(m, l + 1), GridLoop());
-}
-// levels >= 1: one sweep t -> x
-template <class AS>
-__global__ __launch_bounds__(256) void k_mg_post1(AS ms_, int l) {
-  const auto& m = kargs(ms_);
-  using R = typename std::decay_t<decltype(m)>::real;
-  if (*m.done) return;
-  ph_sweep<false>(m, m.L[l], m.L[l].t, m.L[l].x, GridLoop());
 }
 template <class AS>
 __global__ __launch_bounds__(256) void k_mg_post0a(AS ms_) {
@@ -1736,6 +1713,162 @@ __global__ __launch_bounds__(256) void k_mg_dot_rz(AS ms_) {
   double rz = 0;
   for (size_t n = GridLoop::start(); n < L.n; n += GridLoop::stride()) rz += (double)L.b[n] * (double)z[n];
   block_reduce1(rz, part_rz);
+}
+
+// ---- the coarse levels' phases fused over tiles staged in LDS
+// A phase of its own takes 3 to 5 us on a coarse level whatever its size.  The fused
+// kernels form a tile's intermediate values together with the ring around it that the
+// next phase reads (the ring's values are formed again by the neighbouring tile, by the
+// same operations), so a level goes down in one launch and up in one: 13 launches an
+// iteration instead of 17 on a four-level hierarchy.  Every value that is stored has
+// the operations of its phase in their order, so the cycle's result is the same to
+// the bit.  Kernel time a level, mean over levels >= 1, the gap of about 1 us a launch
+// not counted: down 8.2 -> 5.6 us and up 7.8 -> 7.1 at 83 k nodes, 8.0 -> 6.2 and 8.0 ->
+// 7.8 at 263 k, even at 639 k.  On the mesh level, bound by what it reads, the same
+// fusion lost (down 11 -> 13.3 us, up 7.0 -> 8.9 at 83 k; 12.5 -> 23.6, 8.7 -> 12.0 at
+// 263 k; 23 -> 37.5, 12.4 -> 17.5 at 639 k) and is not there.
+constexpr int TILE_THREADS = 256;
+
+// P^T r at coarse node (ci, cj, ck) with r from a tile accessor r(fi, fj, fk)
+// (ph_restrict's sum)
+template <class LV, class RA>
+__device__ __forceinline__ void tile_restrict(const LV& F, const LV& C, const RA& r, int ci, int cj, int ck) {
+  double v = 0;
+#pragma unroll
+  for (int dj = -1; dj <= 1; ++dj)
+#pragma unroll
+    for (int di = -1; di <= 1; ++di) {
+      const double w = (dj == 0 ? 1.0 : 0.5) * (di == 0 ? 1.0 : 0.5);
+#pragma unroll
+      for (int dk = -1; dk <= 1; ++dk) {
+        const int fj = 2 * cj + dj, fi = 2 * ci + di, fk = 2 * ck + dk;
+        const bool ok = (unsigned)fj < (unsigned)F.ny && (unsigned)fi < (unsigned)F.nx && (unsigned)fk < (unsigned)F.nz;
+        v += ok ? w * (dk == 0 ? 1.0 : 0.5) * (double)r(fi, fj, fk) : 0.0;
+      }
+    }
+  const size_t I = ((size_t)cj * C.nx + ci) * C.nz + ck;
+  C.b[I] = v;
+  C.x[I] = (double)C.wdinv[I] * v;
+}
+
+// the sweep from zero wdinv b, + P e, at node n (ph_prolong's value)
+template <class LV, class R>
+__device__ __forceinline__ double tile_prolong(const LV& F, const LV& C, const R* e, size_t n, int i, int j, int k) {
+  const double wd = F.wdinv[n];
+  if (wd == 0.0) return 0.0;
+  int cj[2] = {j >> 1, (j + 1) >> 1}, ci[2] = {i >> 1, (i + 1) >> 1}, ck[2] = {k >> 1, (k + 1) >> 1};
+  bool okj[2] = {cj[0] < C.ny, (j & 1) && cj[1] < C.ny}, oki[2] = {ci[0] < C.nx, (i & 1) && ci[1] < C.nx},
+       okk[2] = {ck[0] < C.nz, (k & 1) && ck[1] < C.nz};
+  double ev[8];
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        const bool ok = okj[a] && oki[b] && okk[c];
+        ev[(a * 2 + b) * 2 + c] = e[ok ? ((size_t)cj[a] * C.nx + ci[b]) * C.nz + ck[c] : 0];
+      }
+  double v = 0;
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      const double w = pw1(j, cj[a]) * pw1(i, ci[b]);
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
+        v += (okj[a] && oki[b] && okk[c]) ? w * pw1(k, ck[c]) * ev[(a * 2 + b) * 2 + c] : 0.0;
+    }
+  return wd * (double)F.b[n] + v;
+}
+
+// Level l >= 1 down: the residual of the sweep from zero (x) and its restriction.
+template <class AS>
+__global__ __launch_bounds__(TILE_THREADS) void k_mg_down(AS ms_, int l) {
+  const auto& m = kargs(ms_);
+  using R = typename std::decay_t<decltype(m)>::real;
+  if (*m.done) return;
+  const auto &F = m.L[l], &C = m.L[l + 1];
+  constexpr int CI = 2, CJ = 2, CK = 4, RI = 2 * CI + 1, RJ = 2 * CJ + 1, RK = 2 * CK + 1;
+  static_assert(RI * RJ * RK <= TILE_THREADS, "one residual per thread");
+  __shared__ R sr[RI * RJ * RK];
+  const int gk = (C.nz + CK - 1) / CK, gi = (C.nx + CI - 1) / CI;
+  const int bk = blockIdx.x % gk, bi = blockIdx.x / gk % gi, bj = blockIdx.x / (gk * gi);
+  const int i0 = 2 * CI * bi, j0 = 2 * CJ * bj, k0 = 2 * CK * bk;
+  const int e = threadIdx.x;
+  if (e < RI * RJ * RK) {
+    const int k = k0 - 1 + e % RK, i = i0 - 1 + e / RK % RI, j = j0 - 1 + e / (RK * RI);
+    if ((unsigned)i < (unsigned)F.nx && (unsigned)j < (unsigned)F.ny && (unsigned)k < (unsigned)F.nz) {
+      const size_t n = ((size_t)j * F.nx + i) * F.nz + k;
+      auto x1 = [&](size_t q) -> double { return F.x[q]; };
+      sr[e] = (R)((double)F.b[n] - mg_Ax<false>(m, F, x1, n, i, j, k));
+    }
+  }
+  __syncthreads();
+  if (e < CI * CJ * CK) {
+    const int ck = CK * bk + e % CK, ci = CI * bi + e / CK % CI, cj = CJ * bj + e / (CK * CI);
+    if (ck < C.nz && ci < C.nx && cj < C.ny) {
+      auto r = [&](int fi, int fj, int fk) { return sr[((fj - j0 + 1) * RI + fi - i0 + 1) * RK + fk - k0 + 1]; };
+      tile_restrict(F, C, r, ci, cj, ck);
+    }
+  }
+}
+
+// Level l >= 1 up: t = sweep from zero + P e, then one sweep t -> x.
+template <class AS>
+__global__ __launch_bounds__(TILE_THREADS) void k_mg_up(AS ms_, int l) {
+  const auto& m = kargs(ms_);
+  using R = typename std::decay_t<decltype(m)>::real;
+  if (*m.done) return;
+  const auto &L = m.L[l], &C = m.L[l + 1];
+  constexpr int NI = 4, NJ = 8, NK = 8, HI = NI + 2, HJ = NJ + 2, HK = NK + 2;
+  __shared__ R st[HI * HJ * HK];
+  const int gk = (L.nz + NK - 1) / NK, gi = (L.nx + NI - 1) / NI;
+  const int i0 = blockIdx.x / gk % gi * NI, j0 = blockIdx.x / (gk * gi) * NJ, k0 = blockIdx.x % gk * NK;
+  const R* e = mg_result(m, l + 1);
+  for (int q = threadIdx.x; q < HI * HJ * HK; q += TILE_THREADS) {
+    const int k = k0 - 1 + q % HK, i = i0 - 1 + q / HK % HI, j = j0 - 1 + q / (HK * HI);
+    R t = 0;
+    if ((unsigned)i < (unsigned)L.nx && (unsigned)j < (unsigned)L.ny && (unsigned)k < (unsigned)L.nz)
+      t = (R)tile_prolong(L, C, e, ((size_t)j * L.nx + i) * L.nz + k, i, j, k);
+    st[q] = t;
+  }
+  __syncthreads();
+  static_assert(NI * NJ * NK == TILE_THREADS, "one node per thread");
+  const int lk = threadIdx.x % NK, li = threadIdx.x / NK % NI, lj = threadIdx.x / (NK * NI);
+  const int k = k0 + lk, i = i0 + li, j = j0 + lj;
+  if (i >= L.nx || j >= L.ny || k >= L.nz) return;
+  const size_t n = ((size_t)j * L.nx + i) * L.nz + k;
+  const int q = ((lj + 1) * HI + li + 1) * HK + lk + 1;
+  // mg_Ax's sum with x from the tile
+  const long long sx = L.nz, sy = (long long)L.nx * L.nz;
+  float c[27];
+  bool ok[27];
+#pragma unroll
+  for (int dj = -1; dj <= 1; ++dj)
+#pragma unroll
+    for (int di = -1; di <= 1; ++di)
+#pragma unroll
+      for (int dk = -1; dk <= 1; ++dk) {
+        const int o = ((dj + 1) * 3 + (di + 1)) * 3 + (dk + 1);
+        ok[o] = (unsigned)(j + dj) < (unsigned)L.ny && (unsigned)(i + di) < (unsigned)L.nx &&
+                (unsigned)(k + dk) < (unsigned)L.nz;
+        const size_t g = ok[o] ? (size_t)((long long)n + dj * sy + di * sx + dk) : n;
+        c[o] = o >= 13 ? L.c14[(size_t)(o - 13) * L.n + n] : L.c14[(size_t)(13 - o) * L.n + g];
+      }
+  const double wd = L.wdinv[n], b = L.b[n];
+  mem_fence_compiler();
+  double v = 0;
+#pragma unroll
+  for (int dj = -1; dj <= 1; ++dj)
+#pragma unroll
+    for (int di = -1; di <= 1; ++di)
+#pragma unroll
+      for (int dk = -1; dk <= 1; ++dk) {
+        const int o = ((dj + 1) * 3 + (di + 1)) * 3 + (dk + 1);
+        v += ok[o] ? (double)c[o] * (double)st[q + (dj * HI + di) * HK + dk] : 0.0;
+      }
+  L.x[n] = (double)st[q] + wd * (b - v);
 }
 
 // ------------------------------------------------------------------ the solve on one XCD
@@ -2191,28 +2324,21 @@ static void launch_vcycle(const SHAPE& m, AS ms, int nblocks, unsigned K, hipStr
     hipLaunchKernelGGL(k_mg_dot_rz<AS>, dim3(nblocks, K), dim3(256), 0, s, ms);
     return;
   }
-  for (int l = 0; l < nl - 1; ++l) {
-    const dim3 g(grid_for((long long)m.L[l].n, 256), K);
-    if (l == 0) {
-      hipLaunchKernelGGL(k_mg_pre2<AS>, g, dim3(256), 0, s, ms);
-      hipLaunchKernelGGL(k_mg_resid<AS>, g, dim3(256), 0, s, ms);
-    } else {
-      hipLaunchKernelGGL(k_mg_resid1<AS>, g, dim3(256), 0, s, ms, l);
-    }
-    hipLaunchKernelGGL(k_mg_restrict<AS>, dim3(grid_for((long long)m.L[l + 1].n, 256), K), dim3(256), 0, s, ms, l);
-  }
+  auto tiles = [&](const auto& L, int i, int j, int k) {
+    return dim3((unsigned)(((L.nx + i - 1) / i) * ((L.ny + j - 1) / j) * ((L.nz + k - 1) / k)), K);
+  };
+  const dim3 g0(grid_for((long long)m.L[0].n, 256), K);
+  hipLaunchKernelGGL(k_mg_pre2<AS>, g0, dim3(256), 0, s, ms);
+  hipLaunchKernelGGL(k_mg_resid<AS>, g0, dim3(256), 0, s, ms);
+  hipLaunchKernelGGL(k_mg_restrict<AS>, dim3(grid_for((long long)m.L[1].n, 256), K), dim3(256), 0, s, ms);
+  for (int l = 1; l < nl - 1; ++l)
+    hipLaunchKernelGGL(k_mg_down<AS>, tiles(m.L[l + 1], 2, 2, 4), dim3(TILE_THREADS), 0, s, ms, l);
   hipLaunchKernelGGL(k_mg_coarse<AS>, dim3(grid_for((long long)m.nc * 64, 256), K), dim3(256), 0, s, ms);
-  for (int l = nl - 2; l >= 0; --l) {
-    const dim3 g(grid_for((long long)m.L[l].n, 256), K);
-    if (l == 0) {
-      hipLaunchKernelGGL(k_mg_prolong<AS>, g, dim3(256), 0, s, ms);
-      hipLaunchKernelGGL(k_mg_post0a<AS>, g, dim3(256), 0, s, ms);
-      hipLaunchKernelGGL(k_mg_sweep_last<AS>, dim3(nblocks, K), dim3(256), 0, s, ms);
-    } else {
-      hipLaunchKernelGGL(k_mg_prolong1<AS>, g, dim3(256), 0, s, ms, l);
-      hipLaunchKernelGGL(k_mg_post1<AS>, g, dim3(256), 0, s, ms, l);
-    }
-  }
+  for (int l = nl - 2; l > 0; --l)
+    hipLaunchKernelGGL(k_mg_up<AS>, tiles(m.L[l], 4, 8, 8), dim3(TILE_THREADS), 0, s, ms, l);
+  hipLaunchKernelGGL(k_mg_prolong<AS>, g0, dim3(256), 0, s, ms);
+  hipLaunchKernelGGL(k_mg_post0a<AS>, g0, dim3(256), 0, s, ms);
+  hipLaunchKernelGGL(k_mg_sweep_last<AS>, dim3(nblocks, K), dim3(256), 0, s, ms);
 }
 
 // the cycle's argument block of the solve's start (r.z partials into part_rz0,
