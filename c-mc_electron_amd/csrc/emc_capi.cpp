@@ -1655,14 +1655,20 @@ static int run_pcg_with(emc_ctx* c, const PA& a, const MA& mg, double rtol, int 
   return finish_pcg(c, rtol, iters, relres);
 }
 
+// ||r|| / ||b|| from a solve's scalars, NaN for a residual that is none (which a
+// std::max with 0 would turn into 0)
+static double rel_residual(const double* scal) {
+  const double bn = std::sqrt(scal[2]) > 0 ? std::sqrt(scal[2]) : 1.0;
+  return std::sqrt(scal[0] < 0.0 ? 0.0 : scal[0]) / bn;
+}
+
 static int finish_pcg(emc_ctx* c, double rtol, int* iters, double* relres) {
   Gpu& g = *c->gpu;
   if (!g.pcg_pending) return EMC_OK;
   g.pcg_pending = false;
   const double* sh = g.pcg_result;
-  const double bn = std::sqrt(sh[2]) > 0 ? std::sqrt(sh[2]) : 1.0;
   const int it = (int)sh[3];
-  const double rel = std::sqrt(std::max(0.0, sh[0])) / bn;
+  const double rel = rel_residual(sh);
   if (!std::isfinite(rel)) return fail(c, EMC_ERR_SOLVER, "PCG residual is not finite");
   if (iters) *iters = it;
   if (relres) *relres = rel;
@@ -1743,8 +1749,7 @@ static int run_pcg_mixed(emc_ctx* c, const double* b, double* x, double rtol, in
     HIPCHECK(c, emc_launch_refine_resid(ra, g.stream));
     HIPCHECK(c, hipMemcpyAsync(sh, ra.a.scal, 8 * sizeof(double), hipMemcpyDeviceToHost, g.stream));
     HIPCHECK(c, hipStreamSynchronize(g.stream));
-    const double bn = std::sqrt(sh[2]) > 0 ? std::sqrt(sh[2]) : 1.0;
-    rel = std::sqrt(std::max(0.0, sh[0])) / bn;
+    rel = rel_residual(sh);
     if (!std::isfinite(rel)) return fail(c, EMC_ERR_SOLVER, "residual of the refinement is not finite");
     if (rel <= rtol) break;
     if (outer >= maxit_outer) return fail(c, EMC_ERR_SOLVER, "iterative refinement did not reach the tolerance");
@@ -2925,8 +2930,7 @@ static int batch_one_step(emc_batch* b, emc_fly_tallies* acc, double tsum[5], in
     Gpu& g = *c->gpu;
     if (last >= 0) {
       const double* sh = b->h_scal + (size_t)(last & 1) * 8 * K + 8 * q;
-      const double bn = std::sqrt(sh[2]) > 0 ? std::sqrt(sh[2]) : 1.0;
-      const double rel = std::sqrt(std::max(0.0, sh[0])) / bn;
+      const double rel = rel_residual(sh);
       c->last_pcg_iters = (int)sh[3];
       c->last_relres = rel;
       imax = std::max(imax, (int)sh[3]);
