@@ -1347,6 +1347,9 @@ static int sync_fly_const(emc_ctx* c) {
   return EMC_OK;
 }
 
+// the gate of a step whose solve the host has not seen yet
+static const int* solve_gate(const Gpu& g) { return g.pcg_pending ? g.done : nullptr; }
+
 static FlyArgs fly_args(emc_ctx* c, uint64_t step, int flag_heat) {
   Gpu& g = *c->gpu;
   FlyArgs a{};
@@ -1357,7 +1360,7 @@ static FlyArgs fly_args(emc_ctx* c, uint64_t step, int flag_heat) {
   a.dead = g.dead; a.ndead = g.ctr + 1; a.dead_cap = g.dead_cap;
   a.slow = g.slow; a.nslow = g.ctr + 3;
   a.wave_slots = g.wave_slots;
-  a.gate = g.pcg_pending ? g.done : nullptr;  // a step whose solve the host has not seen yet
+  a.gate = solve_gate(g);
   return a;
 }
 
@@ -1542,6 +1545,7 @@ static FieldArgs field_args(emc_ctx* c, const double* pot, bool rho_from_cells) 
   const Phys& p = d.phys;
   FieldArgs a{};
   a.ncell = d.ncell; a.cnx = d.cnx; a.cny = d.cny; a.cnz = d.cnz; a.pnx = d.pnx; a.pny = d.pny; a.pnz = d.pnz;
+  a.gate = solve_gate(g);
   a.pot = pot; a.dx = g.dx; a.dy = g.dy; a.dz = g.dz; a.cvol = g.cvol; a.da = g.da; a.eeff_dir = g.eeff;
   a.cell_q = rho_from_cells ? g.cell_q : nullptr;
   a.ex = g.ex; a.ey = g.ey; a.ez = g.ez; a.rho = g.rho;
@@ -2459,13 +2463,12 @@ static int launch_fields(emc_ctx* c, const double* pot_h, const double* pot_e, b
 // potential at the nodes of the quantum region when active.
 static int launch_qc(emc_ctx* c, const double* pot, double* out, bool active) {
   Gpu& g = *c->gpu;
-  HIPCHECK(c, hipMemcpyAsync(out, pot, c->dev.nnode * 8, hipMemcpyDeviceToDevice, g.stream));
-  if (active) {
-    QcArgs a = g.qa;
-    a.pot = pot;
-    a.qc_pot = out;
-    HIPCHECK(c, emc_launch_qc_potential(a, g.stream));
-  }
+  QcArgs a = g.qa;
+  a.gate = solve_gate(g);
+  a.nnode = c->dev.nnode;
+  a.pot = pot;
+  a.qc_pot = out;
+  HIPCHECK(c, emc_launch_qc_potential(a, active, g.stream));
   return EMC_OK;
 }
 
@@ -2536,6 +2539,8 @@ static int one_step(emc_ctx* c, bool heat_phase, emc_fly_tallies* acc, double ts
   }
   const uint64_t count = heat_phase ? c->heat_next++ : c->next_step++;
   const uint64_t step = heat_phase ? HEAT_STEP0 + count : count;
+  // no later call's kernels are gated by a solve of this step
+  struct Pending { bool& p; ~Pending() { p = false; } } pending{g.pcg_pending};
   HIPCHECK(c, hipEventRecord(g.ev[0], g.stream));
   int st = run_sort(c);
   if (st) return st;

@@ -20,6 +20,11 @@ struct FlyConst {
   FieldsDev F;
 };
 
+// The kernels a step queues behind its solve before the host has seen the result do
+// nothing when the solve failed: their `gate` (null: no solve to wait for) points at a
+// word that is GATE_SHUT then.
+constexpr int GATE_SHUT = 2;
+
 struct FlyArgs {
   const FlyConst* C;           // device memory
   TallyDev T;
@@ -36,7 +41,7 @@ struct FlyArgs {
   uint32_t* slow;              // [cap] particles k_fly_fast hands to k_fly_slow
   unsigned long long* nslow;   // device counter, zero before the flight
   long long wave_slots;        // waves the GPU runs at once (CUs x 4 SIMDs)
-  const int* gate;             // may be null; *gate == 2: the step's solve failed, nothing flies
+  const int* gate;             // see GATE_SHUT
 };
 
 // Deposit tiles: TILE_I x TILE_J x TILE_K cells (i, j, k) per workgroup; a tile's
@@ -109,6 +114,8 @@ struct StatArgs {
 // Quantum-correction effective potential at the nodes of the quantum region
 // (effective_potential, src/mcmodel.cpp:2337-2376), from tables built on the host.
 struct QcArgs {
+  const int* gate;                          // see GATE_SHUT
+  size_t nnode;
   long long nq;                             // nodes of the quantum region
   int pnx, pny, pnz;
   int wlen[3];                              // window length per axis (table row stride)
@@ -122,7 +129,7 @@ struct QcArgs {
   const double* w[3];                       // per axis: erf differences [target][src - lo][shape]
   double eb;                                // normalised barrier
   const double* pot;                        // Poisson potential
-  double* qc_pot;                           // effective potential (quantum nodes written)
+  double* qc_pot;                           // effective potential
 };
 
 struct DepositArgs {
@@ -145,6 +152,7 @@ struct DepositArgs {
 struct FieldArgs {
   size_t ncell;
   int cnx, cny, cnz, pnx, pny, pnz;
+  const int* gate;  // see GATE_SHUT
   const double *pot, *dx, *dy, *dz, *cvol, *da;
   const int* eeff_dir;
   const unsigned long long* cell_q;  // null: rho is an input
@@ -353,7 +361,8 @@ hipError_t emc_launch_tile_sort(const emc::SortArgs& a, long long nappend, hipSt
 // nitem: an upper bound of the work items
 hipError_t emc_launch_deposit(const emc::DepositArgs& a, long long nitem, hipStream_t s);
 hipError_t emc_launch_rhs(const emc::RhsArgs& a, hipStream_t s);
-hipError_t emc_launch_qc_potential(const emc::QcArgs& a, hipStream_t s);
+// qc_pot = pot, then with `active` the effective potential at the quantum nodes
+hipError_t emc_launch_qc_potential(const emc::QcArgs& a, bool active, hipStream_t s);
 hipError_t emc_launch_field(const emc::FieldArgs& a, hipStream_t s);
 hipError_t emc_launch_zero(unsigned long long* p, size_t n, hipStream_t s);
 int emc_pcg_blocks(size_t n);

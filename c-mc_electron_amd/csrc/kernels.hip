@@ -62,6 +62,9 @@ __device__ inline void finish_drop(const TallyDev& T, const Flight& f) {
   if (f.drop_reason >= 0) atomicAdd(&T.counters[CNT_DROP0 + f.drop_reason], 1ull);
 }
 
+// the step's solve failed: what was queued behind it does nothing
+__device__ __forceinline__ bool shut(const int* gate) { return gate && *gate == GATE_SHUT; }
+
 // ------------------------------------------------------------------ flight
 // the flight's descriptors as constant memory (see EMC_CST)
 __device__ __forceinline__ const EMC_CST FlyConst& fly_const(const FlyConst* c) {
@@ -93,7 +96,7 @@ __device__ inline void load_particle(Flight& f, const FlyArgs& a, long long q, u
 template <class AS>
 __global__ __launch_bounds__(256, 3) void k_fly_fast(AS as_) {
   const FlyArgs& a = kargs(as_);
-  if (a.gate && *a.gate == 2) return;  // no particle is listed, none flies
+  if (shut(a.gate)) return;  // no particle is listed, none flies
   const long long stride = (long long)gridDim.x * blockDim.x;
   long long ev = 0;
   const int lane = threadIdx.x & 63;
@@ -896,6 +899,7 @@ __global__ __launch_bounds__(256) void k_deposit_gather(AS as_) {
 // Reads every term's five words from memory; only for windows that do not fit a
 // block's LDS (k_qc_potential).
 __global__ __launch_bounds__(256) void k_qc_potential_nodes(QcArgs a) {
+  if (shut(a.gate)) return;
   const long long stride = (long long)gridDim.x * blockDim.x;
   for (long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x; q < a.nq; q += stride) {
     const int p = a.qnodes[q];
@@ -951,6 +955,7 @@ __global__ __launch_bounds__(QC_THREADS) void k_qc_potential(QcArgs a) {
   __shared__ double v[2][QC_PLANE];
   __shared__ uint8_t sh[2][QC_PLANE];
   __shared__ double wt[QC_TABLE];
+  if (shut(a.gate)) return;
   const QcChunk c = a.chunks[blockIdx.x];
   const int tid = threadIdx.x, tgt = tid >> 1, g = tid & 1;
   const bool on = tgt < c.count;
@@ -1049,6 +1054,13 @@ __global__ __launch_bounds__(QC_THREADS) void k_qc_potential(QcArgs a) {
   if (on && g == 0) a.qc_pot[p] = ret * 0.125;
 }
 
+// outside the quantum region the effective potential is the potential
+__global__ void k_qc_start(QcArgs a) {
+  if (shut(a.gate)) return;
+  const size_t stride = (size_t)gridDim.x * blockDim.x;
+  for (size_t n = (size_t)blockIdx.x * blockDim.x + threadIdx.x; n < a.nnode; n += stride) a.qc_pot[n] = a.pot[n];
+}
+
 __global__ void k_rhs(RhsArgs a) {
   const size_t stride = (size_t)gridDim.x * blockDim.x;
   for (size_t n = (size_t)blockIdx.x * blockDim.x + threadIdx.x; n < a.nnode; n += stride) {
@@ -1061,6 +1073,7 @@ __global__ void k_rhs(RhsArgs a) {
 template <class AS>
 __global__ void k_field(AS as_) {
   const FieldArgs& a = kargs(as_);
+  if (shut(a.gate)) return;
   const size_t stride = (size_t)gridDim.x * blockDim.x;
   const int cnx = a.cnx, cnz = a.cnz, pnx = a.pnx, pnz = a.pnz;
   for (size_t c = (size_t)blockIdx.x * blockDim.x + threadIdx.x; c < a.ncell; c += stride) {
@@ -2291,8 +2304,9 @@ hipError_t emc_launch_rhs(const RhsArgs& a, hipStream_t s) {
   hipLaunchKernelGGL(k_rhs, dim3(grid_for((long long)a.nnode, 256)), dim3(256), 0, s, a);
   return hipGetLastError();
 }
-hipError_t emc_launch_qc_potential(const QcArgs& a, hipStream_t s) {
-  if (a.nq <= 0) return hipSuccess;
+hipError_t emc_launch_qc_potential(const QcArgs& a, bool active, hipStream_t s) {
+  hipLaunchKernelGGL(k_qc_start, dim3(grid_for((long long)a.nnode, 256, 1024)), dim3(256), 0, s, a);
+  if (!active || a.nq <= 0) return hipGetLastError();
   if (a.nchunk > 0) hipLaunchKernelGGL(k_qc_potential, dim3(a.nchunk), dim3(QC_THREADS), 0, s, a);
   else hipLaunchKernelGGL(k_qc_potential_nodes, dim3(grid_for(a.nq, 256)), dim3(256), 0, s, a);
   return hipGetLastError();
