@@ -2584,10 +2584,14 @@ static int one_step(emc_ctx* c, bool heat_phase, emc_fly_tallies* acc, double ts
   HIPCHECK(c, hipEventRecord(g.ev[4], g.stream));
   HIPCHECK(c, hipEventSynchronize(g.ev[4]));
   // the one wait of the step: the solve's result, then the flight's counts
+  int solved = EMC_OK;
   if (!heat_phase) {
-    st = finish_pcg(c, c->opts.poisson_rtol, nullptr, nullptr);
-    if (st) return st;
+    // was the gate shut?
+    const bool held = g.pcg_pending && xcd_solve(c) && !std::isfinite(g.pcg_result[0]);
+    solved = finish_pcg(c, c->opts.poisson_rtol, nullptr, nullptr);
+    if (solved && held) return solved;
   }
+  // flown, also behind a solve that missed its tolerance: the step is taken up first
   const int passes = finish_fly(c, fa);
   if (passes < 0) return passes;
   // MultipleRefresh after the flight of every mr_step-th step (src/mcmodel.cpp:535-547)
@@ -2610,7 +2614,7 @@ static int one_step(emc_ctx* c, bool heat_phase, emc_fly_tallies* acc, double ts
   if (acc) acc->n_mr_gen += mr_gen;
   c->win.n_mr_gen += mr_gen;
   ++c->win_steps;
-  return EMC_OK;
+  return solved;
 }
 
 static int run_steps(emc_ctx* c, int nsteps, emc_fly_tallies* acc, bool heat_phase) {
@@ -2667,7 +2671,8 @@ struct emc_batch {
   int nmem = 0;                        // blocks per device of the one-launch solve, 0: kernel by kernel
   BatchTables bt{};
   const CopyArgs *cp_n = nullptr, *cp_scal = nullptr, *cp_tally = nullptr, *cp_zero = nullptr;
-  unsigned long long* d_n = nullptr;   // [K] live counts after the sort
+  unsigned long long* d_n = nullptr;   // [K] live counts after the sort, then the gate
+  int* gate = nullptr;                 // shut when the one-launch solve of any device failed
   double* d_scal = nullptr;            // [2][K][8] PCG scalars of the last two iterations
   unsigned long long* d_tally = nullptr;  // [K][FLYOUT_N]
   unsigned long long* h_n = nullptr;
@@ -2746,12 +2751,13 @@ static int batch_setup(emc_batch* b) {
   const bool f32 = c0->opts.poisson_fp32 == 2;
   b->off_fmg = place(f32 ? 3 * K * sizeof(MgArgsT<float>) : 0);
   b->off_field = place(K * sizeof(FieldArgs));
-  b->off_cp = place(5 * K * sizeof(CopyArgs));
+  b->off_cp = place((5 * K + 1) * sizeof(CopyArgs));
   b->nmem = xcd_solve(c0) ? emc_xcd_blocks(b->nnode, K, g0.ncu) : 0;
   b->off_xcd = place(!b->nmem ? 0 : K * (f32 ? sizeof(XcdArgsT<double, float>) : sizeof(XcdArgsT<double, double>)));
   b->tab_bytes = off;
   b->d_tab = b->mem.alloc<unsigned char>(off);
-  b->d_n = b->mem.alloc<unsigned long long>(K);
+  b->d_n = b->mem.alloc<unsigned long long>(K + 1);
+  b->gate = (int*)(b->d_n + K);
   b->d_scal = b->mem.alloc<double>(2 * 8 * (size_t)K);
   b->d_tally = b->mem.alloc<unsigned long long>((size_t)K * FLYOUT_N);
   if (b->mem.last != hipSuccess) return bfail(b, EMC_ERR_HIP, std::string("batch tables: ") + hipGetErrorString(b->mem.last));
@@ -2779,10 +2785,10 @@ static int batch_setup(emc_batch* b) {
   else if (b->nmem) b->bt.xcd = (const XcdArgsT<double, double>*)(b->d_tab + b->off_xcd);
   b->bt.field = (const FieldArgs*)(b->d_tab + b->off_field);
   const CopyArgs* cp = (const CopyArgs*)(b->d_tab + b->off_cp);
-  b->cp_n = cp;
-  b->cp_scal = cp + K;  // [2][K]
-  b->cp_tally = cp + 3 * K;
-  b->cp_zero = cp + 4 * K;
+  b->cp_n = cp;  // [K + 1]
+  b->cp_scal = cp + K + 1;  // [2][K]
+  b->cp_tally = b->cp_scal + 2 * K;
+  b->cp_zero = b->cp_tally + K;
   // the tables that stay: solver, cycle, fields, readbacks
   PcgArgs* hp = (PcgArgs*)(b->h_tab + b->off_pcg);
   MgArgs* hm = (MgArgs*)(b->h_tab + b->off_mg);
@@ -2812,19 +2818,22 @@ static int batch_setup(emc_batch* b) {
         t[q].maxit = c->opts.poisson_maxit;
         t[q].nmem = b->nmem;
         t[q].xcd = q % 8;
+        t[q].gate = b->gate;
       };
       if (f32) fill((XcdArgsT<double, float>*)(b->h_tab + b->off_xcd), hfm[q]);
       else fill((XcdArgsT<double, double>*)(b->h_tab + b->off_xcd), hm[q]);
     }
     hf[q] = field_args(c, g.pot, true);
+    hf[q].gate = b->nmem ? b->gate : nullptr;
     int st = sync_fly_const(c);
     if (st) return bfail(b, st, c->err);
     hc[q] = CopyArgs{g.toff + g.ntile, b->d_n + q, 1, 1, 0};  // the live count, a 32-bit word
-    hc[K + q] = CopyArgs{g.scal, (unsigned long long*)(b->d_scal + 8 * (size_t)q), 8, 0, 0};
-    hc[2 * K + q] = CopyArgs{g.scal, (unsigned long long*)(b->d_scal + 8 * ((size_t)K + q)), 8, 0, 0};
-    hc[3 * K + q] = CopyArgs{g.contact, b->d_tally + (size_t)q * FLYOUT_N, FLYOUT_N, 0, 0};
-    hc[4 * K + q] = CopyArgs{nullptr, g.contact, FLYOUT_N, 0, 0};
+    hc[K + 1 + q] = CopyArgs{g.scal, (unsigned long long*)(b->d_scal + 8 * (size_t)q), 8, 0, 0};
+    hc[2 * K + 1 + q] = CopyArgs{g.scal, (unsigned long long*)(b->d_scal + 8 * ((size_t)K + q)), 8, 0, 0};
+    hc[3 * K + 1 + q] = CopyArgs{g.contact, b->d_tally + (size_t)q * FLYOUT_N, FLYOUT_N, 0, 0};
+    hc[4 * K + 1 + q] = CopyArgs{nullptr, g.contact, FLYOUT_N, 0, 0};
   }
+  hc[K] = CopyArgs{nullptr, b->d_n + K, 1, 0, 0};  // the gate opens
   BHIP(b, hipMemcpyAsync(b->d_tab + b->off_pcg, b->h_tab + b->off_pcg, b->tab_bytes - b->off_pcg,
                          hipMemcpyHostToDevice, b->s));
   BHIP(b, hipStreamSynchronize(b->s));
@@ -2865,8 +2874,8 @@ static int batch_one_step(emc_batch* b, emc_fly_tallies* acc, double tsum[5], in
   BHIP(b, hipMemcpyAsync(b->d_tab + b->off_sort, b->h_tab + b->off_sort, b->off_fly - b->off_sort,
                          hipMemcpyHostToDevice, s));
   BHIP(b, emc_launch_tile_sort_b(b->bt, b->ntile, nmax, s));
-  // the live counts (32-bit toff[ntile] of each device) into d_n
-  BHIP(b, emc_launch_copy_b(b->cp_n, K, 1, s));
+  // the live counts (32-bit toff[ntile] of each device) into d_n; the gate opens
+  BHIP(b, emc_launch_copy_b(b->cp_n, K + 1, 1, s));
   BHIP(b, hipMemcpyAsync(b->h_n, b->d_n, K * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
   BHIP(b, hipEventRecord(b->ev_n, s));
   BHIP(b, emc_launch_deposit_b(b->bt, b->ntile, nitem, b->nnode, s));
@@ -2916,7 +2925,7 @@ static int batch_one_step(emc_batch* b, emc_fly_tallies* acc, double tsum[5], in
     g.sorted_n = g.n;
     g.n_pending = false;
     hfl[q] = fly_args(c, step[q], 0);
-    hfl[q].gate = b->nmem ? g.done : nullptr;
+    hfl[q].gate = b->nmem ? b->gate : nullptr;
     nmax = std::max(nmax, g.n);
   }
   BHIP(b, hipMemcpyAsync(b->d_tab + b->off_fly, b->h_tab + b->off_fly, K * sizeof(FlyArgs), hipMemcpyHostToDevice, s));
@@ -2928,19 +2937,26 @@ static int batch_one_step(emc_batch* b, emc_fly_tallies* acc, double tsum[5], in
                          hipMemcpyDeviceToHost, s));
   BHIP(b, hipEventRecord(b->ev[4], s));
   BHIP(b, hipEventSynchronize(b->ev[4]));
-  // per device: the solve's result, the flight's counts (finish_fly), the window
-  int imax = 0;
-  for (int q = 0; q < K; ++q) {
+  const double* scal = b->h_scal + (size_t)(last & 1) * 8 * K;
+  // a residual that is none shut the gate: no device has taken its step
+  if (b->nmem)
+    for (int q = 0; q < K; ++q)
+      if (!std::isfinite(scal[8 * q])) return bfail(b, EMC_ERR_SOLVER, "PCG residual is not finite");
+  // per device: the solve's result, the flight's counts (finish_fly), the window.
+  // Every device has flown, so an error of one waits until all are taken up.
+  int imax = 0, first_error = EMC_OK;
+  auto take = [&](int q) -> int {
     emc_ctx* c = b->c[q];
     Gpu& g = *c->gpu;
+    int solved = EMC_OK;
     if (last >= 0) {
-      const double* sh = b->h_scal + (size_t)(last & 1) * 8 * K + 8 * q;
+      const double* sh = scal + 8 * q;
       const double rel = rel_residual(sh);
       c->last_pcg_iters = (int)sh[3];
       c->last_relres = rel;
       imax = std::max(imax, (int)sh[3]);
-      if (!std::isfinite(rel)) return bfail(b, EMC_ERR_SOLVER, "PCG residual is not finite");
-      if (rel > c->opts.poisson_rtol) return bfail(b, EMC_ERR_SOLVER, "PCG did not reach the tolerance");
+      if (!std::isfinite(rel)) solved = bfail(b, EMC_ERR_SOLVER, "PCG residual is not finite");
+      else if (rel > c->opts.poisson_rtol) solved = bfail(b, EMC_ERR_SOLVER, "PCG did not reach the tolerance");
     }
     std::memcpy(g.tally_host, b->h_tally + (size_t)q * FLYOUT_N, FLYOUT_N * sizeof(unsigned long long));
     const int passes = finish_fly(c, hfl[q]);
@@ -2960,7 +2976,13 @@ static int batch_one_step(emc_batch* b, emc_fly_tallies* acc, double tsum[5], in
     ++c->win_steps;
     // work finish_fly or the refresh queued on the device's own stream
     BHIP(b, hipStreamSynchronize(g.stream));
+    return solved;
+  };
+  for (int q = 0; q < K; ++q) {
+    const int st = take(q);
+    if (st && !first_error) first_error = st;
   }
+  if (first_error) return first_error;
   *iters_max = imax;
   float ms;
   for (int q = 0; q < 3; ++q) {

@@ -179,7 +179,8 @@ struct PcgArgsT {
   R *x, *r, *p, *p2, *q, *z;  // p and p2: search direction of even and odd iterations
   double *part_a, *part_pq, *part_rr, *part_rz0, *part_rz1;  // block partial sums: part_a [3*nblocks], the others [nblocks]
   double* scal;  // [0] r.r [1] r.z [2] b.b [3] iterations done [4] r.r at the tolerance
-  int* done;     // set once r.r reaches scal[4]: every later CG / V-cycle kernel returns at once
+  int* done;     // set once r.r reaches scal[4]: every later CG / V-cycle kernel returns at once;
+                 // GATE_SHUT after a solve in one launch that failed
   double rtol;
   int pad0;
   // FP32 preconditioner of the FP64 CG (null otherwise): the residual is also
@@ -240,6 +241,7 @@ struct XcdArgsT {
   XcdSync* sync;
   int maxit, nmem;  // nmem: blocks per device
   int xcd, pad;     // the XCD they run on
+  int* gate;        // shut when the solve fails, for all devices of a batch; null for one device (PcgArgsT::done)
 };
 
 // Iterative refinement of the mixed-precision solve: r = b - A x in FP64, its

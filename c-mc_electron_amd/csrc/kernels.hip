@@ -2134,7 +2134,9 @@ __global__ __launch_bounds__(XCD_THREADS) void k_pcg_xcd(AS as_) {
     }
     if (me == 0 && threadIdx.x == 0) {
       a.scal[0] = rr; a.scal[1] = rz; a.scal[2] = bb; a.scal[3] = it; a.scal[4] = tol;
-      *a.done = dead || !isfinite(rr) ? 2 : 1;  // 2: the step's flight is not to run
+      const bool bad = dead || !isfinite(rr);
+      *a.done = bad ? GATE_SHUT : 1;
+      if (bad && w.gate) *w.gate = GATE_SHUT;
     }
     if (dead && threadIdx.x == 0) a.scal[0] = __builtin_nan("");
   }

@@ -1,7 +1,7 @@
 """A step whose Poisson solve fails (a potential that is not finite) returns the
 solver's error before the fields, the corrected potential and the flight: fields,
-population and counts stay as they were, and stepping goes on from there once the
-potential is good again."""
+population and counts stay as they were, for the device and for every other device
+of its batch, and stepping goes on from there once the potential is good again."""
 import numpy as np
 import pytest
 
@@ -63,3 +63,78 @@ def test_step_leaves_the_state(refine, qc):
             assert np.isfinite(w["stat_qc_pot"]).all()
     finally:
         e.close()
+
+
+@pytest.mark.parametrize("refine,bad", [(1, 0), (1, 1), (1, 2), (2, 1)])
+def test_batch_leaves_every_device(refine, bad):
+    def engines():
+        out = []
+        for q in range(3):
+            e = emcgpu.Engine(cfg1_deck(refine=refine, electrons=4000 + 500 * q, holes=400, vd=0.2 + 0.1 * q), device=0,
+                              seed=5 + q)
+            e.particles_init()
+            out.append(e)
+        return out
+    together, alone = engines(), engines()
+    b = emcgpu.Batch(together)
+    try:
+        b.step(2)
+        before = [state(e) for e in together]
+        start = [(e.potential(), e.fields_get().rho.copy()) for e in together]
+        spoil(together[bad])
+        failing(lambda: b.step(1))
+        for q, e in enumerate(together):
+            same(state(e), before[q], f"device {q} after the failed step")
+        # the others' solves may have moved their start: put it back for all
+        for e, (pot, rho) in zip(together, start):
+            e.compute_field(pot, rho)
+        acc = b.step(2)
+        for q, e in enumerate(alone):
+            # a device alone whose own step failed in between
+            e.step(2)
+            pot, rho = spoil(e)
+            failing(lambda: e.step(1))
+            e.compute_field(pot, rho)
+            t = e.step(2)
+            same(state(together[q]), state(e), f"device {q}")
+            np.testing.assert_array_equal(together[q].potential(), e.potential())
+            for k, v in emcgpu.tallies_dict(t).items():
+                np.testing.assert_array_equal(emcgpu.tallies_dict(acc[q])[k], v, err_msg=f"device {q} {k}")
+    finally:
+        b.close()
+        for e in together + alone:
+            e.close()
+
+
+def test_step_that_missed_the_tolerance_is_taken_up():
+    """One iteration allowed: the step reports the solver's error, but it has flown,
+    and its clones, tallies and window are the device's, alone and in a batch."""
+    def engines():
+        out = []
+        for q in range(3):
+            e = emcgpu.Engine(cfg1_deck(electrons=6000 + 500 * q, holes=600, vd=0.2 + 0.1 * q), device=0, seed=5 + q,
+                              poisson_maxit=1)
+            e.particles_init()
+            out.append(e)
+        return out
+    together, alone = engines(), engines()
+    b = emcgpu.Batch(together)
+    try:
+        for step in range(6):
+            failing(lambda: b.step(1))
+            for e in alone:
+                failing(lambda: e.step(1))
+        made = 0
+        for q, (e, f) in enumerate(zip(together, alone)):
+            same(state(e), state(f), f"device {q}")
+            w, v = e.stat_window(), f.stat_window()
+            assert w["steps"] == v["steps"] == 6
+            t = emcgpu.tallies_dict(w["tallies"])
+            for k, x in emcgpu.tallies_dict(v["tallies"]).items():
+                np.testing.assert_array_equal(t[k], x, err_msg=f"device {q} {k}")
+            made += t["n_gen"]
+        assert made > 0  # the contacts put carriers in
+    finally:
+        b.close()
+        for e in together + alone:
+            e.close()
