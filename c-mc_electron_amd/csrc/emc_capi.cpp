@@ -29,6 +29,23 @@
 
 using namespace emc;
 
+// When a one-launch solve could not be finished (XCD_STATUS), the next ones go kernel by
+// kernel, twice as many each time in a row: what holds the XCD up, another solver's
+// blocks or another process, is likely still there, and a try costs up to its wait.
+struct OneLaunch {
+  int hold = 0, next = 8;
+  bool use() {
+    if (hold <= 0) return true;
+    --hold;
+    return false;
+  }
+  void done() { next = 8; }
+  void failed() {
+    hold = next;
+    next = std::min(2 * next, 1024);
+  }
+};
+
 struct DevBand;
 
 namespace {
@@ -146,6 +163,11 @@ struct Gpu {
   int* done = nullptr;
   XcdSync* sync = nullptr;            // the one-launch solve's words (zero between launches)
   int xcd = 0, ncu = 0;               // the XCD this context's solves run on; CUs of the GPU
+  int form = EMC_SOLVE_AUTO;          // emc_poisson_form
+  OneLaunch one;
+  double* x0 = nullptr;               // the start of a one-launch solve, for its redo
+  bool pcg_one = false;               // the pending solve went in one launch
+  int64_t redone = 0;                 // solves redone kernel by kernel
   MgArgs mg{};                        // device view of the multigrid hierarchy
   // FP32 copies for the bulk of the mixed-precision solve, made on its first use:
   // the level-0 operator, the hierarchy's vectors, damped inverse diagonals and
@@ -502,6 +524,10 @@ static std::string device_band(emc_ctx* c, std::shared_ptr<DevBand>& out) {
   return "";
 }
 
+// Whether the context's solves can go in one launch on one XCD (k_pcg_xcd): meshes
+// whose solve is bound by its launches.
+static bool xcd_solve(const emc_ctx* c) { return c->dev.nnode <= XCD_MAX_NODES && c->gpu->ncu >= 8; }
+
 static int gpu_setup(emc_ctx* c) {
   int ndev = 0;
   if (hipGetDeviceCount(&ndev) != hipSuccess || ndev <= c->opts.device)
@@ -599,6 +625,7 @@ static int gpu_setup(emc_ctx* c) {
   g.scal = m.alloc<double>(8);
   g.done = m.alloc<int>(1);
   g.sync = m.alloc<XcdSync>(1);
+  if (xcd_solve(c)) g.x0 = m.alloc<double>(NN);
   {
     const std::string e = ensure_mg(c);
     if (!e.empty()) return fail(c, EMC_ERR_DECK, e);
@@ -1347,8 +1374,8 @@ static int sync_fly_const(emc_ctx* c) {
   return EMC_OK;
 }
 
-// the gate of a step whose solve the host has not seen yet
-static const int* solve_gate(const Gpu& g) { return g.pcg_pending ? g.done : nullptr; }
+// the gate of a step whose one-launch solve the host has not seen yet
+static const int* solve_gate(const Gpu& g) { return g.pcg_pending && g.pcg_one ? g.done : nullptr; }
 
 static FlyArgs fly_args(emc_ctx* c, uint64_t step, int flag_heat) {
   Gpu& g = *c->gpu;
@@ -1580,11 +1607,12 @@ static PcgArgs pcg_args(emc_ctx* c, const double* b, double* x, double rtol) {
 // With `defer` the solve is only queued past its last check: the result (iteration
 // count, residual) is read by finish_pcg() once the stream has passed it.
 static int finish_pcg(emc_ctx* c, double rtol, int* iters, double* relres);
+// A deferred solve that went in one launch may have to be redone (solve_redo).
 template <class PA, class MA>
 static int run_pcg_with(emc_ctx* c, const PA& a, const MA& mg, double rtol, int maxit, int* iters, double* relres,
-                        bool defer);
+                        bool defer, bool kernels = false);
 static int run_pcg(emc_ctx* c, const double* b, double* x, double rtol, int maxit, int* iters, double* relres,
-                   bool defer = false) {
+                   bool defer = false, bool kernels = false) {
   Gpu& g = *c->gpu;
   if (c->opts.poisson_fp32 == 2) {
     // FP64 CG, FP32 cycle
@@ -1593,24 +1621,41 @@ static int run_pcg(emc_ctx* c, const double* b, double* x, double rtol, int maxi
     PcgArgs a = pcg_args(c, b, x, rtol);
     a.r32 = g.r32;
     a.z32 = g.z32;
-    return run_pcg_with(c, a, g.pmg, rtol, maxit, iters, relres, defer);
+    return run_pcg_with(c, a, g.pmg, rtol, maxit, iters, relres, defer, kernels);
   }
-  return run_pcg_with(c, pcg_args(c, b, x, rtol), g.mg, rtol, maxit, iters, relres, defer);
+  return run_pcg_with(c, pcg_args(c, b, x, rtol), g.mg, rtol, maxit, iters, relres, defer, kernels);
 }
 
-// Whether the context's solves go in one launch on one XCD (k_pcg_xcd): meshes whose
-// solve is bound by its launches.
-static bool xcd_solve(const emc_ctx* c) { return c->dev.nnode <= XCD_MAX_NODES && c->gpu->ncu >= 8; }
+// The bounds of the one-launch solve's waits in the context's form.
+static void xcd_waits(int form, long long& meet, long long& wait) {
+  meet = form == EMC_SOLVE_NO_MEET ? -1 : XCD_MEET;
+  wait = form == EMC_SOLVE_NO_WAIT ? -40 : XCD_WAIT;  // a barrier of the second iteration
+}
+
+// After the stream has passed a one-launch solve: 1 when it is to be redone kernel by
+// kernel, x (of `bytes`) being set back to its start on `s`; 0 when it ran to its end.
+static int solve_redo(emc_ctx* c, const double* scal, void* x, size_t bytes, hipStream_t s) {
+  Gpu& g = *c->gpu;
+  if (scal[XCD_STATUS] == XCD_SOLVED) {
+    g.one.done();
+    return 0;
+  }
+  g.one.failed();
+  ++g.redone;
+  if (scal[XCD_STATUS] == XCD_GIVEN_UP) HIPCHECK(c, hipMemcpyAsync(x, g.x0, bytes, hipMemcpyDeviceToDevice, s));
+  return 1;
+}
 
 // The solve on explicit work vectors: `a` and `mg` name every buffer the
 // kernels write (the solve of the context uses its own, emc_poisson_solve_ws a
 // caller's workspace).
 template <class PA, class MA>
 static int run_pcg_with(emc_ctx* c, const PA& a, const MA& mg, double rtol, int maxit, int* iters, double* relres,
-                        bool defer) {
+                        bool defer, bool kernels) {
   Gpu& g = *c->gpu;
   double* sh = g.scal_host;
-  if (xcd_solve(c)) {
+  g.pcg_one = false;
+  if (!kernels && xcd_solve(c) && g.form != EMC_SOLVE_KERNELS && (g.form != EMC_SOLVE_AUTO || g.one.use())) {
     XcdArgsT<typename PA::real, typename MA::real> w{};
     w.a = a;
     w.m = emc_mg_start_args(a, mg);
@@ -1618,13 +1663,18 @@ static int run_pcg_with(emc_ctx* c, const PA& a, const MA& mg, double rtol, int 
     w.maxit = maxit;
     w.nmem = emc_xcd_blocks(a.n, 1, g.ncu);
     w.xcd = g.xcd;
+    xcd_waits(g.form, w.meet, w.wait);
+    w.x0 = (typename PA::real*)g.x0;
     HIPCHECK(c, emc_launch_pcg_xcd(w, g.stream));
     HIPCHECK(c, hipMemcpyAsync(sh, a.scal, 8 * sizeof(double), hipMemcpyDeviceToHost, g.stream));
     g.pcg_result = sh;
-    g.pcg_pending = true;
+    g.pcg_pending = g.pcg_one = true;
     if (defer) return EMC_OK;
     HIPCHECK(c, hipStreamSynchronize(g.stream));
-    return finish_pcg(c, rtol, iters, relres);
+    const int redo = solve_redo(c, sh, a.x, a.n * sizeof(typename PA::real), g.stream);
+    if (redo < 0) return redo;
+    if (!redo) return finish_pcg(c, rtol, iters, relres);
+    g.pcg_pending = g.pcg_one = false;
   }
   // k_pcg_begin sets done when the start already meets the tolerance: the
   // queued iterations are then no-ops and the first check below stops the loop
@@ -2432,6 +2482,14 @@ int emc_poisson_solve_mixed(emc_ctx* c, const double* rhs, double* sol, double r
   return st;
 }
 
+int emc_poisson_form(emc_ctx* c, int form, int64_t* redone) {
+  if (!c || form > EMC_SOLVE_NO_WAIT) return EMC_ERR_ARG;
+  if (!c->gpu) return fail(c, EMC_ERR_NOGPU, "no GPU attached");
+  if (form >= 0) c->gpu->form = form;
+  if (redone) *redone = c->gpu->redone;
+  return EMC_OK;
+}
+
 int emc_poisson_mg_level(emc_ctx* c, int level, int dims[3], double* a27, double* omega) {
   if (!c || !dims) return EMC_ERR_ARG;
   const std::string e = ensure_mg(c);
@@ -2551,45 +2609,54 @@ static int one_step(emc_ctx* c, bool heat_phase, emc_fly_tallies* acc, double ts
   if (!heat_phase) da.rhs = RhsArgs{NN, g.node_q, g.pvol, g.pdop, g.dirichlet, g.corr, g.kind, g.rhs, nullptr};
   HIPCHECK(c, emc_launch_deposit(da, dep_items_most(g.ntile, g.n), g.stream));
   HIPCHECK(c, hipEventRecord(g.ev[1], g.stream));
-  if (!heat_phase) {
-    if (c->opts.poisson_fp32 == 1)
-      st = run_pcg_mixed(c, g.rhs, g.pot, c->opts.poisson_rtol, 20, c->opts.poisson_inner_rtol, nullptr, nullptr,
-                         nullptr);
-    else
-      st = run_pcg(c, g.rhs, g.pot, c->opts.poisson_rtol, c->opts.poisson_maxit, nullptr, nullptr, true);
-    if (st) return st;
-  }
-  HIPCHECK(c, hipEventRecord(g.ev[2], g.stream));
-  if (heat_phase) {
-    // heat_field (src/heat.cpp:100-103): holes at the window-mean Poisson
-    // potential, electrons at the window-mean corrected one
-    st = launch_fields(c, g.pot_avg, g.qc_avg ? g.qc_avg : g.pot_avg, true);
-  } else {
-    const double* pe = g.pot;
-    if (g.qc_pot) {
-      st = launch_qc(c, g.pot, g.qc_pot, count >= (uint64_t)std::max(0, cf.quantum_start_step));
-      if (st) return st;
-      pe = g.qc_pot;
-    }
-    st = launch_fields(c, g.pot, pe, true);
-  }
-  if (st) return st;
-  HIPCHECK(c, hipEventRecord(g.ev[3], g.stream));
-  st = zero_tallies(c);
-  if (st) return st;
   FlyArgs fa{};
-  // the transient flies without heat tallies: run() clears flag_heat (src/mcmodel.cpp:515)
-  st = launch_fly(c, step, heat_phase ? 1 : 0, fa);
-  if (st) return st;
-  HIPCHECK(c, hipEventRecord(g.ev[4], g.stream));
-  HIPCHECK(c, hipEventSynchronize(g.ev[4]));
-  // the one wait of the step: the solve's result, then the flight's counts
   int solved = EMC_OK;
-  if (!heat_phase) {
-    // was the gate shut?
-    const bool held = g.pcg_pending && xcd_solve(c) && !std::isfinite(g.pcg_result[0]);
+  // a second pass, kernel by kernel, where the one-launch solve has to be redone: its
+  // gate held everything behind it back
+  for (bool kernels = false;; kernels = true) {
+    if (!heat_phase) {
+      if (c->opts.poisson_fp32 == 1)
+        st = run_pcg_mixed(c, g.rhs, g.pot, c->opts.poisson_rtol, 20, c->opts.poisson_inner_rtol, nullptr, nullptr,
+                           nullptr);
+      else
+        st = run_pcg(c, g.rhs, g.pot, c->opts.poisson_rtol, c->opts.poisson_maxit, nullptr, nullptr, true, kernels);
+      if (st) return st;
+    }
+    HIPCHECK(c, hipEventRecord(g.ev[2], g.stream));
+    if (heat_phase) {
+      // heat_field (src/heat.cpp:100-103): holes at the window-mean Poisson
+      // potential, electrons at the window-mean corrected one
+      st = launch_fields(c, g.pot_avg, g.qc_avg ? g.qc_avg : g.pot_avg, true);
+    } else {
+      const double* pe = g.pot;
+      if (g.qc_pot) {
+        st = launch_qc(c, g.pot, g.qc_pot, count >= (uint64_t)std::max(0, cf.quantum_start_step));
+        if (st) return st;
+        pe = g.qc_pot;
+      }
+      st = launch_fields(c, g.pot, pe, true);
+    }
+    if (st) return st;
+    HIPCHECK(c, hipEventRecord(g.ev[3], g.stream));
+    st = zero_tallies(c);
+    if (st) return st;
+    // the transient flies without heat tallies: run() clears flag_heat (src/mcmodel.cpp:515)
+    st = launch_fly(c, step, heat_phase ? 1 : 0, fa);
+    if (st) return st;
+    HIPCHECK(c, hipEventRecord(g.ev[4], g.stream));
+    HIPCHECK(c, hipEventSynchronize(g.ev[4]));
+    // the one wait of the step: the solve's result, then the flight's counts
+    if (heat_phase) break;
+    const bool one = g.pcg_pending && g.pcg_one;
+    if (one) {
+      const int redo = solve_redo(c, g.pcg_result, g.pot, NN * sizeof(double), g.stream);
+      if (redo < 0) return redo;
+      if (redo) continue;
+    }
+    const bool held = one && !std::isfinite(g.pcg_result[0]);  // the gate was shut
     solved = finish_pcg(c, c->opts.poisson_rtol, nullptr, nullptr);
     if (solved && held) return solved;
+    break;
   }
   // flown, also behind a solve that missed its tolerance: the step is taken up first
   const int passes = finish_fly(c, fa);
@@ -2669,6 +2736,8 @@ struct emc_batch {
   size_t off_sort = 0, off_dep = 0, off_pcg = 0, off_mg = 0, off_fmg = 0, off_field = 0, off_fly = 0, off_cp = 0,
          off_xcd = 0, tab_bytes = 0;
   int nmem = 0;                        // blocks per device of the one-launch solve, 0: kernel by kernel
+  bool forced = false;                 // a context's form asks for the one launch
+  OneLaunch one;
   BatchTables bt{};
   const CopyArgs *cp_n = nullptr, *cp_scal = nullptr, *cp_tally = nullptr, *cp_zero = nullptr;
   unsigned long long* d_n = nullptr;   // [K] live counts after the sort, then the gate
@@ -2753,6 +2822,10 @@ static int batch_setup(emc_batch* b) {
   b->off_field = place(K * sizeof(FieldArgs));
   b->off_cp = place((5 * K + 1) * sizeof(CopyArgs));
   b->nmem = xcd_solve(c0) ? emc_xcd_blocks(b->nnode, K, g0.ncu) : 0;
+  for (emc_ctx* c : b->c) {
+    if (c->gpu->form == EMC_SOLVE_KERNELS) b->nmem = 0;
+    if (c->gpu->form > EMC_SOLVE_KERNELS) b->forced = true;
+  }
   b->off_xcd = place(!b->nmem ? 0 : K * (f32 ? sizeof(XcdArgsT<double, float>) : sizeof(XcdArgsT<double, double>)));
   b->tab_bytes = off;
   b->d_tab = b->mem.alloc<unsigned char>(off);
@@ -2819,6 +2892,8 @@ static int batch_setup(emc_batch* b) {
         t[q].nmem = b->nmem;
         t[q].xcd = q % 8;
         t[q].gate = b->gate;
+        xcd_waits(g.form, t[q].meet, t[q].wait);
+        t[q].x0 = g.x0;
       };
       if (f32) fill((XcdArgsT<double, float>*)(b->h_tab + b->off_xcd), hfm[q]);
       else fill((XcdArgsT<double, double>*)(b->h_tab + b->off_xcd), hm[q]);
@@ -2880,66 +2955,92 @@ static int batch_one_step(emc_batch* b, emc_fly_tallies* acc, double tsum[5], in
   BHIP(b, hipEventRecord(b->ev_n, s));
   BHIP(b, emc_launch_deposit_b(b->bt, b->ntile, nitem, b->nnode, s));
   BHIP(b, hipEventRecord(b->ev[1], s));
-  // the solve: as run_pcg, one iteration of every device per launch; the host
-  // checks the iteration before the one just queued, for all devices at once
-  int checked = -1, last = -1;
-  if (b->nmem) {
-    BHIP(b, emc_launch_pcg_xcd_b(b->bt, b->nmem, s));
-    BHIP(b, emc_launch_copy_b(b->cp_scal, K, 8, s));
-    BHIP(b, hipMemcpyAsync(b->h_scal, b->d_scal, 8 * K * sizeof(double), hipMemcpyDeviceToHost, s));
-    last = 0;
-  } else
-    BHIP(b, emc_launch_pcg_start_b(b->bt, b->shape, b->nblocks, s));
-  const int maxit = b->nmem ? 0 : b->c[0]->opts.poisson_maxit;
-  for (int k = 0; k < maxit; ++k) {
-    last = k;
-    BHIP(b, emc_launch_pcg_iter_b(b->bt, b->shape, b->nblocks, k, s));
-    BHIP(b, emc_launch_copy_b(b->cp_scal + (size_t)(k & 1) * K, K, 8, s));
-    BHIP(b, hipMemcpyAsync(b->h_scal + (size_t)(k & 1) * 8 * K, b->d_scal + (size_t)(k & 1) * 8 * K,
-                           8 * K * sizeof(double), hipMemcpyDeviceToHost, s));
-    BHIP(b, hipEventRecord(b->ev_scal[k & 1], s));
-    const int chk = (k + 1 == guess) ? k : k - 1;
-    if (chk < 0 || chk <= checked) continue;
-    BHIP(b, hipEventSynchronize(b->ev_scal[chk & 1]));
-    checked = chk;
-    bool all = true;
-    for (int q = 0; q < K; ++q) {
-      const double* res = b->h_scal + (size_t)(chk & 1) * 8 * K + 8 * q;
-      if (!std::isfinite(res[0])) return bfail(b, EMC_ERR_SOLVER, "PCG residual is not finite");
-      if (!(res[0] <= res[4])) all = false;
+  // a second pass, kernel by kernel, where a device's one-launch solve has to be
+  // redone: the gate held everything behind the solve back, for all devices
+  int last = -1;
+  const bool one_first = b->nmem && (b->forced || b->one.use());
+  bool one = one_first;
+  for (;; one = false) {
+    if (one != one_first) BHIP(b, emc_launch_copy_b(b->cp_n + K, 1, 1, s));  // the gate opens again
+    // the solve: as run_pcg, one iteration of every device per launch; the host
+    // checks the iteration before the one just queued, for all devices at once
+    int checked = -1;
+    last = -1;
+    if (one) {
+      BHIP(b, emc_launch_pcg_xcd_b(b->bt, b->nmem, s));
+      BHIP(b, emc_launch_copy_b(b->cp_scal, K, 8, s));
+      BHIP(b, hipMemcpyAsync(b->h_scal, b->d_scal, 8 * K * sizeof(double), hipMemcpyDeviceToHost, s));
+      last = 0;
+    } else
+      BHIP(b, emc_launch_pcg_start_b(b->bt, b->shape, b->nblocks, s));
+    const int maxit = one ? 0 : b->c[0]->opts.poisson_maxit;
+    for (int k = 0; k < maxit; ++k) {
+      last = k;
+      BHIP(b, emc_launch_pcg_iter_b(b->bt, b->shape, b->nblocks, k, s));
+      BHIP(b, emc_launch_copy_b(b->cp_scal + (size_t)(k & 1) * K, K, 8, s));
+      BHIP(b, hipMemcpyAsync(b->h_scal + (size_t)(k & 1) * 8 * K, b->d_scal + (size_t)(k & 1) * 8 * K,
+                             8 * K * sizeof(double), hipMemcpyDeviceToHost, s));
+      BHIP(b, hipEventRecord(b->ev_scal[k & 1], s));
+      const int chk = (k + 1 == guess) ? k : k - 1;
+      if (chk < 0 || chk <= checked) continue;
+      BHIP(b, hipEventSynchronize(b->ev_scal[chk & 1]));
+      checked = chk;
+      bool all = true;
+      for (int q = 0; q < K; ++q) {
+        const double* res = b->h_scal + (size_t)(chk & 1) * 8 * K + 8 * q;
+        if (!std::isfinite(res[0])) return bfail(b, EMC_ERR_SOLVER, "PCG residual is not finite");
+        if (!(res[0] <= res[4])) all = false;
+      }
+      if (all) break;
     }
-    if (all) break;
+    BHIP(b, hipEventRecord(b->ev[2], s));
+    BHIP(b, emc_launch_field_b(b->bt, b->ncell, s));
+    BHIP(b, hipEventRecord(b->ev[3], s));
+    BHIP(b, emc_launch_copy_b(b->cp_zero, K, FLYOUT_N, s));
+    // the flight needs the live counts of the sort (long since read: the residual
+    // checks waited on later work)
+    BHIP(b, hipEventSynchronize(b->ev_n));
+    nmax = 0;
+    for (int q = 0; q < K; ++q) {
+      emc_ctx* c = b->c[q];
+      Gpu& g = *c->gpu;
+      g.n = (long long)(unsigned)b->h_n[q];
+      g.sorted_n = g.n;
+      g.n_pending = false;
+      hfl[q] = fly_args(c, step[q], 0);
+      hfl[q].gate = b->nmem ? b->gate : nullptr;
+      nmax = std::max(nmax, g.n);
+    }
+    BHIP(b, hipMemcpyAsync(b->d_tab + b->off_fly, b->h_tab + b->off_fly, K * sizeof(FlyArgs), hipMemcpyHostToDevice, s));
+    BHIP(b, hipEventRecord(b->ev[5], s));
+    BHIP(b, emc_launch_fly_b(b->bt, nmax, b->c[0]->gpu->wave_slots, s));
+    BHIP(b, hipEventRecord(b->ev[6], s));
+    BHIP(b, emc_launch_copy_b(b->cp_tally, K, FLYOUT_N, s));
+    BHIP(b, hipMemcpyAsync(b->h_tally, b->d_tally, (size_t)K * FLYOUT_N * sizeof(unsigned long long),
+                           hipMemcpyDeviceToHost, s));
+    BHIP(b, hipEventRecord(b->ev[4], s));
+    BHIP(b, hipEventSynchronize(b->ev[4]));
+    if (!one) break;
+    bool again = false;
+    for (int q = 0; q < K; ++q)
+      if (b->h_scal[8 * q + XCD_STATUS] != XCD_SOLVED) {
+        ++b->c[q]->gpu->redone;
+        again = true;
+      }
+    if (!again) {
+      b->one.done();
+      break;
+    }
+    // every solve that began is set back to its start, so that the second pass is the
+    // one each device would take alone
+    b->one.failed();
+    for (int q = 0; q < K; ++q)
+      if (b->h_scal[8 * q + XCD_STATUS] != XCD_NOT_BEGUN)
+        BHIP(b, hipMemcpyAsync(b->c[q]->gpu->pot, b->c[q]->gpu->x0, b->nnode * sizeof(double), hipMemcpyDeviceToDevice, s));
   }
-  BHIP(b, hipEventRecord(b->ev[2], s));
-  BHIP(b, emc_launch_field_b(b->bt, b->ncell, s));
-  BHIP(b, hipEventRecord(b->ev[3], s));
-  BHIP(b, emc_launch_copy_b(b->cp_zero, K, FLYOUT_N, s));
-  // the flight needs the live counts of the sort (long since read: the residual
-  // checks waited on later work)
-  BHIP(b, hipEventSynchronize(b->ev_n));
-  nmax = 0;
-  for (int q = 0; q < K; ++q) {
-    emc_ctx* c = b->c[q];
-    Gpu& g = *c->gpu;
-    g.n = (long long)(unsigned)b->h_n[q];
-    g.sorted_n = g.n;
-    g.n_pending = false;
-    hfl[q] = fly_args(c, step[q], 0);
-    hfl[q].gate = b->nmem ? b->gate : nullptr;
-    nmax = std::max(nmax, g.n);
-  }
-  BHIP(b, hipMemcpyAsync(b->d_tab + b->off_fly, b->h_tab + b->off_fly, K * sizeof(FlyArgs), hipMemcpyHostToDevice, s));
-  BHIP(b, hipEventRecord(b->ev[5], s));
-  BHIP(b, emc_launch_fly_b(b->bt, nmax, b->c[0]->gpu->wave_slots, s));
-  BHIP(b, hipEventRecord(b->ev[6], s));
-  BHIP(b, emc_launch_copy_b(b->cp_tally, K, FLYOUT_N, s));
-  BHIP(b, hipMemcpyAsync(b->h_tally, b->d_tally, (size_t)K * FLYOUT_N * sizeof(unsigned long long),
-                         hipMemcpyDeviceToHost, s));
-  BHIP(b, hipEventRecord(b->ev[4], s));
-  BHIP(b, hipEventSynchronize(b->ev[4]));
   const double* scal = b->h_scal + (size_t)(last & 1) * 8 * K;
   // a residual that is none shut the gate: no device has taken its step
-  if (b->nmem)
+  if (one)
     for (int q = 0; q < K; ++q)
       if (!std::isfinite(scal[8 * q])) return bfail(b, EMC_ERR_SOLVER, "PCG residual is not finite");
   // per device: the solve's result, the flight's counts (finish_fly), the window.

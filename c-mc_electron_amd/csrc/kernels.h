@@ -229,10 +229,22 @@ struct MgArgsT {
 using MgArgs = MgArgsT<double>;
 
 // The words by which the blocks of the one-launch solve (k_pcg_xcd) find together;
-// zero before a launch and left zero by it.
+// zero before a launch and left zero by it.  arrive and leave count blocks in their
+// low half and those that came on another XCD, or left with a wait expired, in the
+// high one.
 struct XcdSync {
   unsigned arrive, state, xcc, bar, leave, pad[11];
 };
+
+// How a one-launch solve ended (scal[XCD_STATUS]): to its end; not begun, x untouched
+// (its blocks did not find together in time); or given up with x half iterated, x0 as
+// x was (a barrier's wait ran into its bound).  The host redoes the last two.
+constexpr int XCD_STATUS = 5;
+enum { XCD_SOLVED = 0, XCD_NOT_BEGUN = 1, XCD_GIVEN_UP = 2 };
+// Bounds of the waits, in ticks of the 100 MHz clock: 1 ms to find together, about
+// four solves (a team that waits for the CUs of another solve gets them within one),
+// and 20 ms at a barrier.
+constexpr long long XCD_MEET = 100000, XCD_WAIT = 2000000;
 
 template <class RA, class RM>
 struct XcdArgsT {
@@ -241,6 +253,10 @@ struct XcdArgsT {
   XcdSync* sync;
   int maxit, nmem;  // nmem: blocks per device
   int xcd, pad;     // the XCD they run on
+  // bounds of their waits (XCD_MEET, XCD_WAIT); to be given up on purpose: meet < 0 once
+  // all have come, wait < 0 at barrier -wait
+  long long meet, wait;
+  RA* x0;                // takes x as the solve finds it
   int* gate;        // shut when the solve fails, for all devices of a batch; null for one device (PcgArgsT::done)
 };
 

@@ -1896,14 +1896,15 @@ __global__ __launch_bounds__(TILE_THREADS) void k_mg_up(AS ms_, int l) {
 //
 // Which blocks: workgroups go to the XCDs in turn, so of XCD_COUNT * nmem blocks every
 // XCD_COUNT-th lands on one XCD.  Those are the candidates; the others leave at once.
-// The candidates check that they do share an XCD and wait until all have arrived;
-// if they do not (another placement, or the GPU held by other work for XCD_GATHER
-// ticks), the first candidate solves alone, which needs no one.  Once all are
-// resident each runs to its end, so the barriers' waits end; they are bounded all
-// the same (XCD_SPIN) and a bound reached fails the solve.
+// The candidates check that they do share an XCD and wait until all have arrived; if
+// they do not (another placement, or the CUs held by other work for XCD_MEET ticks: two
+// teams that each hold part of an XCD would wait for ever), none begins.  Once all are
+// resident each runs to its end, but the clock runs on while a queue is switched out
+// (other processes on the GPU), so the barriers' waits are bounded as well (XCD_WAIT);
+// a bound reached ends the solve.  Neither is an error: the start is kept in x0, and
+// the host redoes the solve kernel by kernel from it, with the same result to the bit.
 constexpr int XCD_COUNT = 8, XCD_THREADS = 512;
-constexpr long long XCD_GATHER = 2000000, XCD_SPIN = 20000000;  // 20 ms and 0.2 s of the 100 MHz clock
-enum { XCD_OPEN = 0, XCD_GO = 1, XCD_ALONE = 2 };
+enum { XCD_OPEN = 0, XCD_GO = 1, XCD_NONE = 2 };
 
 template <class T>
 __device__ __forceinline__ T ld_l2(const T* p) {
@@ -1924,6 +1925,7 @@ struct XcdTeam {
   unsigned epoch;
   double (*sh)[4];  // [4][4] block sums
   int* dead;        // shared: a wait ran into its bound
+  long long wait;   // that bound
   int flip;
 
   // every store of the team before it is seen by the team's reads after it
@@ -1934,10 +1936,11 @@ struct XcdTeam {
       if (threadIdx.x == 0 && !*dead) {
         const unsigned want = ++epoch * (unsigned)nmem;
         __hip_atomic_fetch_add(&s->bar, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (ld_l2(&s->bar) < want) {
+        if (wait < 0) *dead = (long long)epoch >= -wait;  // given up there on request
+        if (!*dead && ld_l2(&s->bar) < want) {
           const long long t0 = wall_clock64();
           while (ld_l2(&s->bar) < want)
-            if (wall_clock64() - t0 > XCD_SPIN) {
+            if (wall_clock64() - t0 > (wait < 0 ? XCD_WAIT : wait)) {
               *dead = 1;
               break;
             }
@@ -2047,7 +2050,7 @@ __global__ __launch_bounds__(XCD_THREADS) void k_pcg_xcd(AS as_) {
   const auto& m = w.m;
   using RA = typename std::decay_t<decltype(a)>::real;
   __shared__ double sh[4][4];
-  __shared__ int s_state, dead;
+  __shared__ int s_go, dead;
   const int nmem = w.nmem;
   const unsigned lane8 = (blockIdx.x + XCD_COUNT - (unsigned)w.xcd) % XCD_COUNT;
   if (lane8 != 0) return;
@@ -2058,25 +2061,32 @@ __global__ __launch_bounds__(XCD_THREADS) void k_pcg_xcd(AS as_) {
     // HW_REG_XCC_ID, bits 0-3
     const unsigned xcc = ((unsigned)__builtin_amdgcn_s_getreg((3 << 11) | 20) & 15u) + 1u;
     const unsigned old = atomicCAS(&s->xcc, 0u, xcc);
-    if (old != 0u && old != xcc) atomicCAS(&s->state, (unsigned)XCD_OPEN, (unsigned)XCD_ALONE);
-    if (atomicAdd(&s->arrive, 1u) + 1u == (unsigned)nmem)
-      atomicCAS(&s->state, (unsigned)XCD_OPEN, (unsigned)XCD_GO);
+    // the last to come decides; one word tells it of them all
+    const unsigned one = old != 0u && old != xcc ? 0x10001u : 1u;
+    const unsigned all = atomicAdd(&s->arrive, one) + one;
+    if ((all & 0xffffu) == (unsigned)nmem)
+      atomicCAS(&s->state, (unsigned)XCD_OPEN, (unsigned)((all >> 16) || w.meet < 0 ? XCD_NONE : XCD_GO));
     const long long t0 = wall_clock64();
     unsigned st;
     while ((st = ld_l2(&s->state)) == XCD_OPEN)
-      if (wall_clock64() - t0 > XCD_GATHER) atomicCAS(&s->state, (unsigned)XCD_OPEN, (unsigned)XCD_ALONE);
-    s_state = (int)st;
+      if (wall_clock64() - t0 > (w.meet < 0 ? XCD_MEET : w.meet)) atomicCAS(&s->state, (unsigned)XCD_OPEN, (unsigned)XCD_NONE);
+    s_go = st == XCD_GO;
   }
   __syncthreads();
-  const bool alone = s_state == XCD_ALONE;
-  if (!alone || me == 0) {
-    XcdTeam t{s, alone ? 1 : nmem, me, 0u, sh, &dead, 0};
-    const XcdLoop lp{(size_t)me * XCD_THREADS + threadIdx.x, (size_t)t.nmem * XCD_THREADS};
+  const bool go = s_go;
+  double rr = 0, bb = 0, rz = 0, tol = 0;
+  int it = 0;
+  if (go) {
+    XcdTeam t{s, nmem, me, 0u, sh, &dead, w.wait, 0};
+    const XcdLoop lp{(size_t)me * XCD_THREADS + threadIdx.x, (size_t)nmem * XCD_THREADS};
     const int nb = a.nblocks;
     const RA* ax = a.x;
-    // k_pcg_fix, k_pcg_resid
-    for (size_t n = lp.start(); n < a.n; n += lp.stride())
+    // k_pcg_fix, k_pcg_resid; x changes from its start (but for the fixed nodes) only
+    // behind later barriers, so x0 is whole whenever the solve is given up
+    for (size_t n = lp.start(); n < a.n; n += lp.stride()) {
+      w.x0[n] = a.x[n];
       if (a.kind[n] != 0) a.x[n] = a.b[n];
+    }
     t.barrier();
     {
       auto resid = [&](size_t n) -> double {
@@ -2096,11 +2106,10 @@ __global__ __launch_bounds__(XCD_THREADS) void k_pcg_xcd(AS as_) {
     t.barrier();
     xcd_cycle(t, m, lp, a.part_rz0, nb);
     // k_pcg_begin
-    double rr, bb, rz, rz_prev = 0, pq, unused;
+    double rz_prev = 0, pq, unused;
     t.totals(a.part_a, a.part_a + nb, 1, nb, rr, bb);
     t.totals(a.part_rz0, a.part_rz0, 1, nb, rz, unused);
-    const double tol = a.rtol * a.rtol * bb;
-    int it = 0;
+    tol = a.rtol * a.rtol * bb;
     for (; !(rr <= tol) && it < w.maxit && !dead && isfinite(rr); ++it) {
       double* rz_out = (it & 1) ? a.part_rz0 : a.part_rz1;
       RA* p_out = (it & 1) ? a.p2 : a.p;
@@ -2132,18 +2141,23 @@ __global__ __launch_bounds__(XCD_THREADS) void k_pcg_xcd(AS as_) {
       rz_prev = rz;
       t.totals(rz_out, rz_out, 1, nb, rz, unused);
     }
-    if (me == 0 && threadIdx.x == 0) {
+  }
+  // The last candidate to leave says how it went, for the gate and the host alike (all
+  // that ran to the end hold the same scalars), and leaves the words as the next
+  // launch needs them.
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const unsigned one = dead ? 0x10001u : 1u;
+    const unsigned all = atomicAdd(&s->leave, one) + one;
+    if ((all & 0xffffu) == (unsigned)nmem) {
+      const int status = !go ? XCD_NOT_BEGUN : (all >> 16) ? XCD_GIVEN_UP : XCD_SOLVED;
       a.scal[0] = rr; a.scal[1] = rz; a.scal[2] = bb; a.scal[3] = it; a.scal[4] = tol;
-      const bool bad = dead || !isfinite(rr);
+      a.scal[XCD_STATUS] = status;
+      const bool bad = status != XCD_SOLVED || !isfinite(rr);
       *a.done = bad ? GATE_SHUT : 1;
       if (bad && w.gate) *w.gate = GATE_SHUT;
+      s->arrive = 0; s->state = XCD_OPEN; s->xcc = 0; s->bar = 0; s->leave = 0;
     }
-    if (dead && threadIdx.x == 0) a.scal[0] = __builtin_nan("");
-  }
-  // the last candidate leaves the words as the next launch needs them
-  __syncthreads();
-  if (threadIdx.x == 0 && atomicAdd(&s->leave, 1u) + 1u == (unsigned)nmem) {
-    s->arrive = 0; s->state = XCD_OPEN; s->xcc = 0; s->bar = 0; s->leave = 0;
   }
 }
 

@@ -260,6 +260,13 @@ class Engine:
                                                      maxit_outer, inner_rtol, C.byref(o), C.byref(i), C.byref(rr)))
         return sol, o.value, i.value, rr.value
 
+    def poisson_form(self, form=-1):
+        """Sets how the solves are launched (abi.SOLVE_*; -1 leaves it) and returns the
+        number of solves redone kernel by kernel so far."""
+        n = C.c_int64(0)
+        self._check(self.lib.emc_poisson_form(self.ctx, form, C.byref(n)))
+        return n.value
+
     def poisson_solve_noalloc(self, rhs, x0=None, rtol=1e-10, maxit=20000):
         """poisson_solve through emc_poisson_solve_noalloc (work vectors in the
         library's static device array; nothing allocated per call)."""

@@ -132,6 +132,8 @@ class Opts(C.Structure):
     ]
 
 
+SOLVE_AUTO, SOLVE_KERNELS, SOLVE_NO_MEET, SOLVE_NO_WAIT = 0, 1, 2, 3
+
 REQ_QUEUED, REQ_RUNNING, REQ_DONE, REQ_FAILED = 0, 1, 2, 3
 REQ_MAX_WINDOWS = 64
 
@@ -186,6 +188,7 @@ def declare(lib):
         "emc_poisson_solve": (C.c_int, [ctx, _d, _d, C.c_double, C.c_int, _i, _d]),
         "emc_poisson_solve_noalloc": (C.c_int, [ctx, _d, _d, C.c_double, C.c_int, _i, _d]),
         "emc_poisson_solve_mixed": (C.c_int, [ctx, _d, _d, C.c_double, C.c_int, C.c_double, _i, _i, _d]),
+        "emc_poisson_form": (C.c_int, [ctx, C.c_int, _i64]),
         "emc_poisson_mg_level": (C.c_int, [ctx, C.c_int, _i, _d, _d]),
         "emc_compute_field": (C.c_int, [ctx, _d, _d]),
         "emc_step": (C.c_int, [ctx, C.c_int, P(FlyTallies)]),

@@ -331,6 +331,24 @@ int emc_poisson_solve_noalloc(emc_ctx *ctx, const double *rhs, double *sol, doub
 int emc_poisson_solve_mixed(emc_ctx *ctx, const double *rhs, double *sol, double rtol, int maxit_outer,
                             double inner_rtol, int *outer, int *inner, double *relres);
 
+/* How the context's solves are launched; no counterpart in the reference.  Meshes of up
+ * to 32768 nodes are solved in one launch, in which the blocks on one part of the GPU
+ * (an XCD) walk the solve together.  Where other work keeps them from finding together
+ * or from one another for too long, the solve is redone kernel by kernel, as on larger
+ * meshes, and so are the next few (8, doubled up to 1024 while it happens again).
+ * Every form gives the same potential, iterations and residual bit for bit.
+ *   EMC_SOLVE_AUTO      the default
+ *   EMC_SOLVE_KERNELS   kernel by kernel on every mesh
+ *   EMC_SOLVE_NO_MEET, EMC_SOLVE_NO_WAIT   one launch whose blocks give up on finding
+ *                       together, or on waiting in the second iteration (to test the redo)
+ * A negative form leaves it as it is.  redone (may be NULL): solves redone since
+ * emc_create.  A batch takes the forms its contexts have when it is created. */
+#define EMC_SOLVE_AUTO 0
+#define EMC_SOLVE_KERNELS 1
+#define EMC_SOLVE_NO_MEET 2
+#define EMC_SOLVE_NO_WAIT 3
+int emc_poisson_form(emc_ctx *ctx, int form, int64_t *redone);
+
 /* Level `level` of the multigrid hierarchy used by emc_poisson_solve (no reference
  * counterpart: the reference factorises with KLU).  dims[3] = nodes along i, j, k;
  * a27 (may be NULL; levels >= 1) receives the [27][n] Galerkin coefficients, entry
