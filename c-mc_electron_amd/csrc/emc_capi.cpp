@@ -29,6 +29,39 @@
 
 using namespace emc;
 
+// The solves of small meshes under way on a GPU, over every context and batch of the
+// process, in blocks of their one-launch form.  A block takes a CU, and teams that need
+// more CUs than there are wait for one another, so a solve that finds others under way
+// goes kernel by kernel when all together would take more than 5/4 of the CUs.  Batches
+// of 20x35x11-cell devices stepped side by side, us a step of all of them, in one launch
+// and kernel by kernel: four of 4 devices (288 blocks) 710 and 860, four of 9 (576) 1385
+// and 1040, four of 16 (1024) 1700 and 1460.
+class XcdTurn {
+  static std::atomic<int>& load(int device) {
+    static std::atomic<int> n[16];
+    return n[device & 15];
+  }
+  int device = 0, held = 0;
+
+ public:
+  XcdTurn() = default;
+  XcdTurn(const XcdTurn&) = delete;
+  XcdTurn& operator=(const XcdTurn&) = delete;
+  ~XcdTurn() { give(); }
+  // whether the solve may go in one launch; it is under way until give() in any form
+  bool take(int dev, int blocks, int ncu) {
+    give();
+    device = dev;
+    held = blocks;
+    const int others = load(dev).fetch_add(blocks);
+    return others == 0 || others + blocks <= ncu + ncu / 4;
+  }
+  void give() {
+    if (held) load(device).fetch_sub(held);
+    held = 0;
+  }
+};
+
 // When a one-launch solve could not be finished (XCD_STATUS), the next ones go kernel by
 // kernel, twice as many each time in a row: what holds the XCD up, another solver's
 // blocks or another process, is likely still there, and a try costs up to its wait.
@@ -162,9 +195,10 @@ struct Gpu {
   double *part_a = nullptr, *part_pq = nullptr, *part_rr = nullptr, *part_rz0 = nullptr, *part_rz1 = nullptr;
   int* done = nullptr;
   XcdSync* sync = nullptr;            // the one-launch solve's words (zero between launches)
-  int xcd = 0, ncu = 0;               // the XCD this context's solves run on; CUs of the GPU
+  int ncu = 0;                        // CUs of the GPU
   int form = EMC_SOLVE_AUTO;          // emc_poisson_form
   OneLaunch one;
+  XcdTurn turn;                       // of the pending solve
   double* x0 = nullptr;               // the start of a one-launch solve, for its redo
   bool pcg_one = false;               // the pending solve went in one launch
   int64_t redone = 0;                 // solves redone kernel by kernel
@@ -542,9 +576,6 @@ static int gpu_setup(emc_ctx* c) {
     if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, g.device) == hipSuccess && ncu > 0)
       g.wave_slots = 4LL * ncu;
     g.ncu = ncu;
-    // contexts that run side by side solve on different XCDs
-    static std::atomic<unsigned> contexts{0};
-    g.xcd = (int)(contexts++ % 8);
   }
   for (auto& e : g.ev) HIPCHECK(c, hipEventCreate(&e));
   const Device& d = c->dev;
@@ -1626,6 +1657,14 @@ static int run_pcg(emc_ctx* c, const double* b, double* x, double rtol, int maxi
   return run_pcg_with(c, pcg_args(c, b, x, rtol), g.mg, rtol, maxit, iters, relres, defer, kernels);
 }
 
+// The XCDs that the devices of one launch solve on, counted from the one its queue
+// begins its launches at.  That is another one for each hardware queue (four in a row
+// for the four queues of a process), so solves queued side by side are apart by
+// themselves; two devices of a batch go four XCDs apart, and so on, to leave the next
+// queues theirs.  (Counted up from there: four batches of 4 20x35x11-cell devices 1230 us
+// a step of all of them, in this order 710; kernel by kernel 860.)
+static const int XCD_ORDER[8] = {0, 4, 2, 6, 1, 5, 3, 7};
+
 // The bounds of the one-launch solve's waits in the context's form.
 static void xcd_waits(int form, long long& meet, long long& wait) {
   meet = form == EMC_SOLVE_NO_MEET ? -1 : XCD_MEET;
@@ -1653,16 +1692,19 @@ template <class PA, class MA>
 static int run_pcg_with(emc_ctx* c, const PA& a, const MA& mg, double rtol, int maxit, int* iters, double* relres,
                         bool defer, bool kernels) {
   Gpu& g = *c->gpu;
+  struct Turn { XcdTurn* t; ~Turn() { if (t) t->give(); } } turn{defer ? nullptr : &g.turn};
   double* sh = g.scal_host;
   g.pcg_one = false;
-  if (!kernels && xcd_solve(c) && g.form != EMC_SOLVE_KERNELS && (g.form != EMC_SOLVE_AUTO || g.one.use())) {
+  const int nmem = xcd_solve(c) ? emc_xcd_blocks(a.n, 1, g.ncu) : 0;
+  if (!kernels && nmem && g.form != EMC_SOLVE_KERNELS &&
+      (g.form != EMC_SOLVE_AUTO || (g.turn.take(g.device, nmem, g.ncu) && g.one.use()))) {
     XcdArgsT<typename PA::real, typename MA::real> w{};
     w.a = a;
     w.m = emc_mg_start_args(a, mg);
     w.sync = g.sync;
     w.maxit = maxit;
-    w.nmem = emc_xcd_blocks(a.n, 1, g.ncu);
-    w.xcd = g.xcd;
+    w.nmem = nmem;
+    w.xcd = XCD_ORDER[0];
     xcd_waits(g.form, w.meet, w.wait);
     w.x0 = (typename PA::real*)g.x0;
     HIPCHECK(c, emc_launch_pcg_xcd(w, g.stream));
@@ -1718,6 +1760,7 @@ static double rel_residual(const double* scal) {
 
 static int finish_pcg(emc_ctx* c, double rtol, int* iters, double* relres) {
   Gpu& g = *c->gpu;
+  g.turn.give();
   if (!g.pcg_pending) return EMC_OK;
   g.pcg_pending = false;
   const double* sh = g.pcg_result;
@@ -2598,7 +2641,7 @@ static int one_step(emc_ctx* c, bool heat_phase, emc_fly_tallies* acc, double ts
   const uint64_t count = heat_phase ? c->heat_next++ : c->next_step++;
   const uint64_t step = heat_phase ? HEAT_STEP0 + count : count;
   // no later call's kernels are gated by a solve of this step
-  struct Pending { bool& p; ~Pending() { p = false; } } pending{g.pcg_pending};
+  struct Pending { Gpu& g; ~Pending() { g.pcg_pending = false; g.turn.give(); } } pending{g};
   HIPCHECK(c, hipEventRecord(g.ev[0], g.stream));
   int st = run_sort(c);
   if (st) return st;
@@ -2890,7 +2933,7 @@ static int batch_setup(emc_batch* b) {
         t[q].sync = g.sync;
         t[q].maxit = c->opts.poisson_maxit;
         t[q].nmem = b->nmem;
-        t[q].xcd = q % 8;
+        t[q].xcd = XCD_ORDER[q % 8];
         t[q].gate = b->gate;
         xcd_waits(g.form, t[q].meet, t[q].wait);
         t[q].x0 = g.x0;
@@ -2958,7 +3001,9 @@ static int batch_one_step(emc_batch* b, emc_fly_tallies* acc, double tsum[5], in
   // a second pass, kernel by kernel, where a device's one-launch solve has to be
   // redone: the gate held everything behind the solve back, for all devices
   int last = -1;
-  const bool one_first = b->nmem && (b->forced || b->one.use());
+  XcdTurn turn;
+  const bool one_first =
+      b->nmem && (b->forced || (turn.take(b->device, K * b->nmem, b->c[0]->gpu->ncu) && b->one.use()));
   bool one = one_first;
   for (;; one = false) {
     if (one != one_first) BHIP(b, emc_launch_copy_b(b->cp_n + K, 1, 1, s));  // the gate opens again

@@ -252,7 +252,7 @@ struct XcdArgsT {
   MgArgsT<RM> m;  // m.z: the cycle's output
   XcdSync* sync;
   int maxit, nmem;  // nmem: blocks per device
-  int xcd, pad;     // the XCD they run on
+  int xcd, pad;     // the XCD they run on, counted from the one the queue begins at
   // bounds of their waits (XCD_MEET, XCD_WAIT); to be given up on purpose: meet < 0 once
   // all have come, wait < 0 at barrier -wait
   long long meet, wait;
