@@ -749,6 +749,27 @@ static void release_part(DevBuf& m, PartDev& P) {
   P = PartDev{};
 }
 
+// The deposit's work items for the slots of the population.  Allocated with the slots,
+// not by the first step, and grown with them (in use on the device only between a sort
+// and its deposit).
+static int ensure_items(emc_ctx* c) {
+  Gpu& g = *c->gpu;
+  const long long cap = dep_items_most(g.ntile, std::max(g.cap, g.n));
+  if (cap <= g.item_cap) return EMC_OK;
+  HIPCHECK(c, hipStreamSynchronize(g.stream));
+  DevBuf& m = g.mem;
+  m.release(g.itile);
+  m.release(g.xtile);
+  m.release(g.blk);
+  g.item_cap = 0;
+  g.itile = m.alloc<unsigned>(cap);
+  g.xtile = m.alloc<unsigned>(cap);
+  g.blk = m.alloc<unsigned long long>((size_t)cap * DEP_SLOT);
+  if (m.last != hipSuccess) return fail(c, EMC_ERR_HIP, std::string("deposit blocks: ") + hipGetErrorString(m.last));
+  g.item_cap = cap;
+  return EMC_OK;
+}
+
 static int gpu_alloc_particles(emc_ctx* c, long long cap) {
   Gpu& g = *c->gpu;
   if (g.cap >= cap) return EMC_OK;
@@ -776,7 +797,7 @@ static int gpu_alloc_particles(emc_ctx* c, long long cap) {
   g.dead = m.alloc<long long>(g.dead_cap);
   g.slow = m.alloc<uint32_t>(cap);
   if (m.last != hipSuccess) return fail(c, EMC_ERR_HIP, std::string("particle allocation: ") + hipGetErrorString(m.last));
-  return EMC_OK;
+  return ensure_items(c);
 }
 
 // Keeps room for a step's clones: once the population comes within one clone
@@ -817,7 +838,7 @@ static int grow_if_full(emc_ctx* c) {
   g.clones = clones; g.clone_cap = clone_cap;
   g.dead = dead; g.dead_cap = clone_cap;
   g.slow = slow;
-  return EMC_OK;
+  return ensure_items(c);
 }
 
 // MultipleRefresh target counts per cell (src/particle_init.cpp:44-70): the
@@ -1545,27 +1566,6 @@ static long long sort_nappend(emc_ctx* c) {
   return seg_usable(g) ? std::max(0LL, g.n - g.sorted_n) : g.n;
 }
 
-// The deposit's work items for the slots of the population: their blocks grow with
-// it (in use on the device only between a sort and its deposit).
-static int ensure_items(emc_ctx* c) {
-  Gpu& g = *c->gpu;
-  const long long need = dep_items_most(g.ntile, g.n);
-  if (need <= g.item_cap) return EMC_OK;
-  const long long cap = dep_items_most(g.ntile, std::max(g.cap, g.n));
-  HIPCHECK(c, hipStreamSynchronize(g.stream));
-  DevBuf& m = g.mem;
-  m.release(g.itile);
-  m.release(g.xtile);
-  m.release(g.blk);
-  g.item_cap = 0;
-  g.itile = m.alloc<unsigned>(cap);
-  g.xtile = m.alloc<unsigned>(cap);
-  g.blk = m.alloc<unsigned long long>((size_t)cap * DEP_SLOT);
-  if (m.last != hipSuccess) return fail(c, EMC_ERR_HIP, std::string("deposit blocks: ") + hipGetErrorString(m.last));
-  g.item_cap = cap;
-  return EMC_OK;
-}
-
 static int run_sort(emc_ctx* c) {
   Gpu& g = *c->gpu;
   int st = settle_n(c);
@@ -1950,7 +1950,7 @@ static int run_mr(emc_ctx* c, uint64_t step, long long* before, long long* after
     g.seg_valid = false;
     if (before) *before = (long long)h[0];
     if (after) *after = total;
-    return EMC_OK;
+    return ensure_items(c);
   }
   HIPCHECK(c, emc_launch_mr_write(a, g.stream));
   std::swap(g.P, g.P2);
@@ -2968,16 +2968,17 @@ static int batch_one_step(emc_batch* b, emc_fly_tallies* acc, double tsum[5], in
   FlyArgs* hfl = (FlyArgs*)(b->h_tab + b->off_fly);
   long long nmax = 0, nitem = 0;
   int guess = 0;
+  // what can fail comes before any device's buffers are swapped
+  for (emc_ctx* c : b->c) {
+    int st = settle_n(c);
+    if (!st) st = grow_if_full(c);
+    if (!st) st = ensure_items(c);
+    if (st) return bfail(b, st, c->err);
+  }
   for (int q = 0; q < K; ++q) {
     emc_ctx* c = b->c[q];
     Gpu& g = *c->gpu;
     step[q] = c->next_step++;
-    int st = settle_n(c);
-    if (st) return bfail(b, st, c->err);
-    st = grow_if_full(c);
-    if (st) return bfail(b, st, c->err);
-    st = ensure_items(c);
-    if (st) return bfail(b, st, c->err);
     nitem = std::max(nitem, dep_items_most(b->ntile, g.n));
     hs[q] = sort_args(c);
     nmax = std::max(nmax, sort_nappend(c));

@@ -112,13 +112,14 @@ namespace {
 
 // Device bytes a request will hold, from its deck: per node the tallies, window
 // sums, potential, solver and multigrid vectors; per cell the fields, rates, cell
-// sums and deposit tile blocks; per particle slot the two particle buffers and the
-// flight's work lists; the dense inverse of the coarsest multigrid level.
+// sums and the deposit's block of each tile (24 KB for 128 cells); per particle slot the
+// two particle buffers, the flight's work lists and the dense tiles' further blocks
+// (24 KB for 768 slots); the dense inverse of the coarsest multigrid level.
 double estimate_bytes(const emc_mesh_view& m, const std::string& deck, double capacity_factor) {
   const double ne = deck_number(deck, "ElectronNumber", 0), nh = deck_number(deck, "HoleNumber", 0);
   const double slots = (ne + nh + 2.0 * (double)m.ncell) * std::max(1.0, capacity_factor) + 1024;
   const double nc = std::max(600.0, std::min(2500.0, (double)m.nnode / 300));
-  return 320.0 * (double)m.nnode + 360.0 * (double)m.ncell + 222.0 * slots + 8.0 * nc * nc + (8 << 20);
+  return 320.0 * (double)m.nnode + 400.0 * (double)m.ncell + 222.0 * slots + 8.0 * nc * nc + (8 << 20);
 }
 
 void finish_window(Req* r) {
