@@ -342,15 +342,17 @@ hipError_t emc_launch_pcg_iter(const emc::PcgArgsT<float>& a, const emc::MgArgsT
 hipError_t emc_launch_refine_resid(const emc::RefineArgs& r, hipStream_t s);
 hipError_t emc_launch_refine_add(const emc::RefineArgs& r, hipStream_t s);
 hipError_t emc_launch_zero_f32(float* p, size_t n, hipStream_t s);
-// The whole solve in one launch; blocks per device for K devices on a GPU of ncu CUs.
+// The whole solve in one launch; blocks per device for K devices on a GPU of ncu CUs, 0
+// where they are better solved kernel by kernel.
 // Up to XCD_MAX_NODES the solve is bound by its launches and goes in one (us per solve
-// kernel by kernel and in one launch, 6 to 7 iterations: 9.1 k nodes 385 and 250,
-// 11.2 k 368 and 270, 18.8 k 387 and 313; above, 32 CUs are too few: 69 k 489 and 574,
-// 96 k 576 and 715).  Eight devices of 11.2 k nodes in a batch: 413 and 312.
+// kernel by kernel and in one launch, 6 to 7 iterations: 9.1 k nodes 408 and 263,
+// 11.2 k 420 and 266, 18.8 k 442 and 394, 23.9 k 429 and 372, 32.5 k 532 and 538; above,
+// 32 CUs are too few: 69 k 489 and 574, 96 k 576 and 715).  Eight devices in a batch:
+// 11.2 k nodes 454 and 317, 32.5 k 655 and 556.
 namespace emc {
 constexpr size_t XCD_MAX_NODES = 32768;
 }
-int emc_xcd_blocks(size_t n, int K, int ncu);
+extern "C" int emc_xcd_blocks(size_t n, int K, int ncu);
 hipError_t emc_launch_pcg_xcd(const emc::XcdArgsT<double, double>& a, hipStream_t s);
 hipError_t emc_launch_pcg_xcd(const emc::XcdArgsT<double, float>& a, hipStream_t s);
 hipError_t emc_launch_pcg_xcd(const emc::XcdArgsT<float, float>& a, hipStream_t s);

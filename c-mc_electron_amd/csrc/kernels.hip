@@ -2450,13 +2450,19 @@ hipError_t emc_launch_pcg_iter(const PcgArgs& a, const MgArgsT<float>& m, int it
 }
 
 // ---- the solve in one launch
-// One block per node thread, shared CUs divided among the devices of an XCD (us a
+// A thread per node, the CUs of an XCD divided among the devices that share it (us a
 // solve, 11.2 k nodes: 8 blocks 368, 16 317, 24 270, 32 285; 16 devices: 16 blocks
-// each 377, 32 614, 8 427).
-int emc_xcd_blocks(size_t n, int K, int ncu) {
-  const int cus = ncu / XCD_COUNT > 1 ? ncu / XCD_COUNT : 1;   // of one XCD
-  const int per = (K + XCD_COUNT - 1) / XCD_COUNT;              // devices that share it
-  const int most = cus / per > 4 ? cus / per : cus < 4 ? cus : 4;
+// each 377, 32 614, 8 427).  A team has a multiple of the XCD's four shader engines:
+// blocks go to the engines in turn, and teams of 10 put a ninth block on one of eight
+// CUs, so that the third team waits for the others (17 devices of 9.1 k nodes 703 us, in
+// teams of 8 469, kernel by kernel 491).
+// 0, kernel by kernel, above 36 k nodes an XCD: 16 devices of 13.5 k nodes 512 us in one
+// launch and 556 kernel by kernel, 9 of 18.8 k 595 and 515; 32 of 9.1 k 522 and 582,
+// of 13.5 k 751 and 724; 64 of 9.1 k 790 and 811, of 11.2 k 931 and 913.
+extern "C" int emc_xcd_blocks(size_t n, int K, int ncu) {
+  const int per = (K + XCD_COUNT - 1) / XCD_COUNT;   // devices that share an XCD
+  if (n * (size_t)per > XCD_MAX_NODES * 9 / 8) return 0;
+  const int most = ncu / XCD_COUNT / per / 4 * 4;
   const size_t want = (n + XCD_THREADS - 1) / XCD_THREADS;      // a node a thread
   return want < (size_t)most ? (int)want : most;
 }
