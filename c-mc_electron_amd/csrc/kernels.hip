@@ -13,6 +13,7 @@
 //   k_pcg_*      CG on the 7-point operator, preconditioned by
 //   k_mg_*       one multigrid cycle: V(2,2) on the finest level, V(1,1) below
 //                (damped Jacobi, Galerkin coarse levels, dense coarsest solve)
+//   k_pcg_xcd    the whole solve of a small mesh in one launch
 //
 // All HBM-bound integer/FP64 work: no MFMA.  Compiled with -ffp-contract=off so
 // the FP64 results match the CPU restatement bit for bit.
@@ -1394,9 +1395,10 @@ __global__ __launch_bounds__(256) void k_pcg_update(AS as_, int it) {
 }
 
 // ------------------------------------------------------------------ multigrid V-cycle
-// The phases of the cycle are written once per node (grid-stride loops, one
-// launch per phase).  A single workgroup walking the small levels was measured
-// slower (latency bound) than one launch per phase.
+// The phases of the cycle, once per node (grid-stride loops).  On the mesh level each is
+// a launch of its own; the levels below it go down in one launch and up in one
+// (k_mg_down, k_mg_up); small meshes walk all phases in one launch (k_pcg_xcd).  A single
+// workgroup walking the small levels was measured slower (latency bound).
 
 template <class LV>
 __device__ inline void lvl_ijk(const LV& L, size_t n, int& i, int& j, int& k) {
@@ -2371,15 +2373,15 @@ static void launch_vcycle(const SHAPE& m, AS ms, int nblocks, unsigned K, hipStr
   hipLaunchKernelGGL(k_mg_sweep_last<AS>, dim3(nblocks, K), dim3(256), 0, s, ms);
 }
 
-// the cycle's argument block of the solve's start (r.z partials into part_rz0,
-// no residual booking) and of CG iteration `it` (r.z into the partial array the
-// next iteration reads as rz_new; the first kernel books the residual)
 // the cycle's output: the CG's z, or z32 for the FP32 cycle of the FP64 CG
 template <class RM, class RA>
 static RM* cycle_out(const PcgArgsT<RA>& a) {
   if constexpr (std::is_same<RA, RM>::value) return a.z;
   else return const_cast<float*>(a.z32);
 }
+// the cycle's argument block of the solve's start (r.z partials into part_rz0,
+// no residual booking) and of CG iteration `it` (r.z into the partial array the
+// next iteration reads as rz_new; the first kernel books the residual)
 template <class RA, class RM>
 static MgArgsT<RM> mg_start_args(const PcgArgsT<RA>& a, const MgArgsT<RM>& m) {
   MgArgsT<RM> m0 = m;

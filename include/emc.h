@@ -333,10 +333,11 @@ int emc_poisson_solve_mixed(emc_ctx *ctx, const double *rhs, double *sol, double
 
 /* How the context's solves are launched; no counterpart in the reference.  Meshes of up
  * to 32768 nodes are solved in one launch, in which the blocks on one part of the GPU
- * (an XCD) walk the solve together.  Where other work keeps them from finding together
- * or from one another for too long, the solve is redone kernel by kernel, as on larger
- * meshes, and so are the next few (8, doubled up to 1024 while it happens again).
- * Every form gives the same potential, iterations and residual bit for bit.
+ * (an XCD) walk the solve together, or kernel by kernel, as on larger meshes, where more
+ * of them are under way than fit.  Where other work keeps the blocks from finding
+ * together, or from one another for too long, the solve is redone kernel by kernel, and
+ * the next few go that way (8, doubled up to 1024 while it happens again).  Every form
+ * gives the same potential, iterations and residual bit for bit.
  *   EMC_SOLVE_AUTO      the default
  *   EMC_SOLVE_KERNELS   kernel by kernel on every mesh
  *   EMC_SOLVE_NO_MEET, EMC_SOLVE_NO_WAIT   one launch whose blocks give up on finding
