@@ -13,7 +13,7 @@
 //    which redoes it from its stored state with the same random numbers.
 //  * Of the seven faces (four of the tetrahedron, three of the cell) only the
 //    nearest one's time is divided out.  Quotients from the hardware reciprocal
-//    (relative error below 1e-7) find it; a particle with two of them within 1e-6
+//    (relative error up to 2^-23, 1.2e-7) find it; a particle with two of them within 1e-6
 //    of each other, or of the end of the step, goes to the slow kernel.
 //
 // What bounds it: the vector-memory return path (texture data unit busy 96 % of the

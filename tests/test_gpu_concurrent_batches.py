@@ -59,8 +59,8 @@ def test_side_by_side_equals_alone(batches, devices):
                 assert p.n == o.n
                 for k in ("x", "y", "z", "kx", "ky", "kz", "itet", "key"):
                     np.testing.assert_array_equal(getattr(p, k)[:p.n], getattr(o, k)[:p.n], err_msg=f"{g} {q} {k}")
-                # tried at steps 0, 9 and 26 when every try fails
-                assert e.poisson_form() <= 3
+                # at most every tenth solve (eight held off, one that works, the next redone)
+                assert e.poisson_form() <= STEPS // 10
     finally:
         for e in sum(side + alone, []):
             e.close()
