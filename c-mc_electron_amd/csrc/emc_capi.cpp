@@ -1738,7 +1738,10 @@ static int run_pcg_with(emc_ctx* c, const PA& a, const MA& mg, double rtol, int 
     HIPCHECK(c, hipEventSynchronize(g.scal_ready[chk & 1]));
     checked = chk;
     const double* res = sh + 8 * (chk & 1);
-    if (!std::isfinite(res[0])) return fail(c, EMC_ERR_SOLVER, "PCG residual is not finite");
+    if (!std::isfinite(res[0])) {
+      HIPCHECK(c, hipStreamSynchronize(g.stream));  // the iterations queued behind it still write
+      return fail(c, EMC_ERR_SOLVER, "PCG residual is not finite");
+    }
     if (res[0] <= res[4]) break;
   }
   // the kernels queued after convergence leave scal as it was, so the copy of the
@@ -2999,6 +3002,18 @@ static int batch_one_step(emc_batch* b, emc_fly_tallies* acc, double tsum[5], in
   BHIP(b, hipEventRecord(b->ev_n, s));
   BHIP(b, emc_launch_deposit_b(b->bt, b->ntile, nitem, b->nnode, s));
   BHIP(b, hipEventRecord(b->ev[1], s));
+  // The live counts of the sort, which the flight needs and which a step that fails in
+  // its solve leaves behind (long since read: the residual checks waited on later work).
+  auto take_counts = [&]() -> int {
+    BHIP(b, hipEventSynchronize(b->ev_n));
+    for (int q = 0; q < K; ++q) {
+      Gpu& g = *b->c[q]->gpu;
+      g.n = (long long)(unsigned)b->h_n[q];
+      g.sorted_n = g.n;
+      g.n_pending = false;
+    }
+    return EMC_OK;
+  };
   // a second pass, kernel by kernel, where a device's one-launch solve has to be
   // redone: the gate held everything behind the solve back, for all devices
   int last = -1;
@@ -3034,7 +3049,11 @@ static int batch_one_step(emc_batch* b, emc_fly_tallies* acc, double tsum[5], in
       bool all = true;
       for (int q = 0; q < K; ++q) {
         const double* res = b->h_scal + (size_t)(chk & 1) * 8 * K + 8 * q;
-        if (!std::isfinite(res[0])) return bfail(b, EMC_ERR_SOLVER, "PCG residual is not finite");
+        if (!std::isfinite(res[0])) {
+          BHIP(b, hipStreamSynchronize(s));  // the iterations queued behind it still write
+          const int st = take_counts();
+          return st ? st : bfail(b, EMC_ERR_SOLVER, "PCG residual is not finite");
+        }
         if (!(res[0] <= res[4])) all = false;
       }
       if (all) break;
@@ -3043,19 +3062,13 @@ static int batch_one_step(emc_batch* b, emc_fly_tallies* acc, double tsum[5], in
     BHIP(b, emc_launch_field_b(b->bt, b->ncell, s));
     BHIP(b, hipEventRecord(b->ev[3], s));
     BHIP(b, emc_launch_copy_b(b->cp_zero, K, FLYOUT_N, s));
-    // the flight needs the live counts of the sort (long since read: the residual
-    // checks waited on later work)
-    BHIP(b, hipEventSynchronize(b->ev_n));
+    const int counted = take_counts();
+    if (counted) return counted;
     nmax = 0;
     for (int q = 0; q < K; ++q) {
-      emc_ctx* c = b->c[q];
-      Gpu& g = *c->gpu;
-      g.n = (long long)(unsigned)b->h_n[q];
-      g.sorted_n = g.n;
-      g.n_pending = false;
-      hfl[q] = fly_args(c, step[q], 0);
+      hfl[q] = fly_args(b->c[q], step[q], 0);
       hfl[q].gate = b->nmem ? b->gate : nullptr;
-      nmax = std::max(nmax, g.n);
+      nmax = std::max(nmax, b->c[q]->gpu->n);
     }
     BHIP(b, hipMemcpyAsync(b->d_tab + b->off_fly, b->h_tab + b->off_fly, K * sizeof(FlyArgs), hipMemcpyHostToDevice, s));
     BHIP(b, hipEventRecord(b->ev[5], s));

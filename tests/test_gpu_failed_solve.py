@@ -138,3 +138,33 @@ def test_step_that_missed_the_tolerance_is_taken_up():
         b.close()
         for e in together + alone:
             e.close()
+
+
+@pytest.mark.parametrize("refine", [1, 2])
+def test_failed_batch_step_after_losses(refine):
+    """The failed step's sort has dropped the slots of carriers that left in the step
+    before: the count is that of the carriers that are left, none of them twice."""
+    es = [emcgpu.Engine(cfg1_deck(refine=refine, electrons=20000, holes=2000, vd=0.6 + 0.1 * q), device=0, seed=2 + q)
+          for q in range(2)]
+    b = None
+    try:
+        for e in es:
+            e.particles_init()
+        b = emcgpu.Batch(es)
+        for _ in range(200):
+            acc = b.step(1)
+            if all(t.n_catch > t.n_gen + 1 for t in acc):
+                break
+        else:
+            pytest.fail("no step in which both devices lose carriers")
+        before = [state(e) for e in es]
+        spoil(es[1])
+        failing(lambda: b.step(1))
+        for q, e in enumerate(es):
+            assert e.count() == before[q]["n"]
+            same(state(e), before[q], f"device {q}")
+    finally:
+        if b:
+            b.close()
+        for e in es:
+            e.close()
